@@ -1,0 +1,537 @@
+// FP64 brick kernel of the 3D Godunov update (slopes 0-2, one Riemann solver
+// per instance; the 27-point slope and the mixed precision run brick_body of
+// rh_godunov.hip).
+//
+// One workgroup per oct brick, one thread per column of the brick's cells plus
+// one halo cell, marching along z.  Per plane tt there are two phases, each
+// ended by a barrier:
+//   A: the update of plane tt-1 from the face fluxes in LDS (its z flux and that
+//      of tt-2 in registers, so tt-2 becomes final and is stored); the own cell
+//      of plane tt+1 converted to primitives, the loads of plane tt+2 issued;
+//      slopes and Hancock predictor of plane tt, its left x and y states to LDS;
+//   B: primitives of plane tt+1 to LDS (every slope of plane tt has read the
+//      plane by now, so one plane is kept), and the Riemann problems of plane tt,
+//      the x and y fluxes to LDS.
+// The states and the fluxes have buffers of their own: two barriers per plane
+// instead of four when the fluxes overwrite the states, and the update's LDS
+// latency overlaps the conversion and the slopes.
+//
+// The kernel is bound by the issue of its vector instructions at two waves per
+// SIMD, so what counts is instructions per plane.  Where the 4 BX BY interior
+// columns fill whole waves and the halo ring fits one more (8x6, 4x4 bricks),
+// interior and halo waves run loops of their own (the role is uniform in a
+// wave, both loops pass the same barriers): the interior loop has no ring
+// loads, no divergent tests, and solves its three faces in straight line; the
+// halo loop solves one face per lane, converts the ring and updates nothing.
+// Measured against the one-body kernel this replaced (four barriers, every
+// thread testing its role, the expressions of rh_physics.h), with the Courant
+// reduction: 256^3 in 8x6x16 bricks 843 -> 675 us (24.9 G cell-updates/s, 2.0
+// TB/s of the 80 algorithmic bytes per cell), 128^3 in 8x6x8 bricks 140 -> 109
+// us, 90^3 MinMod + LLF (a run-time solver choice before) 105 -> 64 us.
+#pragma once
+#include <type_traits>
+
+#include "rh_courant.h"
+#include "rh_gather.h"
+
+namespace rh {
+
+// Waves per SIMD the kernel is built for: at three (168 VGPRs) it spills.
+constexpr int kBrick64Waves = 2;
+
+template <int BX, int BY> constexpr bool brick64_hw()
+{
+    return (4 * BX * BY) % 64 == 0 && (2 * BX + 2) * (2 * BY + 2) - 4 * BX * BY <= 64;
+}
+
+// LDS of one workgroup.  sacc (coarse-fine refluxes summed per window oct, one
+// atomic per ghost oct at the end) is added where the workgroups of two waves
+// per SIMD still fit the 160 KB of a CU with it.
+template <int BX, int BY, int BZ, bool GEN> struct Brick64Core {
+    static constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY, NI = 4 * BX * BY;
+    static constexpr int NP = (2 * BX + 4) * (2 * BY + 4), NW = (BX + 2) * (BY + 2) * (BZ + 2);
+    static constexpr int NFX = 2 * BY * (2 * BX + 1), NFY = 2 * BX * (2 * BY + 1);
+    int32_t swin[NW];
+    double sq[5][NP];                  // primitives of one plane
+    double qx[5][NFX], qy[5][NFY];     // left states by face
+    double fx[5][NFX], fy[5][NFY];     // fluxes by face
+    double sun[5][NI];                 // new state of the lower plane of an oct layer
+    double sub[GEN ? 1 : 2][5][GEN ? 1 : NI];  // conserved state of the last two planes (the update's base)
+    uint8_t sref[GEN ? 2 : 1][GEN ? NP : 1];   // refined flags of two planes
+};
+template <int BX, int BY, int BZ, bool GEN> struct Brick64Lds : Brick64Core<BX, BY, BZ, GEN> {
+    using Core = Brick64Core<BX, BY, BZ, GEN>;
+    static constexpr int WGS = 4 * kBrick64Waves / ((Core::NT + 63) / 64) > 0 ? 4 * kBrick64Waves / ((Core::NT + 63) / 64) : 1;
+    static constexpr bool RA =
+        GEN && Core::NW <= 512 && sizeof(Core) + (size_t)Core::NW * 40 <= (size_t)160 * 1024 / WGS;
+    double sacc[RA ? Core::NW : 1][5];
+};
+
+// The march over the z layers [zlo, zhi] of brick bid.  Courant partials go to
+// cpart[4*pslot].  A: GodArgs, as a kernel argument or in the constant address
+// space (a work-list descriptor).  GEN = false: a level periodic in every
+// dimension, without refined cells, refluxes or gravity, whose update adds to
+// uold.
+template <int BX, int BY, int BZ, int RS, bool GEN, typename A>
+__device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, const int zhi, const int pslot,
+                                        Brick64Lds<BX, BY, BZ, GEN> &sm)
+{
+    constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY, NI = 4 * BX * BY;
+    constexpr int PX = 2 * BX + 4;
+    constexpr int WX = BX + 2, WY = BY + 2, NW = WX * WY * (BZ + 2);
+    constexpr bool HW = brick64_hw<BX, BY>(), RA = Brick64Lds<BX, BY, BZ, GEN>::RA;
+    const int tid = threadIdx.x;
+    for (int i = tid; i < NW; i += NT) sm.swin[i] = a.win[(size_t)bid * NW + i];
+    const bool rlds = RA && a.reflux && !a.rdet;
+    if (RA && rlds)
+        for (int i = tid; i < NW * 5; i += NT) (&sm.sacc[0][0])[i] = 0.0;
+    const int ox0 = a.org[3 * bid + 0], oy0 = a.org[3 * bid + 1], oz0 = a.org[3 * bid + 2];
+    const int tlo = 2 * zlo, thi = 2 * zhi + 1;
+
+    const double dt = a.dt_dev ? *a.dt_dev : a.dt;
+    const HydroK<double> k = make_k<double>(dt, a.dx, a.gamma, a.smallr, a.smallc2, a.courant_factor, a.smax_cap,
+                                            a.use_smax, a.slope, a.riemann);
+    const double gm1 = a.gamma - 1.0, smalle = a.smallc2 / a.gamma / gm1;
+    double gvec[3] = {0.0, 0.0, 0.0}, gdt[3] = {0.0, 0.0, 0.0};
+    if constexpr (GEN)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            gvec[d] = a.g[d];
+            gdt[d] = a.g[d] * (dt * 0.5);
+        }
+    // The fluxes stay unscaled; the update adds dt/dx times each difference of
+    // the two faces of a dimension with one FMA, both cells of a face reading
+    // the same flux, so the update conserves.  The reference's (F dt)/dx
+    // (hydro/umuscl.f90:135-220) is formed only for the coarse reflux.
+    const double dtdx = dt * a.inv_dx;
+    const int boxmin[3] = {a.boxmin[0], a.boxmin[1], a.boxmin[2]};
+    const int boxmax[3] = {a.boxmax[0], a.boxmax[1], a.boxmax[2]};
+    const bool anyref = GEN && a.any_ref != 0, bnd = GEN && a.bnd != 0, reflux = GEN && a.reflux != 0;
+    int refl = 0;
+    if constexpr (GEN)
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+#pragma unroll
+            for (int sd = 0; sd < 2; sd++) refl |= (a.btype[d][sd] == 1) << (2 * d + sd);
+    const CourantK ck = make_courant_k(a.dx, 3, a.gamma, a.smallr, a.smallc2, a.courant_factor, gvec);
+    const bool courant = a.courant != 0;
+    double c_mass = 0.0, c_ekin = 0.0, c_eint = 0.0, c_sig = 0.0;
+    __syncthreads();
+
+    // ROLE 1: a column of the brick's interior; 2: a column of the halo ring;
+    // 0: either, tested per thread (shapes whose interior does not fill waves)
+    auto run = [&](auto role) __attribute__((always_inline)) {
+        constexpr int ROLE = decltype(role)::value;
+        int cx, cy;
+        if constexpr (ROLE == 1) {
+            cx = tid % (2 * BX);
+            cy = tid / (2 * BX);
+        } else if constexpr (ROLE == 2) {
+            const int h = tid - NI;
+            if (h < 2 * CX) {
+                cx = (h < CX ? h : h - CX) - 1;
+                cy = h < CX ? -1 : 2 * BY;
+            } else {
+                const int g = h - 2 * CX;
+                cx = g < 2 * BY ? -1 : 2 * BX;
+                cy = g < 2 * BY ? g : g - 2 * BY;
+            }
+        } else {
+            cx = tid % CX - 1;
+            cy = tid / CX - 1;
+        }
+        const bool inx = ROLE == 1 || (cx >= 0 && cx < 2 * BX), iny = ROLE == 1 || (cy >= 0 && cy < 2 * BY);
+        const bool interior = ROLE == 1 || (ROLE == 0 && inx && iny);
+        // faces: the column's low x and y faces are solved by it, its left
+        // states belong to its high faces
+        const bool do_fx = ROLE == 1 || (iny && cx >= 0), do_fy = ROLE == 1 || (inx && cy >= 0);
+        const bool has_qx = ROLE == 1 || (iny && cx < 2 * BX), has_qy = ROLE == 1 || (inx && cy < 2 * BY);
+        const int pc = (cy + 2) * PX + (cx + 2);
+        // x face f of row cy: the first 2BX faces row by row, then the last
+        // faces of all rows (the rows of a wave stay 2BX doubles apart)
+        const int ixl = (ROLE != 1 && cx == 2 * BX) ? NI + cy : cy * (2 * BX) + cx;
+        const int ixh = cx == 2 * BX - 1 ? NI + cy : cy * (2 * BX) + cx + 1;
+        const int iyl = cy * (2 * BX) + cx, iyh = iyl + 2 * BX;
+        const int icol = cy * (2 * BX) + cx;  // interior only
+        const int wcol = ((cy + 2) >> 1) * WX + ((cx + 2) >> 1), icell = (cx & 1) + 2 * (cy & 1);
+
+        // ring of cells around the column region: its corners are read by no
+        // slope that feeds a face, and (ROLE 2) neither are the two cells next
+        // to each corner
+        constexpr int NRING = ROLE == 2 ? 4 * (BX + BY) : ROLE == 0 ? 2 * (CX + CY) : 0;
+        const int r = ROLE == 2 ? tid - NI : tid;
+        const bool ring = ROLE != 1 && r < NRING;
+        int rx = 0, ry = 0;
+        if (ring) {
+            constexpr int EX = ROLE == 2 ? 2 * BX : CX, EY = ROLE == 2 ? 2 * BY : CY, E0 = ROLE == 2 ? 0 : -1;
+            if (r < 2 * EX) {
+                rx = (r < EX ? r : r - EX) + E0;
+                ry = r < EX ? -2 : 2 * BY + 1;
+            } else {
+                const int g = r - 2 * EX;
+                rx = g < EY ? -2 : 2 * BX + 1;
+                ry = (g < EY ? g : g - EY) + E0;
+            }
+        }
+        const int pr = (ry + 2) * PX + (rx + 2);
+
+        auto fetch = [&](int px, int py, int tz, double u[5], uint8_t &rf, int &fl) __attribute__((always_inline)) {
+            const int ox = (px + 2) >> 1, oy = (py + 2) >> 1, oz = (tz + 2) >> 1;
+            const int v = sm.swin[(oz * WY + oy) * WX + ox];
+            fl = -1;
+            rf = 0;
+            if (!bnd) {
+                // no boundary ghosts: an oct, or none (then nothing that the
+                // cell feeds is stored, and any cell's values do)
+                const size_t o = (size_t)(v > 1 ? v - 1 : 0);
+                const int ind = (px & 1) + 2 * (py & 1) + 4 * (tz & 1);
+                const double *p = a.uold + o * 40 + ind;
+#pragma unroll
+                for (int n = 0; n < 5; n++) u[n] = p[8 * n];
+                if (anyref && v > 0) rf = a.refined[o * 8 + ind];
+                return;
+            }
+            const int okey[3] = {ox0 + ox - 1, oy0 + oy - 1, oz0 + oz - 1};
+            const int c[3] = {px & 1, py & 1, tz & 1};
+            CellRef cr = cell_ref3(a.uold, a.refined, v, okey, boxmin, boxmax, refl, c);
+            if (!anyref) cr.rf = nullptr;
+            cell_load3(cr, u, rf);
+            fl = cr.flip;
+        };
+
+        double u_o[5], u_r[5];
+        uint8_t rf_o = 0, rf_r = 0;
+        int fl_o = -1, fl_r = -1;
+        auto convert = [&](double u[5], int fl, double q[5]) __attribute__((always_inline)) {
+            if (bnd && fl >= 0) cell_flip(u, fl);  // reflexive ghosts only: skipped by waves without any
+            return prim64(u, q, a.smallr, smalle, gm1, gdt);
+        };
+        auto put = [&](const double q[5], uint8_t rf, int i, int par) __attribute__((always_inline)) {
+#pragma unroll
+            for (int n = 0; n < 5; n++) sm.sq[n][i] = q[n];
+            if (anyref) sm.sref[GEN ? par : 0][GEN ? i : 0] = rf;
+        };
+
+        // own column: primitives of plane tt, their difference from plane tt-1
+        // (the upper difference of the plane before), density of plane tt-1,
+        // 1/rho of plane tt
+        double q0[5], dzm[5], rho_m, ir0;
+        {
+            double q[5];
+            fetch(cx, cy, tlo - 2, u_o, rf_o, fl_o);
+            convert(u_o, fl_o, q);
+            fetch(cx, cy, tlo - 1, u_o, rf_o, fl_o);
+            if (ring) fetch(rx, ry, tlo - 1, u_r, rf_r, fl_r);
+            ir0 = convert(u_o, fl_o, q0);
+            rho_m = q[0];
+#pragma unroll
+            for (int n = 0; n < 5; n++) dzm[n] = q0[n] - q[n];
+            put(q0, rf_o, pc, 1);
+            if (ring) {
+                convert(u_r, fl_r, q);
+                put(q, rf_r, pr, 1);
+            }
+            fetch(cx, cy, tlo, u_o, rf_o, fl_o);
+            if (ring) fetch(rx, ry, tlo, u_r, rf_r, fl_r);
+        }
+        __syncthreads();
+
+        double qmz[5] = {0, 0, 0, 0, 0};   // left state of the low z face of plane tt
+        double fz[5] = {0, 0, 0, 0, 0};    // flux of the low z face of plane tt-1
+        double fzp[5] = {0, 0, 0, 0, 0};   // of plane tt-2
+        double pp[5] = {0, 0, 0, 0, 0};    // u + x and y parts of plane tt-2
+        double ub[5] = {0, 0, 0, 0, 0};    // the update's base of plane tt-1 (GEN)
+        uint8_t ref1 = 0, ref2 = 0;        // refined flags of planes tt-1 and tt-2
+
+        // plane tf of the column is final: un = pp + (dt/dx)(fzp - fz)
+        auto finish = [&](int tf, const bool upper) __attribute__((always_inline)) {
+            const int v = sm.swin[((tf + 2) >> 1) * (WX * WY) + wcol];
+            const bool own = v >= a.head && v < a.head + a.noct && ox0 + (cx >> 1) < boxmax[0] &&
+                             oy0 + (cy >> 1) < boxmax[1] && oz0 + (tf >> 1) < boxmax[2];
+            if (!own) return;
+            double un[5];
+#pragma unroll
+            for (int n = 0; n < 5; n++) un[n] = tfma(dtdx, fzp[n] - fz[n], pp[n]);
+            // the two planes of an oct fill each 64-byte line of unew: the
+            // lower plane's values wait in LDS and both are stored together
+            if (upper) {
+                double *po = a.unew + (size_t)(v - 1) * 40 + icell;
+#pragma unroll
+                for (int n = 0; n < 5; n++) {
+                    po[8 * n] = sm.sun[n][icol];
+                    po[8 * n + 4] = un[n];
+                }
+            } else {
+#pragma unroll
+                for (int n = 0; n < 5; n++) sm.sun[n][icol] = un[n];
+            }
+            if (courant && !ref2) c_sig = tmax(c_sig, courant_cell<3>(un, ck, ck.vol, c_mass, c_ekin, c_eint));
+        };
+
+        // one plane; par = tt & 1
+        auto plane = [&](const int tt, const int par) __attribute__((always_inline)) {
+            // ---- A: update of plane tt-1, plane tt-2 stored ----
+            if (interior && tt > tlo) {
+                double part[5];
+#pragma unroll
+                for (int n = 0; n < 5; n++) {
+                    const double u = GEN ? ub[n] : sm.sub[GEN ? 0 : par ^ 1][n][GEN ? 0 : icol];
+                    part[n] = tfma(dtdx, sm.fy[n][iyl] - sm.fy[n][iyh],
+                                   tfma(dtdx, sm.fx[n][ixl] - sm.fx[n][ixh], u));
+                }
+                if (tt - 2 >= tlo) finish(tt - 2, par != 0);
+#pragma unroll
+                for (int n = 0; n < 5; n++) {
+                    pp[n] = part[n];
+                    fzp[n] = fz[n];
+                }
+            }
+            // ---- the own cell of plane tt+1 ----
+            double qp[5];
+            if constexpr (!GEN) {
+                if (interior)
+#pragma unroll
+                    for (int n = 0; n < 5; n++) sm.sub[GEN ? 0 : par ^ 1][n][GEN ? 0 : icol] = u_o[n];
+            }
+            const double irp = convert(u_o, fl_o, qp);
+            const uint8_t rfp = rf_o;
+            // the next loads below the conversion that consumes the current ones, so that both use the same registers
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(cx, cy, tt < thi ? tt + 2 : thi + 2, u_o, rf_o, fl_o);
+            // ---- T: slopes and predictor of plane tt ----
+            double dq[3][5];
+            auto slopes = [&](const int sl) __attribute__((always_inline)) {
+#pragma unroll
+                for (int n = 0; n < 5; n++) {
+                    dq[0][n] = slope64(sl, q0[n] - sm.sq[n][pc - 1], sm.sq[n][pc + 1] - q0[n]);
+                    dq[1][n] = slope64(sl, q0[n] - sm.sq[n][pc - PX], sm.sq[n][pc + PX] - q0[n]);
+                    dq[2][n] = slope64(sl, dzm[n], qp[n] - q0[n]);
+                }
+                dq[0][1] = vel_bound64(dq[0][1], sm.sq[0][pc - 1], q0[1] - sm.sq[1][pc - 1], ir0, sm.sq[0][pc + 1],
+                                       sm.sq[1][pc + 1] - q0[1]);
+                dq[1][2] = vel_bound64(dq[1][2], sm.sq[0][pc - PX], q0[2] - sm.sq[2][pc - PX], ir0,
+                                       sm.sq[0][pc + PX], sm.sq[2][pc + PX] - q0[2]);
+                dq[2][3] = vel_bound64(dq[2][3], rho_m, dzm[3], ir0, qp[0], qp[3] - q0[3]);
+            };
+            if (k.slope_type == 1)
+                slopes(1);
+            else if (k.slope_type != 0)
+                slopes(2);
+            else
+#pragma unroll
+                for (int n = 0; n < 5; n++) dq[0][n] = dq[1][n] = dq[2][n] = 0.0;
+            double qr[3][5], ql[3][5];
+            trace64(q0, dq, qr, ql, k, ir0);
+            if (has_qx)
+#pragma unroll
+                for (int n = 0; n < 5; n++) sm.qx[n][ixh] = ql[0][n];
+            if (has_qy)
+#pragma unroll
+                for (int n = 0; n < 5; n++) sm.qy[n][iyh] = ql[1][n];
+            const uint8_t myref = anyref ? sm.sref[GEN ? par : 0][GEN ? pc : 0] : 0;
+            __syncthreads();
+            // ---- B: primitives of plane tt+1 to LDS ----
+            put(qp, rfp, pc, par ^ 1);
+            if (ring) {
+                double q[5];
+                convert(u_r, fl_r, q);
+                put(q, rf_r, pr, par ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
+                fetch(rx, ry, tt < thi ? tt + 2 : thi + 1, u_r, rf_r, fl_r);
+            }
+            // ---- F: the low x, y and z faces of plane tt ----
+            const bool xy = tt >= tlo && tt <= thi;
+            double f_x[5], f_y[5];
+            if (ROLE == 2) {
+                // the right column's x face or the top row's y face: one pass,
+                // the direction chosen per lane
+                if (xy && (do_fx || do_fy)) {
+                    const bool dy = do_fy;
+                    double l[5], g[5];
+#pragma unroll
+                    for (int n = 0; n < 5; n++) l[n] = dy ? sm.qy[n][iyl] : sm.qx[n][ixl];
+                    const double l5[5] = {l[0], dy ? l[2] : l[1], dy ? l[1] : l[2], l[3], l[4]};
+                    const double r5[5] = {dy ? qr[1][0] : qr[0][0], dy ? qr[1][2] : qr[0][1], dy ? qr[1][1] : qr[0][2],
+                                          dy ? qr[1][3] : qr[0][3], dy ? qr[1][4] : qr[0][4]};
+                    solve64<RS>(l5, r5, g, k);
+                    bool z = false;
+                    if (anyref) z = myref || sm.sref[GEN ? par : 0][GEN ? (dy ? pc - PX : pc - 1) : 0];
+                    const double f[5] = {z ? 0.0 : g[0], z ? 0.0 : (dy ? g[2] : g[1]), z ? 0.0 : (dy ? g[1] : g[2]),
+                                         z ? 0.0 : g[3], z ? 0.0 : g[4]};
+                    double *fb = dy ? &sm.fy[0][iyl] : &sm.fx[0][ixl];
+                    const int st = dy ? Brick64Lds<BX, BY, BZ, GEN>::NFY : Brick64Lds<BX, BY, BZ, GEN>::NFX;
+#pragma unroll
+                    for (int n = 0; n < 5; n++) {
+                        fb[n * st] = f[n];
+                        f_x[n] = f_y[n] = f[n];
+                    }
+                }
+            } else if (xy) {
+                if (do_fx) {
+                    double l[5];
+#pragma unroll
+                    for (int n = 0; n < 5; n++) l[n] = sm.qx[n][ixl];
+                    face64<RS>(0, l, qr[0], f_x, k);
+                    if (anyref) {
+                        const bool z = myref || sm.sref[GEN ? par : 0][GEN ? pc - 1 : 0];
+#pragma unroll
+                        for (int n = 0; n < 5; n++) f_x[n] = z ? 0.0 : f_x[n];
+                    }
+#pragma unroll
+                    for (int n = 0; n < 5; n++) sm.fx[n][ixl] = f_x[n];
+                }
+                if (do_fy) {
+                    double l[5];
+#pragma unroll
+                    for (int n = 0; n < 5; n++) l[n] = sm.qy[n][iyl];
+                    face64<RS>(1, l, qr[1], f_y, k);
+                    if (anyref) {
+                        const bool z = myref || sm.sref[GEN ? par : 0][GEN ? pc - PX : 0];
+#pragma unroll
+                        for (int n = 0; n < 5; n++) f_y[n] = z ? 0.0 : f_y[n];
+                    }
+#pragma unroll
+                    for (int n = 0; n < 5; n++) sm.fy[n][iyl] = f_y[n];
+                }
+            }
+            if (ROLE != 2 && interior && tt >= tlo) {
+                face64<RS>(2, qmz, qr[2], fz, k);
+                if (anyref) {
+                    const bool z = myref || ref1;
+#pragma unroll
+                    for (int n = 0; n < 5; n++) fz[n] = z ? 0.0 : fz[n];
+                }
+            }
+            if constexpr (GEN) {
+                // the base of this plane's update (unew for the drop-in call,
+                // uold for the device-resident steps)
+                if (interior && xy) {
+                    const int v = sm.swin[((tt + 2) >> 1) * (WX * WY) + wcol];
+                    const double *pb = a.ubase + (size_t)(v > 1 ? v - 1 : 0) * 40 + icell + 4 * par;
+#pragma unroll
+                    for (int n = 0; n < 5; n++) ub[n] = pb[8 * n];
+                }
+            }
+            if (reflux) {
+                auto wi = [&](int x, int y, int z) { return (((z + 2) >> 1) * WY + ((y + 2) >> 1)) * WX + ((x + 2) >> 1); };
+                // one fine face's reflux into the ghost oct of window slot i:
+                // summed in LDS, or straight to the accumulator / parent cell
+                auto radd = [&](int i, int v, double sign, const double F[5], int slot) {
+                    if (RA && rlds) {
+#pragma unroll
+                        for (int n = 0; n < 5; n++)
+                            atomicAdd(&sm.sacc[RA ? i : 0][n], sign * ((F[n] * dt) * a.inv_dx * 0.125));
+                    } else {
+                        double G[5];
+#pragma unroll
+                        for (int n = 0; n < 5; n++) G[n] = (F[n] * dt) * a.inv_dx;
+                        reflux_add(a.unew, a.ghost_parent, a.ngridmax, v, sign, G, 8, a.racc, a.rdet, slot);
+                    }
+                };
+                auto owned = [&](int x, int y, int z, int v) {
+                    return x >= 0 && x < 2 * BX && y >= 0 && y < 2 * BY && z >= 2 * zlo && z <= 2 * zhi + 1 &&
+                           v >= a.head && v < a.head + a.noct && ox0 + (x >> 1) < boxmax[0] &&
+                           oy0 + (y >> 1) < boxmax[1] && oz0 + (z >> 1) < boxmax[2];
+                };
+                if (xy && do_fx && !(anyref && (myref || sm.sref[GEN ? par : 0][GEN ? pc - 1 : 0]))) {
+                    const int il = wi(cx - 1, cy, tt), ih = wi(cx, cy, tt), vl = sm.swin[il], vh = sm.swin[ih];
+                    const int s = (cy & 1) + 2 * (tt & 1);
+                    if (vl > a.ngridmax && owned(cx, cy, tt, vh)) radd(il, vl, -1.0, f_x, 4 + s);
+                    if (vh > a.ngridmax && owned(cx - 1, cy, tt, vl)) radd(ih, vh, 1.0, f_x, s);
+                }
+                if (xy && do_fy && !(anyref && (myref || sm.sref[GEN ? par : 0][GEN ? pc - PX : 0]))) {
+                    const int il = wi(cx, cy - 1, tt), ih = wi(cx, cy, tt), vl = sm.swin[il], vh = sm.swin[ih];
+                    const int s = (cx & 1) + 2 * (tt & 1);
+                    if (vl > a.ngridmax && owned(cx, cy, tt, vh)) radd(il, vl, -1.0, f_y, 12 + s);
+                    if (vh > a.ngridmax && owned(cx, cy - 1, tt, vl)) radd(ih, vh, 1.0, f_y, 8 + s);
+                }
+                if (interior && tt >= tlo && !(myref || ref1)) {
+                    const int il = wi(cx, cy, tt - 1), ih = wi(cx, cy, tt), vl = sm.swin[il], vh = sm.swin[ih];
+                    const int s = (cx & 1) + 2 * (cy & 1);
+                    if (vl > a.ngridmax && owned(cx, cy, tt, vh)) radd(il, vl, -1.0, fz, 20 + s);
+                    if (vh > a.ngridmax && owned(cx, cy, tt - 1, vl)) radd(ih, vh, 1.0, fz, 16 + s);
+                }
+            }
+            __syncthreads();
+            rho_m = q0[0];
+            ir0 = irp;
+#pragma unroll
+            for (int n = 0; n < 5; n++) {
+                qmz[n] = ql[2][n];
+                dzm[n] = qp[n] - q0[n];
+                q0[n] = qp[n];
+            }
+            ref2 = ref1;
+            ref1 = myref;
+        };
+        // planes tlo-1 .. thi+1, two per trip (tlo is even, thi odd): the parity
+        // is a constant and the values carried from plane to plane are renamed
+        for (int tt = tlo - 1; tt <= thi; tt += 2) {
+            plane(tt, 1);
+            plane(tt + 1, 0);
+        }
+        if (interior) finish(thi, true);
+    };
+    // (the upper half of a split brick may hold no layer)
+    if (zlo <= zhi) {
+        if constexpr (HW) {
+            if (__builtin_amdgcn_readfirstlane(tid) < NI)
+                run(std::integral_constant<int, 1>());
+            else
+                run(std::integral_constant<int, 2>());
+        } else {
+            run(std::integral_constant<int, 0>());
+        }
+    }
+
+    if (RA && rlds) {
+        // one atomic per ghost oct of the window and conserved variable
+        __syncthreads();
+        for (int i = tid; i < NW; i += NT) {
+            const int v = sm.swin[i];
+            if (v <= a.ngridmax) continue;
+            double q[5];
+            bool any = false;
+#pragma unroll
+            for (int n = 0; n < 5; n++) {
+                q[n] = sm.sacc[RA ? i : 0][n];
+                any = any || q[n] != 0.0;
+            }
+            if (any) reflux_flush(a.unew, a.ghost_parent, a.ngridmax, v, q, 8, a.racc);
+        }
+    }
+    if (courant) {
+        // the brick's partials of courant_fine in a fixed reduction order; the
+        // last wave may be partial (NT need not be a multiple of 64)
+        const int nv = NT - (tid & ~63) < 64 ? NT - (tid & ~63) : 64;
+        c_mass = wave_sum_n(c_mass, nv);
+        c_ekin = wave_sum_n(c_ekin, nv);
+        c_eint = wave_sum_n(c_eint, nv);
+        c_sig = wave_max_n(c_sig, nv);
+        __syncthreads();
+        double *red = &sm.sq[0][0];
+        const int w = tid >> 6;
+        if ((tid & 63) == 0) {
+            red[4 * w + 0] = c_mass;
+            red[4 * w + 1] = c_ekin;
+            red[4 * w + 2] = c_eint;
+            red[4 * w + 3] = c_sig;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            double m = 0, e = 0, ei = 0, s = red[3];
+            for (int i = 0; i < (NT + 63) / 64; i++) {
+                m += red[4 * i];
+                e += red[4 * i + 1];
+                ei += red[4 * i + 2];
+                s = tmax(s, red[4 * i + 3]);
+            }
+            a.cpart[4 * pslot + 0] = m;
+            a.cpart[4 * pslot + 1] = e;
+            a.cpart[4 * pslot + 2] = ei;
+            a.cpart[4 * pslot + 3] = signal_dt(s, ck);
+        }
+    }
+}
+
+}  // namespace rh

@@ -1,0 +1,134 @@
+// FP64 brick kernels: the instances of brick64 and their launches.  Compiled
+// once per set of brick shapes (RH_SET), so that the sets build in parallel.
+//
+// This file is compiled with -fno-honor-nans: min and max are then single
+// instructions, where the IEEE mode otherwise quiets every operand that comes
+// from memory or from another block (two more instructions per Riemann solve
+// and floor, about 40 of 810 per plane; 256^3 kernel 794 -> 753 us).  No path
+// depends on a NaN: a state that holds one is lost either way.
+#include "rh_brick64.h"
+#include "rh_launch.h"
+
+#ifndef RH_SET
+#error "RH_SET selects the brick shapes of this object"
+#endif
+#define RH_CAT2(a, b) a##b
+#define RH_CAT(a, b) RH_CAT2(a, b)
+#if RH_SET == 0
+#define RH_SHAPES(X) X(7, 7, 8) X(7, 7, 16)
+#elif RH_SET == 1
+#define RH_SHAPES(X) X(8, 6, 8) X(8, 6, 16)
+#elif RH_SET == 2
+#define RH_SHAPES(X) X(4, 4, 4) X(4, 4, 8)
+#elif RH_SET == 3
+#define RH_SHAPES(X) X(15, 7, 8) X(15, 7, 16)
+#elif RH_SET == 4
+#define RH_SHAPES(X) X(7, 7, 4) X(3, 3, 4)
+#else
+#define RH_SHAPES(X) X(3, 3, 8) X(1, 1, 1)
+#endif
+
+namespace rh {
+
+__device__ __forceinline__ void brick_layers(const int32_t *zrs, int bid, int bz, int part, int &zlo, int &zhi)
+{
+    // z layers of the brick that hold octs of the level
+    const int zr = zrs ? zrs[bid] : ((bz - 1) << 16);
+    zlo = zr & 0xffff;
+    zhi = zr >> 16;
+    if (part >= 0) {
+        // half of them (the lower half holds the middle one)
+        const int mid = (zlo + zhi) >> 1;
+        if (part == 0)
+            zhi = mid;
+        else
+            zlo = mid + 1;
+    }
+}
+
+template <int BX, int BY, int BZ, int RS, bool GEN>
+__global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2), kBrick64Waves) k_brick64(const GodArgs a)
+{
+    __shared__ Brick64Lds<BX, BY, BZ, GEN> sm;
+    int bid, part, pslot, zlo, zhi;
+    if (!level_item(a, bid, part, pslot)) return;
+    brick_layers(a.zr, bid, BZ, part, zlo, zhi);
+    brick64<BX, BY, BZ, RS, GEN>(a, bid, zlo, zhi, pslot, sm);
+}
+
+// Work-list form, see k_godunov3d_wl: workgroup b runs item range[b % 8] + b / 8.
+typedef const __attribute__((address_space(4))) GodArgs ConstGodArgs;
+
+template <int BX, int BY, int BZ, int RS, bool GEN>
+__global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2), kBrick64Waves) k_brick64_wl(const WorkList w)
+{
+    __shared__ Brick64Lds<BX, BY, BZ, GEN> sm;
+    const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
+    const int i = w.range[x] + l;
+    if (i >= w.range[x + 1]) return;
+    const int2 it = w.items[i];
+    const int di = __builtin_amdgcn_readfirstlane(it.x), bid = __builtin_amdgcn_readfirstlane(it.y);
+    auto &a = ((ConstGodArgs *)w.descs)[di];
+    int zlo, zhi;
+    brick_layers(a.zr, bid, BZ, -1, zlo, zhi);
+    brick64<BX, BY, BZ, RS, GEN>(a, bid, zlo, zhi, bid, sm);
+}
+
+template <int BX, int BY, int BZ, int RS>
+static void level_launch(const GodArgs &a, bool gen, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int *nparts)
+{
+    constexpr int nt = (2 * BX + 2) * (2 * BY + 2);
+    if (gen)
+        launch_brick(k_brick64<BX, BY, BZ, RS, true>, nt, a, s, e0, e1, nparts);
+    else
+        launch_brick(k_brick64<BX, BY, BZ, RS, false>, nt, a, s, e0, e1, nparts);
+}
+
+template <int BX, int BY, int BZ, int RS>
+static void list_launch(const WorkList &w, int nblocks, bool gen, hipStream_t s)
+{
+    const dim3 g(nblocks), b((2 * BX + 2) * (2 * BY + 2));
+    if (gen)
+        hipLaunchKernelGGL((k_brick64_wl<BX, BY, BZ, RS, true>), g, b, 0, s, w);
+    else
+        hipLaunchKernelGGL((k_brick64_wl<BX, BY, BZ, RS, false>), g, b, 0, s, w);
+}
+
+// The launches of this object's shapes; false for a shape of another set.
+bool RH_CAT(brick64_level_, RH_SET)(const GodArgs &a, int bx, int by, int bz, bool gen, hipStream_t s, hipEvent_t e0,
+                                    hipEvent_t e1, int *nparts)
+{
+#define RH_ONE(A, B, C)                                                \
+    if (bx == A && by == B && bz == C) {                               \
+        if (a.riemann == 3)                                            \
+            level_launch<A, B, C, 3>(a, gen, s, e0, e1, nparts);       \
+        else if (a.riemann == 2)                                       \
+            level_launch<A, B, C, 2>(a, gen, s, e0, e1, nparts);       \
+        else                                                           \
+            level_launch<A, B, C, 1>(a, gen, s, e0, e1, nparts);       \
+        return true;                                                   \
+    }
+    RH_SHAPES(RH_ONE)
+#undef RH_ONE
+    return false;
+}
+
+bool RH_CAT(brick64_list_, RH_SET)(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, bool gen,
+                                   hipStream_t s)
+{
+#define RH_ONE(A, B, C)                                                \
+    if (bx == A && by == B && bz == C) {                               \
+        if (riemann == 3)                                              \
+            list_launch<A, B, C, 3>(w, nblocks, gen, s);               \
+        else if (riemann == 2)                                         \
+            list_launch<A, B, C, 2>(w, nblocks, gen, s);               \
+        else                                                           \
+            list_launch<A, B, C, 1>(w, nblocks, gen, s);               \
+        return true;                                                   \
+    }
+    RH_SHAPES(RH_ONE)
+#undef RH_ONE
+    return false;
+}
+
+}  // namespace rh

@@ -104,11 +104,18 @@ hipError_t launch_godunov1d(const God1Args &a, int prec, hipStream_t s);
 // everywhere, for checking that both give the same bits).
 extern int g_specialized;
 // Work-list launch: items[i] = (descriptor index, brick index), one workgroup per item.
-// gen = false: every descriptor is a periodic level without refined cells or
-// refluxes (bnd, any_ref and reflux all 0) whose update adds to uold (ubase ==
-// uold), which the specialised body needs.
+// gen = false: every descriptor is a periodic level without refined cells,
+// refluxes (bnd, any_ref and reflux all 0) or gravity, whose update adds to uold
+// (ubase == uold), which the specialised body needs.
 hipError_t launch_godunov3d_wl(const WorkList &w, int bx, int by, int bz, int slope, int riemann, int prec,
                                hipStream_t s, bool gen = true);
+
+// The FP64 brick kernels of rh_brick64.hip (slopes 0-2); nblocks: the grid of
+// the work-list launch.
+hipError_t launch_brick64(const GodArgs &a, int bx, int by, int bz, bool gen, hipStream_t s, hipEvent_t e0,
+                          hipEvent_t e1, int *nparts);
+hipError_t launch_brick64_wl(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, bool gen,
+                             hipStream_t s);
 
 // Courant reduction over cells of octs [head, head+noct): per-block partials,
 // then a fixed-order final pass -> out[0..4] = mass, ekin, eint, emag, dt.

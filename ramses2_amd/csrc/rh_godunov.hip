@@ -1,6 +1,8 @@
 // gfx950 kernels of the fine-level Godunov hydro step.
 //
 // 3D: one workgroup per oct brick (BX*BY*BZ octs = 2BX x 2BY x 2BZ cells).
+// FP64 with the one-dimensional slopes runs brick64 (rh_brick64.h); brick_body
+// below is the mixed-precision kernel, and the FP64 one of the 27-point slope.
 // The workgroup marches through the brick along z, one cell plane per
 // iteration.  One thread owns one cell column of the (2BX+2) x (2BY+2) trace
 // region (the brick's cells plus one cell of halo).  Per plane:
@@ -17,168 +19,18 @@
 //      in the order of godfine1 (hydro/godunov_fine.f90:737-816), written to
 //      unew; the courant_fine sums and dt of the new state are reduced from
 //      registers as it is stored.
+// The FP32 results depend on every rounding, down to which of two products the
+// compiler contracts into an FMA, so the FP32 instances are left as they are
+// where the FP64 ones moved on.
 // No MFMA: the work is divides, square roots and compares, not a contraction.
-#include <hip/hip_ext.h>
-
-#include <map>
 #include <type_traits>
 
+#include "rh_courant.h"
 #include "rh_gather.h"
 #include "rh_godunov.h"
+#include "rh_launch.h"
 
 namespace rh {
-
-struct CourantK {
-    double dx, vol, gamma, smallr, smallc, courant_factor, smallp, gsum_dx;
-    int ndim;
-};
-
-// The gravity factor 1 + sqrt(1 + 2 C max(g dx/c_tot^2, 1e-4)) of cmpdt when
-// g = 0: a constant, formed once per thread with the expression cell_dt uses.
-__device__ __forceinline__ double grav_factor0(const CourantK &c)
-{
-    return 1.0 + __builtin_sqrt(1.0 + 2.0 * c.courant_factor * 0.0001);
-}
-
-// cmpdt, hydro/godunov_utils.f90:228-337, for one cell (no MHD).  ir = 1/r
-// (the Newton-refined reciprocal) replaces the reference's three divisions by
-// r, and with no magnetic field c_f = sqrt(c2 + sqrt(c2^2)) with c2 = a^2/2 is
-// exactly sqrt(a^2); gravity's correction is the constant gf0
-// (grav_factor0) when g = 0.
-__device__ __forceinline__ double cell_dt(double uu0, double uu1, double uu2, double uu3, double uu4, const CourantK &c,
-                                          double gf0)
-{
-    double r = uu0 > c.smallr ? uu0 : c.smallr;
-    const double ir = rcp_nr(r);
-    double v[3] = {uu1 * ir, uu2 * ir, uu3 * ir};
-    double e = uu4;
-    e = e - 0.5 * r * (v[0] * v[0]);
-    e = e - 0.5 * r * (v[1] * v[1]);
-    e = e - 0.5 * r * (v[2] * v[2]);
-    double pe = (c.gamma - 1.0) * e, pf = r * c.smallp;
-    double p = pe > pf ? pe : pf;
-    double a2 = c.gamma * p;
-    a2 = a2 * ir;
-    // a2 >= gamma smallp = smallc^2: the square root of the Riemann solvers
-    // (floored where smallc^2 < 2^-900)
-    double cf = sqrt_pos(a2 > 0x1p-900 ? a2 : 0x1p-900);
-    double ctot = 0.0;
-    for (int d = 0; d < c.ndim; d++) ctot = ctot + __builtin_fabs(v[d]) + cf;
-    double gf = gf0;
-    if (c.gsum_dx != 0.0) {
-        double grav = c.gsum_dx / (ctot * ctot);
-        grav = grav > 0.0001 ? grav : 0.0001;
-        gf = 1.0 + __builtin_sqrt(1.0 + 2.0 * c.courant_factor * grav);
-    }
-    double dtmax = c.courant_factor * c.dx / c.smallc;
-    double dtcell = 2.0 * c.courant_factor * c.dx / (ctot * gf);
-    return dtmax < dtcell ? dtmax : dtcell;
-}
-
-__device__ __forceinline__ double wave_sum(double x)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-    return x;
-}
-__device__ __forceinline__ double wave_min(double x)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        double y = __shfl_xor(x, o, 64);
-        x = y < x ? y : x;
-    }
-    return x;
-}
-// The same for a wave of which only lanes [0, nvalid) exist (the last wave of
-// a workgroup whose size is not a multiple of 64): partners at or beyond
-// nvalid are skipped.  Lane 0's partners in the round of offset o are lanes
-// o..2o-1, whose partial results only gather lanes above them, so lane 0
-// ends with the reduction over exactly the existing lanes.
-__device__ __forceinline__ double wave_sum_n(double x, int nvalid)
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const double y = __shfl_xor(x, o, 64);
-        if ((lane ^ o) < nvalid) x += y;
-    }
-    return x;
-}
-__device__ __forceinline__ double wave_min_n(double x, int nvalid)
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const double y = __shfl_xor(x, o, 64);
-        if ((lane ^ o) < nvalid && y < x) x = y;
-    }
-    return x;
-}
-
-__device__ __forceinline__ CourantK make_courant_k(double dx, int ndim, double gamma, double smallr, double smallc2,
-                                                   double courant_factor, const double g[3])
-{
-    CourantK c;
-    c.dx = dx;
-    c.vol = ndim == 1 ? dx : dx * dx * dx;
-    c.gamma = gamma;
-    c.smallr = smallr;
-    c.smallc = __builtin_sqrt(smallc2);
-    c.courant_factor = courant_factor;
-    c.smallp = smallc2 / gamma;
-    double gs = 0.0;
-    for (int d = 0; d < ndim; d++) gs = gs + __builtin_fabs(g[d]);
-    c.gsum_dx = gs * dx;
-    c.ndim = ndim;
-    return c;
-}
-
-// One leaf cell of courant_fine (hydro/courant_fine.f90:120-160).
-__device__ __forceinline__ void courant_cell(const double u[5], const CourantK &c, double gf0, double &mass,
-                                             double &ekin, double &eint, double &dtmin)
-{
-    mass = mass + u[0] * c.vol;
-    ekin = ekin + u[4] * c.vol;
-    eint = eint + u[4] * c.vol;
-    const double rr = u[0] > c.smallr ? u[0] : c.smallr;
-    const double irr = rcp_nr(rr);
-    eint = eint - 0.5 * (u[1] * u[1]) * irr * c.vol;
-    eint = eint - 0.5 * (u[2] * u[2]) * irr * c.vol;
-    eint = eint - 0.5 * (u[3] * u[3]) * irr * c.vol;
-    const double d = cell_dt(u[0], u[1], u[2], u[3], u[4], c, gf0);
-    dtmin = d < dtmin ? d : dtmin;
-}
-
-// courant_fine of one cell for the mixed-precision kernel: the conservation
-// sums and the pressure recovery p=(gamma-1)(E-rho v^2/2) in FP64, the signal
-// speed and the cell's dt in FP32 (cmpdt's c_f = sqrt(c2+sqrt(c2^2)) with
-// c2 = a^2/2 and no magnetic field is a), the dt rounded to FP64 for the
-// min-reduction.
-__device__ __forceinline__ void courant_cell_mixed(const double u[5], const CourantK &c, double &mass, double &ekin,
-                                                   double &eint, double &dtmin)
-{
-    mass = mass + u[0] * c.vol;
-    ekin = ekin + u[4] * c.vol;
-    const double rr = u[0] > c.smallr ? u[0] : c.smallr;
-    const double ir = rcp_nr(rr);
-    const double ke = 0.5 * (u[1] * u[1] + u[2] * u[2] + u[3] * u[3]) * ir;
-    eint = eint + (u[4] - ke) * c.vol;
-    const double pe = (c.gamma - 1.0) * (u[4] - ke), pf = rr * c.smallp;
-    const double p = pe > pf ? pe : pf;
-    const float irf = (float)ir;
-    const float cf = __builtin_amdgcn_sqrtf((float)(c.gamma * p) * irf);
-    const float ctot = (__builtin_fabsf((float)u[1] * irf) + cf) + (__builtin_fabsf((float)u[2] * irf) + cf) +
-                       (__builtin_fabsf((float)u[3] * irf) + cf);
-    const float cfl = (float)c.courant_factor;
-    float grav = (float)c.gsum_dx * __builtin_amdgcn_rcpf(ctot * ctot);
-    grav = grav > 0.0001f ? grav : 0.0001f;
-    const double dtmax = c.courant_factor * c.dx / c.smallc;
-    const float dtcell = 2.0f * cfl * (float)c.dx *
-                         __builtin_amdgcn_rcpf(ctot * (1.0f + __builtin_amdgcn_sqrtf(1.0f + 2.0f * cfl * grav)));
-    const double d = dtmax < (double)dtcell ? dtmax : (double)dtcell;
-    dtmin = d < dtmin ? d : dtmin;
-}
 
 // Gather the conservative state of cell (i2,j2,k2) of the oct at window slot
 // value v, whose oct key is okey.  Boundary ghosts (v<0) follow
@@ -246,25 +98,6 @@ __device__ __forceinline__ void gather_cell(const double *__restrict__ uold, con
     gather_cell_m(uold, refined, v, okey, ndim, boxmin, boxmax, reflexive_mask(btype), c, u, rf);
 }
 
-template <typename T>
-__device__ __forceinline__ HydroK<T> make_k(const double dt, double dx, double gamma, double smallr, double smallc2,
-                                            double courant_factor, double smax_cap, int use_smax, int slope,
-                                            int riemann)
-{
-    HydroK<T> k;
-    k.gamma = T(gamma);
-    k.smallr = T(smallr);
-    k.smallc2 = T(smallc2 > 0x1p-900 ? smallc2 : 0x1p-900);
-    k.smallp_trace = T(smallr * smallc2);
-    k.smallp_riem = T(smallc2 / gamma);
-    k.entho = T(1.0 / (gamma - 1.0));
-    k.dtdx = T(dt / dx);
-    k.smax_cap = T(use_smax ? smax_cap : courant_factor * dx / dt);
-    k.slope_type = slope;
-    k.riemann = riemann;
-    return k;
-}
-
 // Positivity-preserving 27-point slope (slope_type 3, umuscl.f90:2207-2270)
 // for variable n of the cell at ring index (s0, pc), returned halved like
 // slope_half: the centred differences are formed as (q+ - q-)/4 = dfx/2, so
@@ -303,67 +136,10 @@ __device__ __forceinline__ void slope27(const T (*sq)[5][NP], int sm, int s0, in
     dq3[2] = slop * dfz;
 }
 
-// Coarse-fine refluxing, godfine1 (hydro/godunov_fine.f90:894-1052): a face
-// between a cell of the level and an interpolated ghost cell sends -flux/2^ndim
-// (ghost on the low side) or +flux/2^ndim (ghost on the high side) to the
-// ghost's parent cell.  Three ways:
-// - racc null: FP64 atomics into the parent cell of unew;
-// - racc, rdet 0: FP64 atomics into the ghost's accumulator racc[5 g];
-// either way the order of the contributions to one parent cell is not fixed
-// (last-bit differences from run to run and from the serial reference);
-// - racc, rdet 1 (deterministic mode): a plain store into the face's own slot
-//   racc[5 (kReluxSlots g + slot)], slot = 4 side + sub (side: the ghost oct's
-//   face, -x +x -y +y -z +z; sub: which of its 2^(ndim-1) cells), one writer
-//   per slot; k_reflux_fold then adds the slots in slot order.
-constexpr int kRefluxSlots = kRefluxSlotsPerGhost;
-__device__ __forceinline__ void reflux_add(double *unew, const int32_t *ghost_parent, int ngridmax, int vghost,
-                                           double sign, const double F[5], int ttd, double *racc = nullptr,
-                                           int rdet = 0, int slot = 0, bool accumulate = false)
-{
-    const int gi = vghost - ngridmax - 1;
-    if (racc) {
-        const double w = 1.0 / (double)ttd;
-        if (rdet) {
-            // accumulate: the diffusion pass adds to the slot the Godunov launch wrote
-            double *q = racc + 5 * ((size_t)gi * kRefluxSlots + slot);
-#pragma unroll
-            for (int n = 0; n < 5; n++) q[n] = accumulate ? q[n] + sign * (F[n] * w) : sign * (F[n] * w);
-            return;
-        }
-#pragma unroll
-        for (int n = 0; n < 5; n++) atomicAdd(racc + 5 * (size_t)gi + n, sign * (F[n] * w));
-        return;
-    }
-    const int igrid = ghost_parent[2 * gi], icell = ghost_parent[2 * gi + 1];
-    if (igrid <= 0) return;  // parent missing: rh_build_nbor reported it
-    const double w = 1.0 / (double)ttd;
-    double *p = unew + (size_t)(igrid - 1) * 5 * ttd + (icell - 1);
-#pragma unroll
-    for (int n = 0; n < 5; n++) atomicAdd(p + n * ttd, sign * (F[n] * w));
-}
-
-// The summed refluxes q (already weighted by 1/2^ndim, with their signs) of
-// one ghost oct: into its accumulator, or into its parent cell of unew.
-__device__ __forceinline__ void reflux_flush(double *unew, const int32_t *ghost_parent, int ngridmax, int vghost,
-                                             const double q[5], int ttd, double *racc)
-{
-    const int gi = vghost - ngridmax - 1;
-    if (racc) {
-#pragma unroll
-        for (int n = 0; n < 5; n++) atomicAdd(racc + 5 * (size_t)gi + n, q[n]);
-        return;
-    }
-    const int igrid = ghost_parent[2 * gi], icell = ghost_parent[2 * gi + 1];
-    if (igrid <= 0) return;
-    double *p = unew + (size_t)(igrid - 1) * 5 * ttd + (icell - 1);
-#pragma unroll
-    for (int n = 0; n < 5; n++) atomicAdd(p + n * ttd, q[n]);
-}
-
-// Loads of the next plane's P-phase cells issued a plane ahead, per precision
-// (FP32: the per-level kernel only; it runs at two waves per SIMD with them,
-// measured 4% faster at 256^3 than at three without, while the work-list
-// kernel keeps four waves per SIMD).
+// Loads of the next plane's P-phase cells issued a plane ahead (the FP32
+// per-level kernel; it runs at two waves per SIMD with them, measured 4% faster
+// at 256^3 than at three without, while the work-list kernel keeps four waves
+// per SIMD).
 // The z march unrolled by two planes.
 #ifndef RH_MARCH_UNROLL2
 #define RH_MARCH_UNROLL2 0
@@ -372,9 +148,6 @@ __device__ __forceinline__ void reflux_flush(double *unew, const int32_t *ghost_
 // boundary-ghost synthesis (a uniform branch per launch).
 #ifndef RH_FAST_FETCH
 #define RH_FAST_FETCH 1
-#endif
-#ifndef RH_PREFETCH_F64
-#define RH_PREFETCH_F64 1
 #endif
 #ifndef RH_PREFETCH_F32
 #define RH_PREFETCH_F32 1
@@ -385,11 +158,10 @@ __device__ __forceinline__ void reflux_flush(double *unew, const int32_t *ghost_
 #ifndef RH_PAIR_WRITES
 #define RH_PAIR_WRITES 1
 #endif
-// Whole-line stores: the FP64 kernels (writes 1.30x -> 0.97x of the
-// algorithmic bytes, the same time), the FP32 per-level kernel and the FP32
-// specialised work-list kernel (serving): the mixed kernel 0.624 -> 0.581 ms
-// at 256^3, serving's mixed capacity +7%; the FP32 general work-list kernel
-// (AMR) measured 7.6% slower with them and stores each half as it comes.
+// Whole-line stores: the FP32 per-level kernel and the FP32 specialised
+// work-list kernel (serving): the mixed kernel 0.624 -> 0.581 ms at 256^3,
+// serving's mixed capacity +7%; the FP32 general work-list kernel (AMR)
+// measured 7.6% slower with them and stores each half as it comes.
 template <typename T, bool WL, bool GEN> constexpr bool pair_writes()
 {
     return RH_PAIR_WRITES && (sizeof(T) == 8 || !WL || !GEN);
@@ -451,14 +223,14 @@ template <int BX, int BY, int RS, int NS> constexpr bool brick_hw()
     return (4 * BX * BY) % 64 == 0 && (2 * BX + 2) * (2 * BY + 2) - 4 * BX * BY <= 64 && RS == 3 && NS == 2;
 }
 
-// The next-plane prefetch: the HLLC variants of the FP64 kernels and of the
-// FP32 per-level kernel, with a thread for every cell of the P-phase ring.
+// The next-plane prefetch: the HLLC variants of the FP32 per-level kernel, with
+// a thread for every cell of the P-phase ring.
 template <int BX, int BY, typename T, int RS, int NS, bool WL> constexpr bool brick_prefetch()
 {
     constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY, NI = 4 * BX * BY;
     constexpr bool HW = brick_hw<BX, BY, RS, NS>();
     constexpr int NRING = HW ? 4 * (BX + BY) : 2 * (CX + CY);
-    return (sizeof(T) == 8 ? RH_PREFETCH_F64 : RH_PREFETCH_F32 && !WL) && RS == 3 && NS == 2 &&
+    return sizeof(T) == 4 && RH_PREFETCH_F32 && !WL && RS == 3 && NS == 2 &&
            (HW ? NRING <= NT - NI : NRING <= NT);
 }
 
@@ -520,14 +292,10 @@ template <int BX, int BY, int BZ, typename T, int NS> constexpr bool sep_flux()
 // values through LDS (UBL) pay in the FP32 kernel, whose three waves per SIMD
 // leave no registers to load them early (a load at the update waits, by the
 // in-order memory counter, for the next-plane prefetch issued before it): at
-// 256^3 the mixed kernel 0.666 -> 0.618 ms.  The general FP64 body loads them
-// early into registers (through LDS behind a runtime test it measured 4%
-// slower in the AMR work-list step: the compiler then waits for the early
-// loads of the other path); the specialised FP64 body (GEN = false, launched
-// only where the update adds to uold) takes them through LDS.
+// 256^3 the mixed kernel 0.666 -> 0.618 ms.
 template <int BX, int BY, int BZ, typename T, int RS, int NS, bool WL, bool GEN>
 using BrickLds = BrickSmem<BX, BY, BZ, T, NS, sep_flux<BX, BY, BZ, T, NS>(), brick_waves<BX, BY, BZ, T, WL>(),
-                           brick_prefetch<BX, BY, T, RS, NS, WL>() && (sizeof(T) == 4 || !GEN),
+                           brick_prefetch<BX, BY, T, RS, NS, WL>(),
                            pair_writes<T, WL, GEN>()>;
 
 __device__ __forceinline__ int ring_slot2(int t) { return t & 1; }
@@ -541,8 +309,7 @@ __device__ __forceinline__ int ring_slot3(int t) { return (t + 3) % 3; }
 // GEN = false compiles the body for a level that is periodic in every
 // dimension, has no refined cell and no coarse-fine faces (every uniform
 // level): without the boundary-ghost gather, the refined-face zeroing and the
-// reflux code, the FP64 kernel needs 224 instead of 245 VGPRs and no SGPR
-// spills (39 with them), and runs 2-3% faster.  The launch checks the level.
+// reflux code.  The launch checks the level.
 template <int BX, int BY, int BZ, typename T, int RS, int NS, bool WL, bool GEN = true, typename A>
 __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY, BZ, T, RS, NS, WL, GEN> &sm,
                                            const int part = -1, const int pslot = -1)
@@ -724,11 +491,11 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
         cell_load3(r, u, rf);
         fl = r.flip;
     };
-    // prefetch a plane ahead (about 45 more VGPRs, load latency hidden) in the
-    // HLLC variants: the FP64 kernels, and the FP32 per-level kernel, which
-    // drops to two waves per SIMD with it and is faster for it; the FP32
-    // work-list kernel and the other variants load at use, as they would
-    // spill or lose waves (it also needs a thread for every ring cell)
+    // prefetch a plane ahead (load latency hidden) in the HLLC variants of the
+    // FP32 per-level kernel, which drops to two waves per SIMD with it and is
+    // faster for it; the work-list kernel and the other variants load at use,
+    // as they would spill or lose waves (it also needs a thread for every
+    // ring cell)
     constexpr bool PF = brick_prefetch<BX, BY, T, RS, NS, WL>();
     double u_o[5], u_r[5];
     uint8_t rf_o, rf_r = 0;
@@ -812,13 +579,13 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
         rotate(qcol_p);
     }
     // courant_fine of the state written (the dt of the next step), when asked
-    // for: the FP64 kernel and the FP32 per-level kernel take each leaf
-    // cell's new state as they store it; the FP32 work-list kernel re-reads
-    // the brick's cells after the march (RH_COURANT_IN_UPDATE_F32)
+    // for: taken from each leaf cell's new state as it is stored; the FP32
+    // work-list kernel re-reads the brick's cells after the march
+    // (RH_COURANT_IN_UPDATE_F32)
     constexpr bool CU = sizeof(T) == 8 || (RH_COURANT_IN_UPDATE_F32 && !WL);
     const CourantK ck = make_courant_k(a.dx, 3, a.gamma, a.smallr, a.smallc2, a.courant_factor, gvec);
-    const double gf0 = grav_factor0(ck);
-    double c_mass = 0.0, c_ekin = 0.0, c_eint = 0.0, c_dt = a.dx / ck.smallc;
+    // c_dt: the smallest dt (FP32), the largest summed signal speed (FP64)
+    double c_mass = 0.0, c_ekin = 0.0, c_eint = 0.0, c_dt = sizeof(T) == 8 ? 0.0 : a.dx / ck.smallc;
     // one plane of the march; par = t & 1 (the ring slot of plane t when NS == 2)
     auto march = [&](const int t, const int par) __attribute__((always_inline)) {
         const int st = NS == 3 ? ring_slot3(t) : par;
@@ -1068,7 +835,7 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
                         if constexpr (sizeof(T) == 4)
                             courant_cell_mixed(un, ck, c_mass, c_ekin, c_eint, c_dt);
                         else
-                            courant_cell(un, ck, gf0, c_mass, c_ekin, c_eint, c_dt);
+                            c_dt = tmax(c_dt, courant_cell<3>(un, ck, ck.vol, c_mass, c_ekin, c_eint));
                     }
                 }
             }
@@ -1131,7 +898,7 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
         c_mass = wave_sum_n(c_mass, nv);
         c_ekin = wave_sum_n(c_ekin, nv);
         c_eint = wave_sum_n(c_eint, nv);
-        c_dt = wave_min_n(c_dt, nv);
+        c_dt = sizeof(T) == 8 ? wave_max_n(c_dt, nv) : wave_min_n(c_dt, nv);
         __syncthreads();
         double *red = (double *)&sf[0][0][0];
         const int w = tid >> 6;
@@ -1148,8 +915,12 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
                 m += red[4 * i];
                 e += red[4 * i + 1];
                 ei += red[4 * i + 2];
-                d = red[4 * i + 3] < d ? red[4 * i + 3] : d;
+                if constexpr (sizeof(T) == 8)
+                    d = tmax(red[4 * i + 3], d);
+                else
+                    d = red[4 * i + 3] < d ? red[4 * i + 3] : d;
             }
+            if constexpr (sizeof(T) == 8) d = signal_dt(d, ck);
             const int ps = pslot >= 0 ? pslot : bid;
             a.cpart[4 * ps + 0] = m;
             a.cpart[4 * ps + 1] = e;
@@ -1167,35 +938,8 @@ __global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2),
     k_godunov3d(const GodArgs a)
 {
     __shared__ BrickLds<BX, BY, BZ, T, RS, NS, false, GEN> sm;
-    // XCD-aware brick assignment: consecutive bricks to the same XCD so that
-    // their shared halo octs meet in that XCD's L2.
-    int bid = blockIdx.x;
-    int part = -1, pslot = bid;
-    if (a.xcd_remap && a.nsplit == 0) {
-        const int nb = gridDim.x, x = bid & 7, l = bid >> 3;
-        const int q = nb >> 3, r = nb & 7;
-        bid = x * q + (x < r ? x : r) + l;
-        pslot = bid;
-    } else if (a.xcd_remap) {
-        // the last nsplit bricks of each XCD's range run as two work items,
-        // one per half of the brick's z layers, so that the final round of
-        // workgroups on the XCD is half as long
-        const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
-        const int q = a.nbricks >> 3, r = a.nbricks & 7, m = a.nsplit;
-        const int start = x * q + (x < r ? x : r), count = q + (x < r ? 1 : 0);
-        if (l >= count + m) return;
-        if (l < count - m) {
-            bid = start + l;
-            pslot = bid;
-        } else {
-            const int j = l - (count - m);
-            bid = start + count - m + (j >> 1);
-            part = j & 1;
-            // Courant partial of the upper half: after the nbricks whole-brick slots
-            pslot = part == 0 ? bid : a.nbricks + x * m + (j >> 1);
-        }
-    }
-    if (bid >= a.nbricks) return;
+    int bid, part, pslot;
+    if (!level_item(a, bid, part, pslot)) return;
     brick_body<BX, BY, BZ, T, RS, NS, false, GEN>(a, bid, sm, part, pslot);
 }
 
@@ -1297,13 +1041,46 @@ __global__ void __launch_bounds__(256) k_godunov1d(const God1Args a)
 // ---------------------------------------------------------------------------
 constexpr int kCourantThreads = 256;
 
+// The block's partials {mass, ekin, eint, dt} in a fixed order; dt_of turns the
+// block's largest signal speed into its dt.
+template <typename F>
+__device__ __forceinline__ void courant_block(double mass, double ekin, double eint, double sig, F dt_of,
+                                              double *__restrict__ part)
+{
+    __shared__ double red[kCourantThreads / 64][4];
+    mass = wave_sum(mass);
+    ekin = wave_sum(ekin);
+    eint = wave_sum(eint);
+    sig = wave_max(sig);
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    if (l == 0) {
+        red[w][0] = mass;
+        red[w][1] = ekin;
+        red[w][2] = eint;
+        red[w][3] = sig;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s0 = 0, s1 = 0, s2 = 0, m = red[0][3];
+        for (int i = 0; i < kCourantThreads / 64; i++) {
+            s0 += red[i][0];
+            s1 += red[i][1];
+            s2 += red[i][2];
+            m = red[i][3] > m ? red[i][3] : m;
+        }
+        part[4 * blockIdx.x + 0] = s0;
+        part[4 * blockIdx.x + 1] = s1;
+        part[4 * blockIdx.x + 2] = s2;
+        part[4 * blockIdx.x + 3] = dt_of(m);
+    }
+}
+
 template <int TTD>
 __global__ void __launch_bounds__(kCourantThreads) k_courant(const double *__restrict__ uold,
                                                              const uint8_t *__restrict__ refined, int head, int noct,
                                                              const CourantK c, double *__restrict__ part)
 {
-    double mass = 0, ekin = 0, eint = 0, dtmin = c.dx / c.smallc;
-    const double gf0 = grav_factor0(c);
+    double mass = 0, ekin = 0, eint = 0, sig = 0;
     constexpr int ttd = TTD, stride = 5 * TTD;
     const long ncell = (long)noct * ttd;
     const long step = (long)gridDim.x * blockDim.x;
@@ -1327,41 +1104,20 @@ __global__ void __launch_bounds__(kCourantThreads) k_courant(const double *__res
         }
 #pragma unroll
         for (int k = 0; k < U; k++)
-            if (leaf[k]) courant_cell(u[k], c, gf0, mass, ekin, eint, dtmin);
+            if (leaf[k])
+                sig = tmax(sig, courant_cell < TTD == 8 ? 3 : 1 > (u[k], c, c.vol, mass, ekin, eint));
     }
-    __shared__ double red[kCourantThreads / 64][4];
-    mass = wave_sum(mass);
-    ekin = wave_sum(ekin);
-    eint = wave_sum(eint);
-    dtmin = wave_min(dtmin);
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    if (l == 0) {
-        red[w][0] = mass;
-        red[w][1] = ekin;
-        red[w][2] = eint;
-        red[w][3] = dtmin;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s0 = 0, s1 = 0, s2 = 0, m = red[0][3];
-        for (int i = 0; i < kCourantThreads / 64; i++) {
-            s0 += red[i][0];
-            s1 += red[i][1];
-            s2 += red[i][2];
-            m = red[i][3] < m ? red[i][3] : m;
-        }
-        part[4 * blockIdx.x + 0] = s0;
-        part[4 * blockIdx.x + 1] = s1;
-        part[4 * blockIdx.x + 2] = s2;
-        part[4 * blockIdx.x + 3] = m;
-    }
+    courant_block(mass, ekin, eint, sig, [&](double x) { return signal_dt(x, c); }, part);
 }
 
 // courant_fine over octs of several levels: c0 carries the level-independent
 // constants (c0.dx = finest dx, c0.gsum_dx = sum |g|), dx of an oct is
-// boxlen*2^-lev (the same value the host computes as boxlen/2^lev).  MIXED:
-// the cell's signal speed and dt in FP32, as the mixed-precision kernels'
-// fused reduction (courant_cell_mixed).
+// boxlen*2^-lev (the same value the host computes as boxlen/2^lev).  Without
+// gravity dt = dx / (signal speed) times a constant, and dx scales by powers
+// of two, so the block reduces max ctot 2^lev (exact) and takes one dt of it;
+// with gravity (and in FP32) each cell's dt is formed and -dt reduced.  MIXED:
+// the signal speed and dt in FP32, as the mixed-precision kernels' fused
+// reduction (courant_cell_mixed).
 template <bool MIXED>
 __global__ void __launch_bounds__(kCourantThreads) k_courant_ml(const double *__restrict__ uold,
                                                                 const uint8_t *__restrict__ refined,
@@ -1369,51 +1125,41 @@ __global__ void __launch_bounds__(kCourantThreads) k_courant_ml(const double *__
                                                                 const CourantK c0, double boxlen,
                                                                 double *__restrict__ part)
 {
-    double mass = 0, ekin = 0, eint = 0, dtmin = c0.dx / c0.smallc;
-    const double gf0 = grav_factor0(c0);
+    const bool percell = MIXED || c0.gsum_dx != 0.0;
+    double mass = 0, ekin = 0, eint = 0, dtmin = c0.dx / c0.smallc, sig = 0.0;
     const long ncell = (long)noct * 8;
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < ncell; i += (long)gridDim.x * blockDim.x) {
         const long o = (long)(head - 1) + i / 8;
         const int ind = (int)(i % 8);
         if (refined[o * 8 + ind]) continue;
         CourantK c = c0;
-        const double dx = __builtin_ldexp(boxlen, -lev[o]);
+        const int l = lev[o];
+        const double dx = __builtin_ldexp(boxlen, -l);
         c.dx = dx;
         c.vol = dx * dx * dx;
         c.gsum_dx = c0.gsum_dx * dx;
         const double *p = uold + o * 40 + ind;
         const double u[5] = {p[0], p[8], p[16], p[24], p[32]};
-        if constexpr (MIXED)
+        if constexpr (MIXED) {
             courant_cell_mixed(u, c, mass, ekin, eint, dtmin);
-        else
-            courant_cell(u, c, gf0, mass, ekin, eint, dtmin);
-    }
-    __shared__ double red[kCourantThreads / 64][4];
-    mass = wave_sum(mass);
-    ekin = wave_sum(ekin);
-    eint = wave_sum(eint);
-    dtmin = wave_min(dtmin);
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    if (l == 0) {
-        red[w][0] = mass;
-        red[w][1] = ekin;
-        red[w][2] = eint;
-        red[w][3] = dtmin;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s0 = 0, s1 = 0, s2 = 0, m = red[0][3];
-        for (int i = 0; i < kCourantThreads / 64; i++) {
-            s0 += red[i][0];
-            s1 += red[i][1];
-            s2 += red[i][2];
-            m = red[i][3] < m ? red[i][3] : m;
+        } else {
+            const double ctot = courant_cell<3>(u, c, c.vol, mass, ekin, eint);
+            if (percell)
+                dtmin = tmin(dtmin, signal_dt(ctot, c));
+            else
+                sig = tmax(sig, __builtin_ldexp(ctot, l));
         }
-        part[4 * blockIdx.x + 0] = s0;
-        part[4 * blockIdx.x + 1] = s1;
-        part[4 * blockIdx.x + 2] = s2;
-        part[4 * blockIdx.x + 3] = m;
     }
+    courant_block(
+        mass, ekin, eint, percell ? -dtmin : sig,
+        [&](double x) {
+            if (percell) return -x;
+            if (!(x > 0.0)) return c0.dx / c0.smallc;  // no leaf cell
+            CourantK c = c0;
+            c.dx = boxlen;
+            return signal_dt(x, c);
+        },
+        part);
 }
 
 // Block b of a grid of nb blocks renumbered so that the blocks the hardware
@@ -1788,6 +1534,8 @@ hipError_t launch_upload(double *uold, const int32_t *father, int head, int noct
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
+// (a build for one workload may name fewer)
+#ifndef RH_BRICK_SHAPES
 #define RH_BRICK_SHAPES(X) \
     X(7, 7, 8)             \
     X(7, 7, 16)            \
@@ -1801,6 +1549,7 @@ hipError_t launch_upload(double *uold, const int32_t *father, int head, int noct
     X(3, 3, 4)             \
     X(3, 3, 8)             \
     X(1, 1, 1)
+#endif
 
 bool brick_shape_supported(int bx, int by, int bz)
 {
@@ -1811,66 +1560,36 @@ bool brick_shape_supported(int bx, int by, int bz)
     return false;
 }
 
-// Kernel launch, optionally with start/stop events tracked by the dispatch
-// itself (hipExtLaunchKernelGGL): timing without separate event packets on
-// the stream between the kernels of a step.
-template <typename K, typename... Args>
-static void launch_ev(K kernel, dim3 g, dim3 b, hipStream_t s, hipEvent_t e0, hipEvent_t e1, Args... args)
-{
-    if (e0 || e1)
-        hipExtLaunchKernelGGL(kernel, g, b, 0, s, e0, e1, 0, args...);
-    else
-        hipLaunchKernelGGL(kernel, g, b, 0, s, args...);
-}
-
-// Half-brick split of the final round (GodArgs::nsplit).  With equal work
-// per brick, q bricks per XCD on `slots` concurrent workgroups per XCD run in
-// ceil(q / slots) rounds; when the last round holds rem = q mod slots <=
-// slots/2 bricks, running those rem bricks as 2 rem half-bricks ends the
-// launch about half a round earlier (e.g. 352 bricks per XCD on 64 slots:
-// 5.53 instead of 6 rounds, by a list-scheduling model).
-#ifndef RH_TAIL_SPLIT
-#define RH_TAIL_SPLIT 1
-#endif
-template <typename K> static int tail_split(K kernel, int nthreads, const GodArgs &a)
-{
-    if (!RH_TAIL_SPLIT || !a.xcd_remap || a.reflux) return 0;
-    static std::map<const void *, int> occ_cache;
-    static int cus_per_xcd = 0;
-    if (!cus_per_xcd) {
-        int dev = 0, ncu = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return 0;
-        cus_per_xcd = ncu / 8 > 0 ? ncu / 8 : 1;
-    }
-    auto it = occ_cache.find((const void *)kernel);
-    int occ;
-    if (it == occ_cache.end()) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, nthreads, 0) != hipSuccess) occ = 0;
-        occ_cache[(const void *)kernel] = occ;
-    } else {
-        occ = it->second;
-    }
-    const int slots = occ * cus_per_xcd, q = a.nbricks >> 3;
-    if (slots <= 1 || q <= 0) return 0;
-    const int rem = q % slots;
-    return rem > 0 && 2 * rem <= slots ? rem : 0;
-}
-
-template <typename K>
-static void launch_brick(K kernel, int nt, const GodArgs &a0, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
-                         int *nparts)
-{
-    GodArgs a = a0;
-    a.nsplit = tail_split(kernel, nt, a);
-    const int q = a.nbricks >> 3, r = a.nbricks & 7;
-    const dim3 g(a.nsplit ? 8 * (q + (r ? 1 : 0) + a.nsplit) : a.nbricks), b(nt);
-    if (nparts) *nparts = a.nbricks + 8 * a.nsplit;
-    launch_ev(kernel, g, b, s, e0, e1, a);
-}
-
 int g_specialized = 1;
+
+// The objects of rh_brick64.hip, one per set of brick shapes
+#define RH_SETS(X) X(0) X(1) X(2) X(3) X(4) X(5)
+#define RH_DECL(N)                                                                                               \
+    bool brick64_level_##N(const GodArgs &a, int bx, int by, int bz, bool gen, hipStream_t s, hipEvent_t e0,      \
+                           hipEvent_t e1, int *nparts);                                                          \
+    bool brick64_list_##N(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, bool gen, hipStream_t s);
+RH_SETS(RH_DECL)
+#undef RH_DECL
+
+hipError_t launch_brick64(const GodArgs &a, int bx, int by, int bz, bool gen, hipStream_t s, hipEvent_t e0,
+                          hipEvent_t e1, int *nparts)
+{
+#define RH_TRY(N) \
+    if (brick64_level_##N(a, bx, by, bz, gen, s, e0, e1, nparts)) return hipGetLastError();
+    RH_SETS(RH_TRY)
+#undef RH_TRY
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_brick64_wl(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, bool gen,
+                             hipStream_t s)
+{
+#define RH_TRY(N) \
+    if (brick64_list_##N(w, nblocks, bx, by, bz, riemann, gen, s)) return hipGetLastError();
+    RH_SETS(RH_TRY)
+#undef RH_TRY
+    return hipErrorInvalidValue;
+}
 
 hipError_t launch_godunov3d(const GodArgs &a, int bx, int by, int bz, int prec, hipStream_t s, hipEvent_t e0,
                             hipEvent_t e1, int *nparts)
@@ -1878,8 +1597,12 @@ hipError_t launch_godunov3d(const GodArgs &a, int bx, int by, int bz, int prec, 
     if (nparts) *nparts = a.nbricks > 0 ? a.nbricks : 0;
     if (a.nbricks <= 0) return hipSuccess;
     // the specialised body: periodic in every dimension, no refined cells,
-    // no refluxes
-    const bool gen = a.bnd || a.any_ref || a.reflux || a.ubase != a.uold || !g_specialized;
+    // no refluxes, (FP64) no gravity
+    bool gen = a.bnd || a.any_ref || a.reflux || a.ubase != a.uold || !g_specialized;
+    if (prec == 0 && a.slope != 3) {
+        gen = gen || a.g[0] != 0.0 || a.g[1] != 0.0 || a.g[2] != 0.0;
+        return launch_brick64(a, bx, by, bz, gen, s, e0, e1, nparts);
+    }
 #define RH_LAUNCH_SHAPE(A, B, C)                                                                         \
     if (bx == A && by == B && bz == C) {                                                                 \
         constexpr int nt = (2 * A + 2) * (2 * B + 2);                                                     \
@@ -1889,20 +1612,11 @@ hipError_t launch_godunov3d(const GodArgs &a, int bx, int by, int bz, int prec, 
             else                                                                                         \
                 launch_brick(k_godunov3d<A, B, C, float, 0, 3>, nt, a, s, e0, e1, nparts);               \
         } else if (a.riemann == 3 && !gen) {                                                             \
-            if (prec == 0)                                                                               \
-                launch_brick(k_godunov3d<A, B, C, double, 3, 2, false>, nt, a, s, e0, e1, nparts);       \
-            else                                                                                         \
-                launch_brick(k_godunov3d<A, B, C, float, 3, 2, false>, nt, a, s, e0, e1, nparts);        \
+            launch_brick(k_godunov3d<A, B, C, float, 3, 2, false>, nt, a, s, e0, e1, nparts);            \
         } else if (a.riemann == 3) {                                                                     \
-            if (prec == 0)                                                                               \
-                launch_brick(k_godunov3d<A, B, C, double, 3, 2>, nt, a, s, e0, e1, nparts);              \
-            else                                                                                         \
-                launch_brick(k_godunov3d<A, B, C, float, 3, 2>, nt, a, s, e0, e1, nparts);               \
+            launch_brick(k_godunov3d<A, B, C, float, 3, 2>, nt, a, s, e0, e1, nparts);                   \
         } else {                                                                                         \
-            if (prec == 0)                                                                               \
-                launch_brick(k_godunov3d<A, B, C, double, 0, 2>, nt, a, s, e0, e1, nparts);              \
-            else                                                                                         \
-                launch_brick(k_godunov3d<A, B, C, float, 0, 2>, nt, a, s, e0, e1, nparts);               \
+            launch_brick(k_godunov3d<A, B, C, float, 0, 2>, nt, a, s, e0, e1, nparts);                   \
         }                                                                                                \
         return hipGetLastError();                                                                        \
     }
@@ -1919,6 +1633,7 @@ hipError_t launch_godunov3d_wl(const WorkList &w, int bx, int by, int bz, int sl
     int maxr = 0;
     for (int r = 0; r < 8; r++) maxr = w.range[r + 1] - w.range[r] > maxr ? w.range[r + 1] - w.range[r] : maxr;
     const int nblocks = 8 * maxr;
+    if (prec == 0 && slope != 3) return launch_brick64_wl(w, nblocks, bx, by, bz, riemann, gen, s);
 #define RH_LAUNCH_WL(A, B, C)                                                                            \
     if (bx == A && by == B && bz == C) {                                                                 \
         constexpr int nt = (2 * A + 2) * (2 * B + 2);                                                     \
@@ -1929,20 +1644,11 @@ hipError_t launch_godunov3d_wl(const WorkList &w, int bx, int by, int bz, int sl
             else                                                                                         \
                 hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, float, 0, 3>), g, b, 0, s, w);               \
         } else if (riemann == 3 && !gen) {                                                               \
-            if (prec == 0)                                                                               \
-                hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, double, 3, 2, false>), g, b, 0, s, w);       \
-            else                                                                                         \
-                hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, float, 3, 2, false>), g, b, 0, s, w);        \
+            hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, float, 3, 2, false>), g, b, 0, s, w);            \
         } else if (riemann == 3) {                                                                       \
-            if (prec == 0)                                                                               \
-                hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, double, 3, 2>), g, b, 0, s, w);              \
-            else                                                                                         \
-                hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, float, 3, 2>), g, b, 0, s, w);               \
+            hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, float, 3, 2>), g, b, 0, s, w);                   \
         } else {                                                                                         \
-            if (prec == 0)                                                                               \
-                hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, double, 0, 2>), g, b, 0, s, w);              \
-            else                                                                                         \
-                hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, float, 0, 2>), g, b, 0, s, w);               \
+            hipLaunchKernelGGL((k_godunov3d_wl<A, B, C, float, 0, 2>), g, b, 0, s, w);                   \
         }                                                                                                \
         return hipGetLastError();                                                                        \
     }

@@ -1,0 +1,276 @@
+// FP64 physics of the brick kernels: the routines of rh_physics.h in forms that
+// take fewer instructions.  The FP64 kernels are bound by the issue of their
+// vector instructions, so each routine here is written for its count of issue
+// slots and the length of its dependent chain; the results agree with the
+// reference's expressions to rounding.  (The mixed-precision kernels use
+// rh_physics.h: their FP32 results depend on every rounding.)
+#pragma once
+#include "rh_physics.h"
+
+namespace rh {
+
+__device__ __forceinline__ double tfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// 1/b from the hardware reciprocal (about 2^-24) refined by one third-order
+// step, r (1 + e + e^2) with e = 1 - b r: three dependent FMAs instead of the
+// four of two Newton steps (rcp_nr), the remaining error e^3 far below an ulp, so
+// the result is off by its last rounding only.
+__device__ __forceinline__ double rcp_h(double b)
+{
+    const double r = __builtin_amdgcn_rcp(b);
+    const double e = __builtin_fma(-b, r, 1.0);
+    return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+// 1/sqrt(x) for x in [2^-1020, 2^1020]: the hardware reciprocal square root
+// refined by one third-order step, y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2
+// (five dependent operations; the remaining error is of the order of e^3).
+__device__ __forceinline__ double rsq_pos(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = __builtin_fma(-(x * y), y, 1.0);
+    return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+// max(sqrt(na/da), sqrt(nb/db)) for positive operands without a division: the
+// larger quotient is found by cross multiplication, and sqrt(n/d) = n/sqrt(n d)
+// takes one refined reciprocal square root.  Two sound speeds of a face cost
+// 19 issue slots this way against 35 as two refined reciprocals and a square
+// root.  The products are floored where sqrt would leave the normal range.
+__device__ __forceinline__ double sqrt_quot_max(double na, double da, double nb, double db)
+{
+    const bool a = na * db > nb * da;
+    const double n = a ? na : nb, d = a ? da : db;
+    return n * rsq_pos(__builtin_fmax(n * d, 0x1p-1020));
+}
+// sqrt(n/d): a sound speed from gamma*P and rho
+__device__ __forceinline__ double sound_speed64(double n, double d)
+{
+    return n * rsq_pos(__builtin_fmax(n * d, 0x1p-1020));
+}
+
+// ctoprim (prim_from_cons) of one cell: m = rho v gives the kinetic energy as
+// m.v/2, three operations fewer.  Returns 1/rho, which the predictor of the
+// same cell uses again.
+__device__ __forceinline__ double prim64(const double u[5], double q[5], double smallr, double smalle, double gm1,
+                                         const double gdt_half[3])
+{
+    const double r = u[0] > smallr ? u[0] : smallr;
+    const double ir = rcp_h(r);
+    const double vx = u[1] * ir, vy = u[2] * ir, vz = u[3] * ir;
+    const double s = __builtin_fma(u[3], vz, __builtin_fma(u[2], vy, u[1] * vx));
+    q[0] = r;
+    q[1] = vx + gdt_half[0];
+    q[2] = vy + gdt_half[1];
+    q[3] = vz + gdt_half[2];
+    q[4] = gm1 * tmax(__builtin_fma(-0.5, s, u[4]), smalle * r);
+    return ir;
+}
+
+// uslope (slope_half) from the differences a = q0-qm1 and b = qp1-q0, halved:
+// MinMod is half the median of a, b and 0; MonCen is the centred slope clamped
+// to [min(max(a,b),0), max(min(a,b),0)], an interval that is [0, min] or
+// [max, 0] where a and b agree in sign and only 0 where they do not.  min and
+// max are exact, so the values are those of slope_half, one or two
+// instructions sooner.
+__device__ __forceinline__ double slope64(int st, double a, double b)
+{
+    const double lo = tmin(a, b), hi = tmax(a, b);
+    if (st == 1) return 0.5 * tmax(lo, tmin(hi, 0.0));
+    const double c = (a + b) * 0.25;  // dcen/2
+    return tmax(tmin(c, tmax(lo, 0.0)), tmin(hi, 0.0));
+}
+// vel_bound_half from the same differences
+__device__ __forceinline__ double vel_bound64(double dqh, double rl, double a, double inv_r0, double rr, double b)
+{
+    const double lim = tmin(rl * fabs_(a), rr * fabs_(b)) * inv_r0;
+    return tcopysign(tmin(fabs_(dqh), lim), dqh);
+}
+
+// trace3d, hydro/umuscl.f90:860-1466, hydro part for one cell.
+// q: cell primitives; dqh[d][n]: halved slopes (the reference's 0.5*dq).
+// Outputs qp[d][n] (right state at the left interface) and qm[d][n] (left
+// state at the right interface).
+__device__ __forceinline__ void trace64(const double q[5], const double dqh[3][5], double qp[3][5], double qm[3][5],
+                                        const HydroK<double> &k, double inv_r)
+{
+    using T = double;
+    T r = q[0], u = q[1], v = q[2], w = q[3], p = q[4];
+    T drx = dqh[0][0], dux = dqh[0][1], dvx = dqh[0][2], dwx = dqh[0][3], dpx = dqh[0][4];
+    T dry = dqh[1][0], duy = dqh[1][1], dvy = dqh[1][2], dwy = dqh[1][3], dpy = dqh[1][4];
+    T drz = dqh[2][0], duz = dqh[2][1], dvz = dqh[2][2], dwz = dqh[2][3], dpz = dqh[2][4];
+    T divv = dux + dvy + dwz;
+    T sr0 = -u * drx - v * dry - w * drz - divv * r;
+    T su0 = -u * dux - v * duy - w * duz - dpx * inv_r;
+    T sv0 = -u * dvx - v * dvy - w * dvz - dpy * inv_r;
+    T sw0 = -u * dwx - v * dwy - w * dwz - dpz * inv_r;
+    T sp0 = -u * dpx - v * dpy - w * dpz - divv * k.gamma * p;
+    T ws[5];
+    ws[0] = r + sr0 * k.dtdx;
+    ws[1] = u + su0 * k.dtdx;
+    ws[2] = v + sv0 * k.dtdx;
+    ws[3] = w + sw0 * k.dtdx;
+    ws[4] = p + sp0 * k.dtdx;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+#pragma unroll
+        for (int n = 0; n < 5; n++) {
+            T h = dqh[d][n];
+            qp[d][n] = ws[n] - h;
+            qm[d][n] = ws[n] + h;
+        }
+    }
+    // The floors (a state below smallr or smallp falls back to the cell's
+    // value) rarely bite.  The smallest of the six states is ws - max|h|
+    // (rounding is monotonic, so the test is exact): a wave without a floored
+    // state skips the 12 compares and 24 selects.
+    const T hr = tmax(tmax(fabs_(drx), fabs_(dry)), fabs_(drz));
+    const T hp = tmax(tmax(fabs_(dpx), fabs_(dpy)), fabs_(dpz));
+    if (__builtin_expect(ws[0] - hr < k.smallr || ws[4] - hp < k.smallp_trace, 0)) {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            if (qp[d][0] < k.smallr) qp[d][0] = r;
+            if (qp[d][4] < k.smallp_trace) qp[d][4] = p;
+            if (qm[d][0] < k.smallr) qm[d][0] = r;
+            if (qm[d][4] < k.smallp_trace) qm[d][4] = p;
+        }
+    }
+}
+
+// riemann_hllc, hydro/godunov_utils.f90:638-857 (mass, momenta, energy fluxes).
+// Only the star state and the energy of the side that is sampled are formed;
+// the sampled values are those of the reference, which forms both.  The states
+// come from trace64, whose densities are at least smallr, and with the
+// pressure floor no sound speed is below smallc, so those two floors of the
+// reference's are not repeated.
+__device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
+{
+    // contraction is spelled out, so that every kernel that solves a face gets
+    // the same bits
+#pragma clang fp contract(off)
+    using T = double;
+    const T half = T(0.5);
+    T rl = ql[0];
+    T ul = ql[1], vl = ql[2], wl = ql[3];
+    T Pl = tmax(ql[4], rl * k.smallp_riem);
+    T rr = qr[0];
+    T ur = qr[1], vr = qr[2], wr = qr[3];
+    T Pr = tmax(qr[4], rr * k.smallp_riem);
+    // max(sqrt(a), sqrt(b)) = sqrt(max(a, b)): one root for the two sound speeds
+    T cmax = sqrt_quot_max(k.gamma * Pl, rl, k.gamma * Pr, rr);
+    T SL = tmin(ul, ur) - cmax;
+    T SR = tmax(ul, ur) + cmax;
+    T dl = ul - SL, dr = SR - ur;
+    T rcl = rl * dl, rcr = rr * dr;
+    T inv_den = rcp_h(tfma(rr, dr, rcl));
+    T num = (Pl - Pr) + tfma(rcr, ur, rcl * ul);
+    T ustar = num * inv_den;
+    T Ptotstar = tfma(rcl * rcr, ul - ur, tfma(rcr, Pl, rcl * Pr)) * inv_den;
+    // The reference samples, in this order: SL > 0 -> left state; ustar > 0
+    // -> left star state; SR > 0 -> right star state; else right state.  The
+    // side whose values are used is left exactly when SL > 0 or ustar > 0,
+    // and the star state is taken when SL <= 0 and (ustar > 0 or SR > 0); in
+    // both star cases the side is the reference's ustar > 0.  So one select
+    // of the side's six values and one of four values (state or star) give
+    // the reference's result (its chain costs three selects per value), and
+    // the total energy is formed for the sampled side only.
+    const bool sl_pos = SL > T(0), us_pos = ustar > T(0);
+    const bool left = sl_pos || us_pos;
+    const bool star = !sl_pos && (us_pos || SR > T(0));
+    T S = left ? SL : SR;
+    T rs = left ? rl : rr, us = left ? ul : ur, Ps = left ? Pl : Pr;
+    T vo = left ? vl : vr, wo = left ? wl : wr;
+    T es = tfma(half * rs, tfma(wo, wo, tfma(us, us, vo * vo)), Ps * k.entho);
+    T ds = S - us;
+    T inv_sd = rcp_h(tfma(-inv_den, num, S));  // 1/(S - ustar)
+    T rstar = rs * ds * inv_sd;
+    T etotstar = tfma(Ptotstar, ustar, tfma(ds, es, -(Ps * us))) * inv_sd;
+    T ro = star ? rstar : rs, uo = star ? ustar : us, Po = star ? Ptotstar : Ps, eo = star ? etotstar : es;
+    f[0] = ro * uo;
+    f[1] = tfma(f[0], uo, Po);
+    f[2] = f[0] * vo;
+    f[3] = f[0] * wo;
+    f[4] = (eo + Po) * uo;
+}
+
+// riemann_llf, hydro/godunov_utils.f90:338-485.
+__device__ __forceinline__ void llf64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
+{
+    using T = double;
+    T rl = ql[0], pl = tmax(ql[4], rl * k.smallp_riem);
+    T cl = sound_speed64(k.gamma * pl, rl);
+    T rr = qr[0], pr = tmax(qr[4], rr * k.smallp_riem);
+    T cr = sound_speed64(k.gamma * pr, rr);
+    T cmax = tmin(tmax(fabs_(ql[1]) + cl, fabs_(qr[1]) + cr), k.smax_cap);
+    T uL[5], uR[5];
+    side_state(ql, k.entho, uL);
+    side_state(qr, k.entho, uR);
+    T fL[5], fR[5];
+    fL[0] = ql[1] * uL[0];
+    fR[0] = qr[1] * uR[0];
+    fL[1] = ql[1] * uL[1] + ql[4];
+    fR[1] = qr[1] * uR[1] + qr[4];
+    fL[2] = ql[1] * uL[2];
+    fR[2] = qr[1] * uR[2];
+    fL[3] = ql[1] * uL[3];
+    fR[3] = qr[1] * uR[3];
+    fL[4] = ql[1] * (uL[4] + ql[4]);
+    fR[4] = qr[1] * (uR[4] + qr[4]);
+#pragma unroll
+    for (int n = 0; n < 5; n++) f[n] = T(0.5) * (fL[n] + fR[n] - cmax * (uR[n] - uL[n]));
+}
+
+// riemann_hll, hydro/godunov_utils.f90:486-637.
+__device__ __forceinline__ void hll64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
+{
+    using T = double;
+    T rl = ql[0], ul = ql[1], pl = tmax(ql[4], rl * k.smallp_riem);
+    T rr = qr[0], ur = qr[1], pr = tmax(qr[4], rr * k.smallp_riem);
+    T cmax = sqrt_quot_max(k.gamma * pl, rl, k.gamma * pr, rr);
+    T SL = tmax(tmin(tmin(ul, ur) - cmax, T(0)), -k.smax_cap);
+    T SR = tmin(tmax(tmax(ul, ur) + cmax, T(0)), k.smax_cap);
+    T uL[5], uR[5];
+    side_state(ql, k.entho, uL);
+    side_state(qr, k.entho, uR);
+    T fL[5], fR[5];
+    fL[0] = uL[1];
+    fR[0] = uR[1];
+    fL[1] = ql[4] + uL[1] * ql[1];
+    fR[1] = qr[4] + uR[1] * qr[1];
+    fL[2] = ql[1] * uL[2];
+    fR[2] = qr[1] * uR[2];
+    fL[3] = ql[1] * uL[3];
+    fR[3] = qr[1] * uR[3];
+    fL[4] = ql[1] * (uL[4] + ql[4]);
+    fR[4] = qr[1] * (uR[4] + qr[4]);
+    const T inv = rcp_h(SR - SL);  // SR - SL >= 2c > 0, the same for all five
+#pragma unroll
+    for (int n = 0; n < 5; n++) f[n] = (SR * fL[n] - SL * fR[n] + SR * SL * (uR[n] - uL[n])) * inv;
+}
+
+// cmpflxm for the solver RS (1 LLF, 2 HLL, 3 HLLC) with states already rotated
+// to the face normal: (rho, u_n, u_t1, u_t2, p).
+template <int RS> __device__ __forceinline__ void solve64(const double a[5], const double b[5], double g[5], const HydroK<double> &k)
+{
+    if constexpr (RS == 3)
+        hllc64(a, b, g, k);
+    else if constexpr (RS == 2)
+        hll64(a, b, g, k);
+    else
+        llf64(a, b, g, k);
+}
+template <int RS>
+__device__ __forceinline__ void face64(int idim, const double ql[5], const double qr[5], double f[5],
+                                       const HydroK<double> &k)
+{
+    const int ln = idim + 1, lt1 = idim == 0 ? 2 : 1, lt2 = idim == 2 ? 2 : 3;
+    const double a[5] = {ql[0], ql[ln], ql[lt1], ql[lt2], ql[4]};
+    const double b[5] = {qr[0], qr[ln], qr[lt1], qr[lt2], qr[4]};
+    double g[5];
+    solve64<RS>(a, b, g, k);
+    f[0] = g[0];
+    f[ln] = g[1];
+    f[lt1] = g[2];
+    f[lt2] = g[3];
+    f[4] = g[4];
+}
+
+}  // namespace rh
