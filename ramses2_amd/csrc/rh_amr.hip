@@ -136,7 +136,7 @@ int rh_amr_prepare(int levelmin, int levelmax, const int32_t *head, const int32_
     m.levels.clear();
     int end = -1;
     std::vector<GodArgs> descs;
-    std::vector<int2> items;
+    std::vector<int4> items;
     std::vector<std::array<int, 3>> shapes;  // brick shape of each level's descriptor
     std::vector<const LevelBricks *> lbs;    // bricks of each level's descriptor
     const double gz[3] = {0, 0, 0};
@@ -168,19 +168,25 @@ int rh_amr_prepare(int levelmin, int levelmax, const int32_t *head, const int32_
         for (size_t e = 0; e < d; e++) seen = seen || shapes[e] == shapes[d];
         if (seen) continue;
         AmrPlan::Group gr{shapes[d][0], shapes[d][1], shapes[d][2], (int)items.size(), 0};
+        long nb = 0;
+        for (size_t e = d; e < descs.size(); e++)
+            if (shapes[e] == shapes[d]) nb += descs[e].nbricks;
+        const int n = worklist_zsplit(nb, gr.bx, gr.by, gr.bz, 0);  // parts of each brick (few bricks)
         for (size_t e = d; e < descs.size(); e++)
             if (shapes[e] == shapes[d])
-                for (int b = 0; b < descs[e].nbricks; b++) items.push_back(make_int2((int)e, b));
+                for (int b = 0; b < descs[e].nbricks; b++)
+                    for (int k = 0; k < n; k++) items.push_back(make_int4((int)e, b, k, n));
         gr.count = (int)items.size() - gr.first;
         // one range of the items per XCD, of equal modelled work: the bricks
         // come in z-slab order, and a thin shell's bricks march fewer planes
         // where it lies flat in z, so equal counts leave the XCDs unequal
         std::vector<double> pre((size_t)gr.count + 1, 0.0);
         for (int i = 0; i < gr.count; i++) {
-            const int2 it = items[(size_t)gr.first + i];
+            const int4 it = items[(size_t)gr.first + i];
             const LevelBricks &lb = *lbs[it.x];
             const int zr = lb.h_zr.size() > (size_t)it.y ? lb.h_zr[it.y] : ((lb.bz - 1) << 16);
-            pre[i + 1] = pre[i] + brick_work(lb.bx, lb.by, 2.0 * ((zr >> 16) - (zr & 0xffff) + 1));
+            const int len = (zr >> 16) - (zr & 0xffff) + 1, m = len * (it.z + 1) / it.w - len * it.z / it.w;
+            pre[i + 1] = pre[i] + (m > 0 ? brick_work(lb.bx, lb.by, 2.0 * m) : 0.0);
         }
         gr.range[0] = 0;
         gr.range[8] = gr.count;
@@ -234,9 +240,9 @@ int rh_amr_prepare(int levelmin, int levelmax, const int32_t *head, const int32_
     m.nitems = (int)items.size();
     m.h_descs = both;
     RH_HIP_CHECK(dmalloc((void **)&m.d_descs, both.size() * sizeof(GodArgs)));
-    RH_HIP_CHECK(dmalloc((void **)&m.d_items, std::max<size_t>(items.size(), 1) * sizeof(int2)));
+    RH_HIP_CHECK(dmalloc((void **)&m.d_items, std::max<size_t>(items.size(), 1) * sizeof(int4)));
     RH_HIP_CHECK(hipMemcpyAsync(m.d_descs, both.data(), both.size() * sizeof(GodArgs), hipMemcpyHostToDevice, s.stream));
-    RH_HIP_CHECK(hipMemcpyAsync(m.d_items, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice, s.stream));
+    RH_HIP_CHECK(hipMemcpyAsync(m.d_items, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice, s.stream));
     // the courant pass writes one partial per block, up to red_cap blocks
     if (int r = ensure_partials(1024)) return r;
     // dt of the first step from the current state; time starts at 0

@@ -76,6 +76,7 @@ template <int BX, int BY, int BZ, int RS, bool GEN, typename A>
 __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, const int zhi, const int pslot,
                                         Brick64Lds<BX, BY, BZ, GEN> &sm)
 {
+#pragma clang fp contract(off)
     constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY, NI = 4 * BX * BY;
     constexpr int PX = 2 * BX + 4;
     constexpr int WX = BX + 2, WY = BY + 2, NW = WX * WY * (BZ + 2);
@@ -472,7 +473,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
         }
         if (interior) finish(thi, true);
     };
-    // (the upper half of a split brick may hold no layer)
+    // (a part of a brick may hold no layer)
     if (zlo <= zhi) {
         if constexpr (HW) {
             if (__builtin_amdgcn_readfirstlane(tid) < NI)

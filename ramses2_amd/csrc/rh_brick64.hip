@@ -30,29 +30,12 @@
 
 namespace rh {
 
-__device__ __forceinline__ void brick_layers(const int32_t *zrs, int bid, int bz, int part, int &zlo, int &zhi)
-{
-    // z layers of the brick that hold octs of the level
-    const int zr = zrs ? zrs[bid] : ((bz - 1) << 16);
-    zlo = zr & 0xffff;
-    zhi = zr >> 16;
-    if (part >= 0) {
-        // half of them (the lower half holds the middle one)
-        const int mid = (zlo + zhi) >> 1;
-        if (part == 0)
-            zhi = mid;
-        else
-            zlo = mid + 1;
-    }
-}
-
 template <int BX, int BY, int BZ, int RS, bool GEN>
 __global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2), kBrick64Waves) k_brick64(const GodArgs a)
 {
     __shared__ Brick64Lds<BX, BY, BZ, GEN> sm;
-    int bid, part, pslot, zlo, zhi;
-    if (!level_item(a, bid, part, pslot)) return;
-    brick_layers(a.zr, bid, BZ, part, zlo, zhi);
+    int bid, zlo, zhi, pslot;
+    if (!level_item(a, BZ, bid, zlo, zhi, pslot)) return;
     brick64<BX, BY, BZ, RS, GEN>(a, bid, zlo, zhi, pslot, sm);
 }
 
@@ -66,12 +49,13 @@ __global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2), kBrick64Waves) k_
     const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
     const int i = w.range[x] + l;
     if (i >= w.range[x + 1]) return;
-    const int2 it = w.items[i];
+    const int4 it = w.items[i];
     const int di = __builtin_amdgcn_readfirstlane(it.x), bid = __builtin_amdgcn_readfirstlane(it.y);
+    const int part = __builtin_amdgcn_readfirstlane(it.z), n = __builtin_amdgcn_readfirstlane(it.w);
     auto &a = ((ConstGodArgs *)w.descs)[di];
     int zlo, zhi;
-    brick_layers(a.zr, bid, BZ, -1, zlo, zhi);
-    brick64<BX, BY, BZ, RS, GEN>(a, bid, zlo, zhi, bid, sm);
+    part_layers(a.zr ? a.zr[bid] : ((BZ - 1) << 16), part, n, zlo, zhi);
+    brick64<BX, BY, BZ, RS, GEN>(a, bid, zlo, zhi, bid * n + part, sm);
 }
 
 template <int BX, int BY, int BZ, int RS>
@@ -79,9 +63,9 @@ static void level_launch(const GodArgs &a, bool gen, hipStream_t s, hipEvent_t e
 {
     constexpr int nt = (2 * BX + 2) * (2 * BY + 2);
     if (gen)
-        launch_brick(k_brick64<BX, BY, BZ, RS, true>, nt, a, s, e0, e1, nparts);
+        launch_brick(k_brick64<BX, BY, BZ, RS, true>, nt, BZ, kBrick64Waves, a, s, e0, e1, nparts);
     else
-        launch_brick(k_brick64<BX, BY, BZ, RS, false>, nt, a, s, e0, e1, nparts);
+        launch_brick(k_brick64<BX, BY, BZ, RS, false>, nt, BZ, kBrick64Waves, a, s, e0, e1, nparts);
 }
 
 template <int BX, int BY, int BZ, int RS>

@@ -35,6 +35,9 @@ struct GodArgs {
     // set by launch_godunov3d: bricks at the end of each XCD's range that run
     // as two half-brick work items (0 for levels with refluxes)
     int nsplit = 0;
+    // set by launch_godunov3d: parts along z of every brick (launches of fewer
+    // bricks than the chip holds)
+    int zsplit = 1;
     // coarse-fine refluxing (levels above levelmin): octs > ngridmax are
     // interpolated ghosts whose parent cell is ghost_parent[2*(v-ngridmax-1)+{0,1}]
     int reflux;
@@ -60,12 +63,13 @@ struct GodArgs {
 };
 
 // Work list of bricks over several descriptors (levels / jobs): item i is
-// (descriptor index, brick index); range[0..8] splits the items into one
-// contiguous range per XCD.  Descriptors must stay unchanged while a launch
+// (descriptor index, brick index, part, parts): one of `parts` parts of the
+// brick's z layers, whose Courant partial goes to slot brick*parts + part;
+// range[0..8] splits the items into one contiguous range per XCD.  Descriptors must stay unchanged while a launch
 // runs (the kernel reads them through the constant address space).
 struct WorkList {
     const GodArgs *descs;
-    const int2 *items;
+    const int4 *items;
     int range[9];
 };
 
@@ -92,10 +96,15 @@ struct God1Args {
     int rdet = 0;
 };
 
+// Parts along z for a work-list launch of nbricks bricks of one shape in
+// precision prec (see zsplit_for in rh_launch.h).
+int worklist_zsplit(long nbricks, int bx, int by, int bz, int prec);
+
 // Launch the 3D brick kernel for brick shape (bx,by,bz) in precision prec
 // (0 = FP64, 1 = FP32 reconstruction/fluxes with FP64 accumulation).
 // *nparts (if non-null) receives the number of Courant partials the launch
-// writes (bricks plus split halves), at most 2 nbricks + 8.
+// writes (bricks plus split halves, or the bricks' parts), at most
+// max(2 nbricks + 8, 4096).
 hipError_t launch_godunov3d(const GodArgs &a, int bx, int by, int bz, int prec, hipStream_t s,
                             hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, int *nparts = nullptr);
 hipError_t launch_godunov1d(const God1Args &a, int prec, hipStream_t s);

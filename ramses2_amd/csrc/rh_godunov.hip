@@ -312,7 +312,7 @@ __device__ __forceinline__ int ring_slot3(int t) { return (t + 3) % 3; }
 // reflux code.  The launch checks the level.
 template <int BX, int BY, int BZ, typename T, int RS, int NS, bool WL, bool GEN = true, typename A>
 __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY, BZ, T, RS, NS, WL, GEN> &sm,
-                                           const int part = -1, const int pslot = -1)
+                                           const int zlo, const int zhi, const int pslot)
 {
     constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY;
     constexpr int PX = 2 * BX + 4, PY = 2 * BY + 4, NP = PX * PY;
@@ -337,18 +337,8 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
     if (rlds)
         for (int i = tid; i < NW * 5; i += NT) (&sm.sacc[0][0])[i] = 0.0;
     const int ox0 = a.org[3 * bid + 0], oy0 = a.org[3 * bid + 1], oz0 = a.org[3 * bid + 2];
-    // cell planes [tlo, thi] of the brick hold octs of the level; the march
-    // covers them plus two halo planes on each side
-    const int zr = a.zr ? a.zr[bid] : ((BZ - 1) << 16);
-    int zlo = zr & 0xffff, zhi = zr >> 16;
-    if (part >= 0) {
-        // half of the brick's z layers (the lower half holds the middle one)
-        const int mid = (zlo + zhi) >> 1;
-        if (part == 0)
-            zhi = mid;
-        else
-            zlo = mid + 1;
-    }
+    // cell planes [tlo, thi] (the z layers of this part that hold octs of the
+    // level); the march covers them plus two halo planes on each side
     const int tlo = 2 * zlo, thi = 2 * zhi + 1;
 
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
@@ -738,7 +728,7 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
                 }
             };
             auto owned = [&](int x, int y, int z, int v) {
-                return x >= 0 && x < 2 * BX && y >= 0 && y < 2 * BY && z >= 0 && z < 2 * BZ && v >= a.head &&
+                return x >= 0 && x < 2 * BX && y >= 0 && y < 2 * BY && z >= tlo && z <= thi && v >= a.head &&
                        v < a.head + a.noct && ox0 + (x >> 1) < boxmax[0] && oy0 + (y >> 1) < boxmax[1] &&
                        oz0 + (z >> 1) < boxmax[2];
             };
@@ -885,6 +875,7 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
         for (int i = tid; !CU && i < BX * BY * BZ * 8; i += NT) {
             const int oc = i >> 3, ind = i & 7;
             const int ox = oc % BX + 1, oy = (oc / BX) % BY + 1, oz = oc / (BX * BY) + 1;
+            if (oz <= zlo || oz > zhi + 1) continue;  // another part's layers
             const int v = swin[(oz * WY + oy) * WX + ox];
             const bool own = v >= a.head && v < a.head + a.noct && ox0 + ox - 1 < boxmax[0] &&
                              oy0 + oy - 1 < boxmax[1] && oz0 + oz - 1 < boxmax[2];
@@ -921,11 +912,10 @@ __device__ __forceinline__ void brick_body(A &a, const int bid, BrickLds<BX, BY,
                     d = red[4 * i + 3] < d ? red[4 * i + 3] : d;
             }
             if constexpr (sizeof(T) == 8) d = signal_dt(d, ck);
-            const int ps = pslot >= 0 ? pslot : bid;
-            a.cpart[4 * ps + 0] = m;
-            a.cpart[4 * ps + 1] = e;
-            a.cpart[4 * ps + 2] = ei;
-            a.cpart[4 * ps + 3] = d;
+            a.cpart[4 * pslot + 0] = m;
+            a.cpart[4 * pslot + 1] = e;
+            a.cpart[4 * pslot + 2] = ei;
+            a.cpart[4 * pslot + 3] = d;
         }
     }
 }
@@ -938,9 +928,9 @@ __global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2),
     k_godunov3d(const GodArgs a)
 {
     __shared__ BrickLds<BX, BY, BZ, T, RS, NS, false, GEN> sm;
-    int bid, part, pslot;
-    if (!level_item(a, bid, part, pslot)) return;
-    brick_body<BX, BY, BZ, T, RS, NS, false, GEN>(a, bid, sm, part, pslot);
+    int bid, zlo, zhi, pslot;
+    if (!level_item(a, BZ, bid, zlo, zhi, pslot)) return;
+    brick_body<BX, BY, BZ, T, RS, NS, false, GEN>(a, bid, sm, zlo, zhi, pslot);
 }
 
 // Work-list kernel: work item i = (descriptor, brick), where a descriptor
@@ -963,9 +953,13 @@ __global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2), (brick_waves<BX, 
     const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
     const int i = w.range[x] + l;
     if (i >= w.range[x + 1]) return;
-    const int2 it = w.items[i];
+    const int4 it = w.items[i];
     const int di = __builtin_amdgcn_readfirstlane(it.x), bi = __builtin_amdgcn_readfirstlane(it.y);
-    brick_body<BX, BY, BZ, T, RS, NS, true, GEN>(((ConstGodArgs *)w.descs)[di], bi, sm);
+    const int part = __builtin_amdgcn_readfirstlane(it.z), n = __builtin_amdgcn_readfirstlane(it.w);
+    auto &a = ((ConstGodArgs *)w.descs)[di];
+    int zlo, zhi;
+    part_layers(a.zr ? a.zr[bi] : ((BZ - 1) << 16), part, n, zlo, zhi);
+    brick_body<BX, BY, BZ, T, RS, NS, true, GEN>(a, bi, sm, zlo, zhi, bi * n + part);
 }
 
 
@@ -1606,23 +1600,29 @@ hipError_t launch_godunov3d(const GodArgs &a, int bx, int by, int bz, int prec, 
 #define RH_LAUNCH_SHAPE(A, B, C)                                                                         \
     if (bx == A && by == B && bz == C) {                                                                 \
         constexpr int nt = (2 * A + 2) * (2 * B + 2);                                                     \
+        const int wv = prec == 0 ? RH_BRICK_MIN_WAVES : brick_waves<A, B, C, float, false>();            \
         if (a.slope == 3) {                                                                              \
             if (prec == 0)                                                                               \
-                launch_brick(k_godunov3d<A, B, C, double, 0, 3>, nt, a, s, e0, e1, nparts);              \
+                launch_brick(k_godunov3d<A, B, C, double, 0, 3>, nt, C, wv, a, s, e0, e1, nparts);              \
             else                                                                                         \
-                launch_brick(k_godunov3d<A, B, C, float, 0, 3>, nt, a, s, e0, e1, nparts);               \
+                launch_brick(k_godunov3d<A, B, C, float, 0, 3>, nt, C, wv, a, s, e0, e1, nparts);               \
         } else if (a.riemann == 3 && !gen) {                                                             \
-            launch_brick(k_godunov3d<A, B, C, float, 3, 2, false>, nt, a, s, e0, e1, nparts);            \
+            launch_brick(k_godunov3d<A, B, C, float, 3, 2, false>, nt, C, wv, a, s, e0, e1, nparts);            \
         } else if (a.riemann == 3) {                                                                     \
-            launch_brick(k_godunov3d<A, B, C, float, 3, 2>, nt, a, s, e0, e1, nparts);                   \
+            launch_brick(k_godunov3d<A, B, C, float, 3, 2>, nt, C, wv, a, s, e0, e1, nparts);                   \
         } else {                                                                                         \
-            launch_brick(k_godunov3d<A, B, C, float, 0, 2>, nt, a, s, e0, e1, nparts);                   \
+            launch_brick(k_godunov3d<A, B, C, float, 0, 2>, nt, C, wv, a, s, e0, e1, nparts);                   \
         }                                                                                                \
         return hipGetLastError();                                                                        \
     }
     RH_BRICK_SHAPES(RH_LAUNCH_SHAPE)
 #undef RH_LAUNCH_SHAPE
     return hipErrorInvalidValue;
+}
+
+int worklist_zsplit(long nbricks, int bx, int by, int bz, int prec)
+{
+    return zsplit_for(nbricks, bz, (2 * bx + 2) * (2 * by + 2), prec == 0 ? 2 : 4);
 }
 
 hipError_t launch_godunov3d_wl(const WorkList &w, int bx, int by, int bz, int slope, int riemann,

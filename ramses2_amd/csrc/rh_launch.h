@@ -23,6 +23,20 @@ static void launch_ev(K kernel, dim3 g, dim3 b, hipStream_t s, hipEvent_t e0, hi
         hipLaunchKernelGGL(kernel, g, b, 0, s, args...);
 }
 
+// Compute units of the current device.
+inline int device_cus()
+{
+    static int ncu = 0;
+    if (!ncu) {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1)
+            return 256;
+        ncu = n;
+    }
+    return ncu;
+}
+
 // Half-brick split of the final round (GodArgs::nsplit).  With equal work
 // per brick, q bricks per XCD on `slots` concurrent workgroups per XCD run in
 // ceil(q / slots) rounds; when the last round holds rem = q mod slots <=
@@ -36,14 +50,7 @@ template <typename K> static int tail_split(K kernel, int nthreads, const GodArg
 {
     if (!RH_TAIL_SPLIT || !a.xcd_remap || a.reflux) return 0;
     static std::map<const void *, int> occ_cache;
-    static int cus_per_xcd = 0;
-    if (!cus_per_xcd) {
-        int dev = 0, ncu = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return 0;
-        cus_per_xcd = ncu / 8 > 0 ? ncu / 8 : 1;
-    }
+    const int cus_per_xcd = device_cus() / 8 > 0 ? device_cus() / 8 : 1;
     auto it = occ_cache.find((const void *)kernel);
     int occ;
     if (it == occ_cache.end()) {
@@ -58,32 +65,72 @@ template <typename K> static int tail_split(K kernel, int nthreads, const GodArg
     return rem > 0 && 2 * rem <= slots ? rem : 0;
 }
 
+// Parts along z of each brick of a launch of nbricks bricks of bz oct layers
+// and nt threads at `waves` waves per SIMD.  A brick marches its planes one
+// after another (2.4 us each where it has the CU to itself, 3.5 us at two
+// waves per SIMD), so a launch of fewer bricks than the chip holds takes the
+// time of one brick, however few they are.  Cutting each brick into n parts
+// shortens the march to 2 ceil(bz/n) + 3 planes, at three halo planes more per
+// part; n minimises the modelled time while all parts still run at once.
+// Bricks of 8x6x8: 32^3 cells in FP64 (12 bricks, 96 parts) 46.8 -> 14.8 us,
+// 64^3 (96 bricks, 384 parts) 31.2 -> 29.2 us, mixed 33.5 -> 27 us; mixed 32^3 in
+// 4x4x4 bricks 19.4 -> 14.9 us.  Once the whole bricks fill the chip the parts'
+// extra planes cost more than the shorter march gains, and they stay whole.
+inline int zsplit_for(long nbricks, int bz, int nt, int waves)
+{
+    const int wg = (nt + 63) / 64, ncu = device_cus();
+    const int percu = 4 * waves / wg > 0 ? 4 * waves / wg : 1;
+    int best = 1;
+    double cost = 0;
+    for (int n = 1; n <= bz && nbricks * n <= (long)percu * ncu; n++) {
+        const long c = (nbricks * n + ncu - 1) / ncu;   // workgroups per CU
+        const double w = c * wg / 4.0;                   // waves per SIMD
+        const double t = (2 * ((bz + n - 1) / n) + 3) * (0.54 + 0.46 * (w > 1 ? w : 1.0));
+        if (n == 1 || t < 0.97 * cost) {
+            best = n;
+            cost = t;
+        }
+    }
+    return best;
+}
+// z layers [zlo, zhi] of part `part` of n of a brick whose layers are zr (zlo |
+// zhi << 16; may be empty: zlo > zhi)
+__device__ __forceinline__ void part_layers(int zr, int part, int n, int &zlo, int &zhi)
+{
+    const int lo = zr & 0xffff, len = (zr >> 16) - lo + 1;
+    zlo = lo + len * part / n;
+    zhi = lo + len * (part + 1) / n - 1;
+}
+
 template <typename K>
-static void launch_brick(K kernel, int nt, const GodArgs &a0, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
-                         int *nparts)
+static void launch_brick(K kernel, int nt, int bz, int waves, const GodArgs &a0, hipStream_t s, hipEvent_t e0,
+                         hipEvent_t e1, int *nparts)
 {
     GodArgs a = a0;
-    a.nsplit = tail_split(kernel, nt, a);
+    a.zsplit = a.xcd_remap ? zsplit_for(a.nbricks, bz, nt, waves) : 1;
+    a.nsplit = a.zsplit > 1 ? 0 : tail_split(kernel, nt, a);
     const int q = a.nbricks >> 3, r = a.nbricks & 7;
-    const dim3 g(a.nsplit ? 8 * (q + (r ? 1 : 0) + a.nsplit) : a.nbricks), b(nt);
-    if (nparts) *nparts = a.nbricks + 8 * a.nsplit;
+    const dim3 g(a.nsplit ? 8 * (q + (r ? 1 : 0) + a.nsplit) : a.nbricks * a.zsplit), b(nt);
+    if (nparts) *nparts = a.nbricks * a.zsplit + 8 * a.nsplit;
     launch_ev(kernel, g, b, s, e0, e1, a);
 }
 
-// The work item of workgroup blockIdx.x of a per-level launch: brick bid, its
-// part (-1 the whole brick, 0 / 1 its lower / upper half) and its slot among the
-// Courant partials; false where the workgroup has none.  Consecutive bricks go
-// to the same XCD, so that their shared halo octs meet in that XCD's L2.
-__device__ __forceinline__ bool level_item(const GodArgs &a, int &bid, int &part, int &pslot)
+// The work item of workgroup blockIdx.x of a per-level launch: brick bid, part
+// `part` of n of its z layers (of bz) and its slot among the Courant partials;
+// false where the workgroup has none.  Consecutive items go to the same XCD, so
+// that the bricks' shared halo octs meet in that XCD's L2.
+__device__ __forceinline__ bool level_item(const GodArgs &a, int bz, int &bid, int &zlo, int &zhi, int &pslot)
 {
     bid = blockIdx.x;
-    part = -1;
+    int part = 0, n = 1;
     pslot = bid;
     if (a.xcd_remap && a.nsplit == 0) {
         const int nb = gridDim.x, x = bid & 7, l = bid >> 3;
         const int q = nb >> 3, r = nb & 7;
-        bid = x * q + (x < r ? x : r) + l;
-        pslot = bid;
+        pslot = x * q + (x < r ? x : r) + l;
+        n = a.zsplit;
+        bid = pslot / n;
+        part = pslot - bid * n;
     } else if (a.xcd_remap) {
         // the last nsplit bricks of each XCD's range run as two work items,
         // one per half of the brick's z layers, so that the final round of
@@ -98,12 +145,15 @@ __device__ __forceinline__ bool level_item(const GodArgs &a, int &bid, int &part
         } else {
             const int j = l - (count - m);
             bid = start + count - m + (j >> 1);
+            n = 2;
             part = j & 1;
             // Courant partial of the upper half: after the nbricks whole-brick slots
             pslot = part == 0 ? bid : a.nbricks + x * m + (j >> 1);
         }
     }
-    return bid < a.nbricks;
+    if (bid >= a.nbricks) return false;
+    part_layers(a.zr ? a.zr[bid] : ((bz - 1) << 16), part, n, zlo, zhi);
+    return true;
 }
 
 }  // namespace rh

@@ -4,6 +4,11 @@
 // slots and the length of its dependent chain; the results agree with the
 // reference's expressions to rounding.  (The mixed-precision kernels use
 // rh_physics.h: their FP32 results depend on every rounding.)
+//
+// Contraction is off and every FMA written out: the compiler otherwise contracts
+// the same expression differently from one copy of the code to the next (a
+// peeled first iteration, another brick shape), and a plane's bits would depend
+// on where a march begins.
 #pragma once
 #include "rh_physics.h"
 
@@ -53,6 +58,7 @@ __device__ __forceinline__ double sound_speed64(double n, double d)
 __device__ __forceinline__ double prim64(const double u[5], double q[5], double smallr, double smalle, double gm1,
                                          const double gdt_half[3])
 {
+#pragma clang fp contract(off)
     const double r = u[0] > smallr ? u[0] : smallr;
     const double ir = rcp_h(r);
     const double vx = u[1] * ir, vy = u[2] * ir, vz = u[3] * ir;
@@ -92,23 +98,21 @@ __device__ __forceinline__ double vel_bound64(double dqh, double rl, double a, d
 __device__ __forceinline__ void trace64(const double q[5], const double dqh[3][5], double qp[3][5], double qm[3][5],
                                         const HydroK<double> &k, double inv_r)
 {
+#pragma clang fp contract(off)
     using T = double;
     T r = q[0], u = q[1], v = q[2], w = q[3], p = q[4];
     T drx = dqh[0][0], dux = dqh[0][1], dvx = dqh[0][2], dwx = dqh[0][3], dpx = dqh[0][4];
     T dry = dqh[1][0], duy = dqh[1][1], dvy = dqh[1][2], dwy = dqh[1][3], dpy = dqh[1][4];
     T drz = dqh[2][0], duz = dqh[2][1], dvz = dqh[2][2], dwz = dqh[2][3], dpz = dqh[2][4];
     T divv = dux + dvy + dwz;
-    T sr0 = -u * drx - v * dry - w * drz - divv * r;
-    T su0 = -u * dux - v * duy - w * duz - dpx * inv_r;
-    T sv0 = -u * dvx - v * dvy - w * dvz - dpy * inv_r;
-    T sw0 = -u * dwx - v * dwy - w * dwz - dpz * inv_r;
-    T sp0 = -u * dpx - v * dpy - w * dpz - divv * k.gamma * p;
+    // -(v . grad) of each variable
+    auto adv = [&](T dx, T dy, T dz) { return tfma(-w, dz, tfma(-v, dy, -u * dx)); };
     T ws[5];
-    ws[0] = r + sr0 * k.dtdx;
-    ws[1] = u + su0 * k.dtdx;
-    ws[2] = v + sv0 * k.dtdx;
-    ws[3] = w + sw0 * k.dtdx;
-    ws[4] = p + sp0 * k.dtdx;
+    ws[0] = tfma(tfma(-r, divv, adv(drx, dry, drz)), k.dtdx, r);
+    ws[1] = tfma(tfma(-inv_r, dpx, adv(dux, duy, duz)), k.dtdx, u);
+    ws[2] = tfma(tfma(-inv_r, dpy, adv(dvx, dvy, dvz)), k.dtdx, v);
+    ws[3] = tfma(tfma(-inv_r, dpz, adv(dwx, dwy, dwz)), k.dtdx, w);
+    ws[4] = tfma(tfma(-(divv * k.gamma), p, adv(dpx, dpy, dpz)), k.dtdx, p);
 #pragma unroll
     for (int d = 0; d < 3; d++) {
 #pragma unroll
@@ -143,8 +147,6 @@ __device__ __forceinline__ void trace64(const double q[5], const double dqh[3][5
 // reference's are not repeated.
 __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
 {
-    // contraction is spelled out, so that every kernel that solves a face gets
-    // the same bits
 #pragma clang fp contract(off)
     using T = double;
     const T half = T(0.5);
@@ -191,59 +193,52 @@ __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], d
     f[4] = (eo + Po) * uo;
 }
 
+// Conservative state and physical flux of one side (side_state).
+__device__ __forceinline__ void side64(const double q[5], double entho, double u[5], double f[5])
+{
+#pragma clang fp contract(off)
+    const double ke = tfma(q[3], q[3], tfma(q[2], q[2], q[1] * q[1]));
+    u[0] = q[0];
+    u[1] = q[0] * q[1];
+    u[2] = q[0] * q[2];
+    u[3] = q[0] * q[3];
+    u[4] = tfma(0.5 * q[0], ke, q[4] * entho);
+    f[0] = u[1];
+    f[1] = tfma(q[1], u[1], q[4]);
+    f[2] = q[1] * u[2];
+    f[3] = q[1] * u[3];
+    f[4] = q[1] * (u[4] + q[4]);
+}
+
 // riemann_llf, hydro/godunov_utils.f90:338-485.
 __device__ __forceinline__ void llf64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
 {
-    using T = double;
-    T rl = ql[0], pl = tmax(ql[4], rl * k.smallp_riem);
-    T cl = sound_speed64(k.gamma * pl, rl);
-    T rr = qr[0], pr = tmax(qr[4], rr * k.smallp_riem);
-    T cr = sound_speed64(k.gamma * pr, rr);
-    T cmax = tmin(tmax(fabs_(ql[1]) + cl, fabs_(qr[1]) + cr), k.smax_cap);
-    T uL[5], uR[5];
-    side_state(ql, k.entho, uL);
-    side_state(qr, k.entho, uR);
-    T fL[5], fR[5];
-    fL[0] = ql[1] * uL[0];
-    fR[0] = qr[1] * uR[0];
-    fL[1] = ql[1] * uL[1] + ql[4];
-    fR[1] = qr[1] * uR[1] + qr[4];
-    fL[2] = ql[1] * uL[2];
-    fR[2] = qr[1] * uR[2];
-    fL[3] = ql[1] * uL[3];
-    fR[3] = qr[1] * uR[3];
-    fL[4] = ql[1] * (uL[4] + ql[4]);
-    fR[4] = qr[1] * (uR[4] + qr[4]);
+#pragma clang fp contract(off)
+    const double pl = tmax(ql[4], ql[0] * k.smallp_riem), pr = tmax(qr[4], qr[0] * k.smallp_riem);
+    const double cl = sound_speed64(k.gamma * pl, ql[0]), cr = sound_speed64(k.gamma * pr, qr[0]);
+    const double cmax = tmin(tmax(fabs_(ql[1]) + cl, fabs_(qr[1]) + cr), k.smax_cap);
+    double uL[5], uR[5], fL[5], fR[5];
+    side64(ql, k.entho, uL, fL);
+    side64(qr, k.entho, uR, fR);
 #pragma unroll
-    for (int n = 0; n < 5; n++) f[n] = T(0.5) * (fL[n] + fR[n] - cmax * (uR[n] - uL[n]));
+    for (int n = 0; n < 5; n++) f[n] = 0.5 * tfma(-cmax, uR[n] - uL[n], fL[n] + fR[n]);
 }
 
 // riemann_hll, hydro/godunov_utils.f90:486-637.
 __device__ __forceinline__ void hll64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
 {
-    using T = double;
-    T rl = ql[0], ul = ql[1], pl = tmax(ql[4], rl * k.smallp_riem);
-    T rr = qr[0], ur = qr[1], pr = tmax(qr[4], rr * k.smallp_riem);
-    T cmax = sqrt_quot_max(k.gamma * pl, rl, k.gamma * pr, rr);
-    T SL = tmax(tmin(tmin(ul, ur) - cmax, T(0)), -k.smax_cap);
-    T SR = tmin(tmax(tmax(ul, ur) + cmax, T(0)), k.smax_cap);
-    T uL[5], uR[5];
-    side_state(ql, k.entho, uL);
-    side_state(qr, k.entho, uR);
-    T fL[5], fR[5];
-    fL[0] = uL[1];
-    fR[0] = uR[1];
-    fL[1] = ql[4] + uL[1] * ql[1];
-    fR[1] = qr[4] + uR[1] * qr[1];
-    fL[2] = ql[1] * uL[2];
-    fR[2] = qr[1] * uR[2];
-    fL[3] = ql[1] * uL[3];
-    fR[3] = qr[1] * uR[3];
-    fL[4] = ql[1] * (uL[4] + ql[4]);
-    fR[4] = qr[1] * (uR[4] + qr[4]);
-    const T inv = rcp_h(SR - SL);  // SR - SL >= 2c > 0, the same for all five
+#pragma clang fp contract(off)
+    const double ul = ql[1], ur = qr[1];
+    const double pl = tmax(ql[4], ql[0] * k.smallp_riem), pr = tmax(qr[4], qr[0] * k.smallp_riem);
+    const double cmax = sqrt_quot_max(k.gamma * pl, ql[0], k.gamma * pr, qr[0]);
+    const double SL = tmax(tmin(tmin(ul, ur) - cmax, 0.0), -k.smax_cap);
+    const double SR = tmin(tmax(tmax(ul, ur) + cmax, 0.0), k.smax_cap);
+    double uL[5], uR[5], fL[5], fR[5];
+    side64(ql, k.entho, uL, fL);
+    side64(qr, k.entho, uR, fR);
+    const double inv = rcp_h(SR - SL), ss = SR * SL;  // SR - SL >= 2c > 0, the same for all five
 #pragma unroll
-    for (int n = 0; n < 5; n++) f[n] = (SR * fL[n] - SL * fR[n] + SR * SL * (uR[n] - uL[n])) * inv;
+    for (int n = 0; n < 5; n++) f[n] = tfma(ss, uR[n] - uL[n], tfma(SR, fL[n], -(SL * fR[n]))) * inv;
 }
 
 // cmpflxm for the solver RS (1 LLF, 2 HLL, 3 HLLC) with states already rotated

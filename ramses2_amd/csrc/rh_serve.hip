@@ -330,7 +330,7 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
     if (precision != 0 && precision != 1) return efail(RH_ERR_ARG, "precision must be 0 or 1");
     if (njobs == 0 || nsteps == 0) return 0;
     std::vector<State *> js(njobs);
-    long nitems = 0;
+    long nbricks = 0;
     bool gen = false;  // some job needs the general brick body
     for (int j = 0; j < njobs; j++) {
         State *s = ctx_get(ids[j]);
@@ -342,21 +342,25 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
         if (s->job_bx != js[0]->job_bx || s->job_by != js[0]->job_by || s->job_bz != js[0]->job_bz ||
             s->job.slope != js[0]->job.slope || s->job.riemann != js[0]->job.riemann)
             return efail(RH_ERR_ARG, "the jobs of one batch need the same brick shape, slope and Riemann solver");
-        nitems += s->job.nbricks;
+        nbricks += s->job.nbricks;
         // (batches add to uold: ubase == uold)
         gen = gen || s->job.bnd || s->job.any_ref || s->job.reflux || s->job.g[0] != 0.0 || s->job.g[1] != 0.0 ||
               s->job.g[2] != 0.0;
     }
-    if (nitems > (1l << 30)) return efail(RH_ERR_ARG, "too many bricks in one batch");
+    if (nbricks > (1l << 29)) return efail(RH_ERR_ARG, "too many bricks in one batch");
+    // few bricks: each in nz parts along z (no more parts than the chip runs at
+    // once, fewer than a context's Courant partials)
+    const int nz = worklist_zsplit(nbricks, js[0]->job_bx, js[0]->job_by, js[0]->job_bz, precision);
+    const long nitems = nbricks * nz;
     hipStream_t stream = js[0]->stream;
     const size_t off_c = align256(2 * (size_t)njobs * sizeof(GodArgs));
     const size_t off_i = off_c + align256((size_t)njobs * sizeof(CourantJob));
-    const size_t bytes = off_i + (size_t)nitems * sizeof(int2);
+    const size_t bytes = off_i + (size_t)nitems * sizeof(int4);
     if (int r = batch_reserve(bytes, stream)) return r;
     Batch &b = g_batch;
     GodArgs *h_descs = (GodArgs *)b.h_buf;
     CourantJob *h_cjobs = (CourantJob *)(b.h_buf + off_c);
-    int2 *h_items = (int2 *)(b.h_buf + off_i);
+    int4 *h_items = (int4 *)(b.h_buf + off_i);
     int pos = 0;
     for (int j = 0; j < njobs; j++) {
         State &s = *js[j];
@@ -369,8 +373,9 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
         a.unew = s.uold;
         a.ubase = s.unew;
         h_descs[njobs + j] = a;
-        h_cjobs[j] = CourantJob{s.red_part, s.job.nbricks, s.job_dtmax, s.red_out, s.dt_dev, s.t_dev};
-        for (int i = 0; i < s.job.nbricks; i++) h_items[pos++] = make_int2(j, i);
+        h_cjobs[j] = CourantJob{s.red_part, s.job.nbricks * nz, s.job_dtmax, s.red_out, s.dt_dev, s.t_dev};
+        for (int i = 0; i < s.job.nbricks; i++)
+            for (int k = 0; k < nz; k++) h_items[pos++] = make_int4(j, i, k, nz);
     }
     RH_HIP_CHECK(hipMemcpyAsync(b.d_buf, b.h_buf, bytes, hipMemcpyHostToDevice, stream));
     RH_HIP_CHECK(hipEventRecord(b.staged, stream));
@@ -378,7 +383,7 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
     const GodArgs *d_descs = (const GodArgs *)b.d_buf;
     const CourantJob *d_cjobs = (const CourantJob *)(b.d_buf + off_c);
     WorkList w;
-    w.items = (const int2 *)(b.d_buf + off_i);
+    w.items = (const int4 *)(b.d_buf + off_i);
     for (int r = 0; r <= 8; r++) w.range[r] = (int)((nitems * r) / 8);
     for (int k = 0; k < nsteps; k++) {
         w.descs = d_descs + (k & 1) * njobs;

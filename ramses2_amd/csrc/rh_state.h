@@ -70,7 +70,7 @@ struct AmrPlan {
     int ndesc = 0, nitems = 0;
     GodArgs *d_descs = nullptr;    // [2][ndesc]: arrays in both orders
     std::vector<GodArgs> h_descs;  // host copy of d_descs
-    int2 *d_items = nullptr;       // [nitems] (level descriptor, brick), grouped by brick shape
+    int4 *d_items = nullptr;       // [nitems] (level descriptor, brick, part, parts), grouped by brick shape
     // one work-list launch per brick shape among the levels
     struct Group {
         int bx, by, bz;

@@ -64,3 +64,29 @@ def test_gravity_runs_the_general_body(riemann):
     p = HydroParams(gamma=1.4, courant_factor=0.5, slope_type=2, riemann=riemann)
     g, o = _steps(20, p, (8, 6, 8), 3, gravity=(0.5, -0.25, 0.125))
     assert np.all(rel_err_per_var(g, o) < TOL), rel_err_per_var(g, o)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("brick", [(8, 6, 8), (4, 4, 4)])
+def test_parts_of_a_brick_give_the_whole_bricks_bits(brick, precision):
+    """A batch of few bricks cuts each into parts along z, a batch that fills
+    the chip does not (zsplit_for): the same job steps bit for bit alike in
+    both, its sums to rounding."""
+    from ramses2_amd.serving import HipEngine, JobSpec
+    eng = HipEngine(precision=precision, brick=brick)
+    job = JobSpec(0, 0.0, 34, 1, (1.0, 1e-3, 400.0, 16.0, 0.0), 3)
+    big = JobSpec(1, 0.0, 128, 1, (1.0, 1e-2, 100.0, 63.0, 0.0), 3)
+    alone, mixed, filler = eng.open(job), eng.open(job), eng.open(big)
+    try:
+        for _ in range(3):
+            eng.step([alone])
+            eng.step([filler, mixed])
+        assert np.array_equal(eng.state(alone, job), eng.state(mixed, job))
+        a, m = eng.status(alone), eng.status(mixed)
+        assert a["t"] == m["t"] and a["dt_next"] == m["dt_next"]
+        for k in ("mass", "ekin", "eint"):
+            assert abs(a[k] - m[k]) <= 1e-13 * abs(m[k])
+    finally:
+        for h in (alone, mixed, filler):
+            eng.close(h)
+        eng.close_all()
