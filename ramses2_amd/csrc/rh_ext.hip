@@ -372,7 +372,12 @@ int rh_level_run(int head_idx, int num_octs, int ilevel, double dx, double gamma
                                     __builtin_sqrt(smallc2), courant_factor, g ? g : gz, s.red_part, s.red_cap,
                                     s.red_out, s.dt_dev, s.stream, nullptr));
     }
-    if (use_graph && nsteps >= 2) {
+    // a small 1D level in FP64: every step in one launch (which also leaves unew
+    // equal to uold), unless the Godunov launches are to be timed
+    const bool tube = s.ndim == 1 && s.precision == 0 && nsteps > 0 && !kernel_ms && tube_fits(a1);
+    if (tube) {
+        RH_HIP_CHECK(launch_tube(a1, nsteps, dt_fixed, s.red_out, s.dt_dev, s.t_dev, s.stream));
+    } else if (use_graph && nsteps >= 2) {
         // the pair of steps uold->unew, unew->uold as one graph, captured once
         // for each order of the two arrays and kept for later calls with the
         // same arguments, arrays and tables
@@ -483,8 +488,9 @@ int rh_level_run(int head_idx, int num_octs, int ilevel, double dx, double gamma
     }
     // unew mirrors uold as after set_uold
     const size_t per = (size_t)s.nvar * s.ttd;
-    RH_HIP_CHECK(hipMemcpyAsync(s.unew + per * (head_idx - 1), s.uold + per * (head_idx - 1),
-                                per * num_octs * sizeof(double), hipMemcpyDeviceToDevice, s.stream));
+    if (!tube)
+        RH_HIP_CHECK(hipMemcpyAsync(s.unew + per * (head_idx - 1), s.uold + per * (head_idx - 1),
+                                    per * num_octs * sizeof(double), hipMemcpyDeviceToDevice, s.stream));
     double h[2] = {0, 0};
     RH_HIP_CHECK(hipMemcpyAsync(s.h_red, s.red_out, 5 * sizeof(double), hipMemcpyDeviceToHost, s.stream));
     RH_HIP_CHECK(hipMemcpyAsync(h, s.t_dev, sizeof(double), hipMemcpyDeviceToHost, s.stream));

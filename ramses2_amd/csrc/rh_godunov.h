@@ -108,6 +108,13 @@ int worklist_zsplit(long nbricks, int bx, int by, int bz, int prec);
 hipError_t launch_godunov3d(const GodArgs &a, int bx, int by, int bz, int prec, hipStream_t s,
                             hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, int *nparts = nullptr);
 hipError_t launch_godunov1d(const God1Args &a, int prec, hipStream_t s);
+// All steps of a call on a small 1D level in one launch (rh_tube.hip, FP64):
+// nsteps steps with the Courant dt, or dt_fixed > 0, the final state in a.uold
+// and a.unew; out and dt_dev receive the sums before the last step and its dt
+// (as launch_courant), t_dev advances.  Where tube_fits().
+bool tube_fits(const God1Args &a);
+hipError_t launch_tube(const God1Args &a, int nsteps, double dt_fixed, double *out, double *dt_dev, double *t_dev,
+                       hipStream_t s);
 // The specialised brick bodies (GEN = false) are used where a level allows
 // them unless this is 0 (rh_set_specialized; the general body then runs
 // everywhere, for checking that both give the same bits).
