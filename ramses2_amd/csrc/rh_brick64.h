@@ -5,8 +5,8 @@
 // One workgroup per oct brick, one thread per column of the brick's cells plus
 // one halo cell, marching along z.  Per plane tt there are two phases, each
 // ended by a barrier:
-//   A: the update of plane tt-1 from the face fluxes in LDS (its z flux and that
-//      of tt-2 in registers, so tt-2 becomes final and is stored); the own cell
+//   A: the update of plane tt-1 from the face fluxes (the column's own low faces
+//      in registers, its high faces in LDS), tt-2 final and stored; the own cell
 //      of plane tt+1 converted to primitives, the loads of plane tt+2 issued;
 //      slopes and Hancock predictor of plane tt, its left x and y states to LDS;
 //   B: primitives of plane tt+1 to LDS (every slope of plane tt has read the
@@ -25,9 +25,10 @@
 // halo loop solves one face per lane, converts the ring and updates nothing.
 // Measured against the one-body kernel this replaced (four barriers, every
 // thread testing its role, the expressions of rh_physics.h), with the Courant
-// reduction: 256^3 in 8x6x16 bricks 843 -> 675 us (24.9 G cell-updates/s, 2.0
-// TB/s of the 80 algorithmic bytes per cell), 128^3 in 8x6x8 bricks 140 -> 109
-// us, 90^3 MinMod + LLF (a run-time solver choice before) 105 -> 64 us.
+// reduction: 256^3 in 8x6x16 bricks 843 -> 660 us (25.4 G cell-updates/s, 2.0
+// TB/s of the 80 algorithmic bytes per cell; 680 with the column's own low faces
+// read back from LDS and two reciprocals per HLLC face), 128^3 in 8x6x8 bricks
+// 140 -> 106 us, 90^3 MinMod + LLF (a run-time solver choice before) 105 -> 64 us.
 #pragma once
 #include <type_traits>
 
@@ -239,12 +240,13 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
 
         double qmz[5] = {0, 0, 0, 0, 0};   // left state of the low z face of plane tt
         double fz[5] = {0, 0, 0, 0, 0};    // flux of the low z face of plane tt-1
-        double fzp[5] = {0, 0, 0, 0, 0};   // of plane tt-2
-        double pp[5] = {0, 0, 0, 0, 0};    // u + x and y parts of plane tt-2
+        double fxo[5] = {0, 0, 0, 0, 0};   // fluxes of the low x and y faces of plane tt-1
+        double fyo[5] = {0, 0, 0, 0, 0};
+        double pp[5] = {0, 0, 0, 0, 0};    // plane tt-2 but for its high z face
         double ub[5] = {0, 0, 0, 0, 0};    // the update's base of plane tt-1 (GEN)
         uint8_t ref1 = 0, ref2 = 0;        // refined flags of planes tt-1 and tt-2
 
-        // plane tf of the column is final: un = pp + (dt/dx)(fzp - fz)
+        // plane tf of the column is final: un = pp - (dt/dx) fz
         auto finish = [&](int tf, const bool upper) __attribute__((always_inline)) {
             const int v = sm.swin[((tf + 2) >> 1) * (WX * WY) + wcol];
             const bool own = v >= a.head && v < a.head + a.noct && ox0 + (cx >> 1) < boxmax[0] &&
@@ -252,7 +254,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
             if (!own) return;
             double un[5];
 #pragma unroll
-            for (int n = 0; n < 5; n++) un[n] = tfma(dtdx, fzp[n] - fz[n], pp[n]);
+            for (int n = 0; n < 5; n++) un[n] = tfma(-dtdx, fz[n], pp[n]);
             // the two planes of an oct fill each 64-byte line of unew: the
             // lower plane's values wait in LDS and both are stored together
             if (upper) {
@@ -277,15 +279,11 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
 #pragma unroll
                 for (int n = 0; n < 5; n++) {
                     const double u = GEN ? ub[n] : sm.sub[GEN ? 0 : par ^ 1][n][GEN ? 0 : icol];
-                    part[n] = tfma(dtdx, sm.fy[n][iyl] - sm.fy[n][iyh],
-                                   tfma(dtdx, sm.fx[n][ixl] - sm.fx[n][ixh], u));
+                    part[n] = tfma(dtdx, fyo[n] - sm.fy[n][iyh], tfma(dtdx, fxo[n] - sm.fx[n][ixh], u));
                 }
                 if (tt - 2 >= tlo) finish(tt - 2, par != 0);
 #pragma unroll
-                for (int n = 0; n < 5; n++) {
-                    pp[n] = part[n];
-                    fzp[n] = fz[n];
-                }
+                for (int n = 0; n < 5; n++) pp[n] = tfma(dtdx, fz[n], part[n]);
             }
             // ---- the own cell of plane tt+1 ----
             double qp[5];
@@ -342,7 +340,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
             }
             // ---- F: the low x, y and z faces of plane tt ----
             const bool xy = tt >= tlo && tt <= thi;
-            double f_x[5], f_y[5];
+            double (&f_x)[5] = fxo, (&f_y)[5] = fyo;
             if (ROLE == 2) {
                 // the right column's x face or the top row's y face: one pass,
                 // the direction chosen per lane

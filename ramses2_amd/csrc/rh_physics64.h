@@ -35,15 +35,15 @@ __device__ __forceinline__ double rsq_pos(double x)
     const double e = __builtin_fma(-(x * y), y, 1.0);
     return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
 }
-// max(sqrt(na/da), sqrt(nb/db)) for positive operands without a division: the
+// max(sqrt(g na/da), sqrt(g nb/db)) for positive operands without a division: the
 // larger quotient is found by cross multiplication, and sqrt(n/d) = n/sqrt(n d)
 // takes one refined reciprocal square root.  Two sound speeds of a face cost
 // 19 issue slots this way against 35 as two refined reciprocals and a square
 // root.  The products are floored where sqrt would leave the normal range.
-__device__ __forceinline__ double sqrt_quot_max(double na, double da, double nb, double db)
+__device__ __forceinline__ double sqrt_quot_max(double na, double da, double nb, double db, double g)
 {
     const bool a = na * db > nb * da;
-    const double n = a ? na : nb, d = a ? da : db;
+    const double n = g * (a ? na : nb), d = a ? da : db;
     return n * rsq_pos(__builtin_fmax(n * d, 0x1p-1020));
 }
 // sqrt(n/d): a sound speed from gamma*P and rho
@@ -157,24 +157,24 @@ __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], d
     T ur = qr[1], vr = qr[2], wr = qr[3];
     T Pr = tmax(qr[4], rr * k.smallp_riem);
     // max(sqrt(a), sqrt(b)) = sqrt(max(a, b)): one root for the two sound speeds
-    T cmax = sqrt_quot_max(k.gamma * Pl, rl, k.gamma * Pr, rr);
+    T cmax = sqrt_quot_max(Pl, rl, Pr, rr, k.gamma);
     T SL = tmin(ul, ur) - cmax;
     T SR = tmax(ul, ur) + cmax;
     T dl = ul - SL, dr = SR - ur;
     T rcl = rl * dl, rcr = rr * dr;
-    T inv_den = rcp_h(tfma(rr, dr, rcl));
+    T den = tfma(rr, dr, rcl);  // positive: ustar = num/den has the sign of num
     T num = (Pl - Pr) + tfma(rcr, ur, rcl * ul);
-    T ustar = num * inv_den;
-    T Ptotstar = tfma(rcl * rcr, ul - ur, tfma(rcr, Pl, rcl * Pr)) * inv_den;
     // The reference samples, in this order: SL > 0 -> left state; ustar > 0
     // -> left star state; SR > 0 -> right star state; else right state.  The
     // side whose values are used is left exactly when SL > 0 or ustar > 0,
     // and the star state is taken when SL <= 0 and (ustar > 0 or SR > 0); in
     // both star cases the side is the reference's ustar > 0.  So one select
-    // of the side's six values and one of four values (state or star) give
-    // the reference's result (its chain costs three selects per value), and
-    // the total energy is formed for the sampled side only.
-    const bool sl_pos = SL > T(0), us_pos = ustar > T(0);
+    // of the side's values gives the reference's result (its chain costs three
+    // selects per value), and the total energy is formed for that side only.
+    // Outside the star states the contact's velocity and pressure are the
+    // side's own, with which the star state's formulas return the side's state
+    // (S - ustar = S - us): two selects instead of one for each of four values.
+    const bool sl_pos = SL > T(0), us_pos = num > T(0);
     const bool left = sl_pos || us_pos;
     const bool star = !sl_pos && (us_pos || SR > T(0));
     T S = left ? SL : SR;
@@ -182,10 +182,16 @@ __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], d
     T vo = left ? vl : vr, wo = left ? wl : wr;
     T es = tfma(half * rs, tfma(wo, wo, tfma(us, us, vo * vo)), Ps * k.entho);
     T ds = S - us;
-    T inv_sd = rcp_h(tfma(-inv_den, num, S));  // 1/(S - ustar)
-    T rstar = rs * ds * inv_sd;
-    T etotstar = tfma(Ptotstar, ustar, tfma(ds, es, -(Ps * us))) * inv_sd;
-    T ro = star ? rstar : rs, uo = star ? ustar : us, Po = star ? Ptotstar : Ps, eo = star ? etotstar : es;
+    // 1/den and 1/(S - ustar) = den/(S den - num) from one reciprocal: the
+    // hardware one takes four issue slots, and the two would depend on each other
+    T nu = star ? num : us * den;
+    T t = tfma(S, den, -nu);
+    T ri = rcp_h(den * t);
+    T inv_den = ri * t, inv_sd = (ri * den) * den;
+    T uo = nu * inv_den;
+    T Po = star ? tfma(rcl * rcr, ul - ur, tfma(rcr, Pl, rcl * Pr)) * inv_den : Ps;
+    T ro = rs * ds * inv_sd;
+    T eo = tfma(Po, uo, tfma(ds, es, -(Ps * us))) * inv_sd;
     f[0] = ro * uo;
     f[1] = tfma(f[0], uo, Po);
     f[2] = f[0] * vo;
@@ -230,7 +236,7 @@ __device__ __forceinline__ void hll64(const double ql[5], const double qr[5], do
 #pragma clang fp contract(off)
     const double ul = ql[1], ur = qr[1];
     const double pl = tmax(ql[4], ql[0] * k.smallp_riem), pr = tmax(qr[4], qr[0] * k.smallp_riem);
-    const double cmax = sqrt_quot_max(k.gamma * pl, ql[0], k.gamma * pr, qr[0]);
+    const double cmax = sqrt_quot_max(pl, ql[0], pr, qr[0], k.gamma);
     const double SL = tmax(tmin(tmin(ul, ur) - cmax, 0.0), -k.smax_cap);
     const double SR = tmin(tmax(tmax(ul, ur) + cmax, 0.0), k.smax_cap);
     double uL[5], uR[5], fL[5], fR[5];
