@@ -96,7 +96,8 @@ hipError_t enqueue_amr_step(State &s, int parity, int precision)
         w.descs = m.d_descs + parity * m.ndesc;
         w.items = m.d_items + gr.first;
         for (int r = 0; r <= 8; r++) w.range[r] = gr.range[r];
-        if ((e = launch_godunov3d_wl(w, gr.bx, gr.by, gr.bz, m.slope, m.riemann, precision, s.stream)) != hipSuccess)
+        if ((e = launch_godunov3d_wl(w, gr.bx, gr.by, gr.bz, m.slope, m.riemann, precision, s.stream, m.kind)) !=
+            hipSuccess)
             return e;
     }
     if ((e = launch_reflux_fold(unext, m.racc, s.ghost_parent, s.ghost_order, s.nghost_total, 8, s.stream,
@@ -239,6 +240,8 @@ int rh_amr_prepare(int levelmin, int levelmax, const int32_t *head, const int32_
     }
     m.nitems = (int)items.size();
     m.h_descs = both;
+    m.kind = kBrickPeriodic;
+    for (const auto &a : both) m.kind = std::max(m.kind, brick_kind(a));
     RH_HIP_CHECK(dmalloc((void **)&m.d_descs, both.size() * sizeof(GodArgs)));
     RH_HIP_CHECK(dmalloc((void **)&m.d_items, std::max<size_t>(items.size(), 1) * sizeof(int4)));
     RH_HIP_CHECK(hipMemcpyAsync(m.d_descs, both.data(), both.size() * sizeof(GodArgs), hipMemcpyHostToDevice, s.stream));

@@ -58,7 +58,7 @@ template <int BX, int BY, int BZ, bool GEN> struct Brick64Core {
     double fx[5][NFX], fy[5][NFY];     // fluxes by face
     double sun[5][NI];                 // new state of the lower plane of an oct layer
     double sub[GEN ? 1 : 2][5][GEN ? 1 : NI];  // conserved state of the last two planes (the update's base)
-    uint8_t sref[GEN ? 2 : 1][GEN ? NP : 1];   // refined flags of two planes
+    uint8_t sref[GEN ? NW : 1];                // refined cells of each window oct (bit: cell)
 };
 template <int BX, int BY, int BZ, bool GEN> struct Brick64Lds : Brick64Core<BX, BY, BZ, GEN> {
     using Core = Brick64Core<BX, BY, BZ, GEN>;
@@ -70,20 +70,19 @@ template <int BX, int BY, int BZ, bool GEN> struct Brick64Lds : Brick64Core<BX, 
 
 // The march over the z layers [zlo, zhi] of brick bid.  Courant partials go to
 // cpart[4*pslot].  A: GodArgs, as a kernel argument or in the constant address
-// space (a work-list descriptor).  GEN = false: a level periodic in every
-// dimension, without refined cells, refluxes or gravity, whose update adds to
-// uold.
-template <int BX, int BY, int BZ, int RS, bool GEN, typename A>
+// space (a work-list descriptor).  KIND: which inputs the instance takes, see
+// BrickKind.
+template <int BX, int BY, int BZ, int RS, int KIND, typename A>
 __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, const int zhi, const int pslot,
-                                        Brick64Lds<BX, BY, BZ, GEN> &sm)
+                                        Brick64Lds<BX, BY, BZ, KIND != kBrickUniform> &sm)
 {
 #pragma clang fp contract(off)
+    constexpr bool GEN = KIND != kBrickUniform;
     constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY, NI = 4 * BX * BY;
     constexpr int PX = 2 * BX + 4;
     constexpr int WX = BX + 2, WY = BY + 2, NW = WX * WY * (BZ + 2);
     constexpr bool HW = brick64_hw<BX, BY>(), RA = Brick64Lds<BX, BY, BZ, GEN>::RA;
     const int tid = threadIdx.x;
-    for (int i = tid; i < NW; i += NT) sm.swin[i] = a.win[(size_t)bid * NW + i];
     const bool rlds = RA && a.reflux && !a.rdet;
     if (RA && rlds)
         for (int i = tid; i < NW * 5; i += NT) (&sm.sacc[0][0])[i] = 0.0;
@@ -105,10 +104,10 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
     // the two faces of a dimension with one FMA, both cells of a face reading
     // the same flux, so the update conserves.  The reference's (F dt)/dx
     // (hydro/umuscl.f90:135-220) is formed only for the coarse reflux.
-    const double dtdx = dt * a.inv_dx;
+    const double dtdx = dt * a.inv_dx, dtdx8 = 0.125 * dtdx;
     const int boxmin[3] = {a.boxmin[0], a.boxmin[1], a.boxmin[2]};
     const int boxmax[3] = {a.boxmax[0], a.boxmax[1], a.boxmax[2]};
-    const bool anyref = GEN && a.any_ref != 0, bnd = GEN && a.bnd != 0, reflux = GEN && a.reflux != 0;
+    const bool bnd = KIND == kBrickBounded && a.bnd != 0, reflux = GEN && a.reflux != 0;
     int refl = 0;
     if constexpr (GEN)
 #pragma unroll
@@ -118,7 +117,34 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
     const CourantK ck = make_courant_k(a.dx, 3, a.gamma, a.smallr, a.smallc2, a.courant_factor, gvec);
     const bool courant = a.courant != 0;
     double c_mass = 0.0, c_ekin = 0.0, c_eint = 0.0, c_sig = 0.0;
-    __syncthreads();
+    // The window, and the refined cells of its octs as one byte each: the flags
+    // of a face's cells are then two LDS bytes away, and a brick without any
+    // refined cell skips them (a flag per cell, fetched, staged and read with
+    // the plane's primitives, cost a refined mesh 6%).
+    bool mine = false;
+    for (int i = tid; i < NW; i += NT) {
+        const int v = a.win[(size_t)bid * NW + i];
+        sm.swin[i] = v;
+        if constexpr (GEN) {
+            int m = 0;
+            if (a.any_ref && v > 0) {
+                const uint64_t f = *(const uint64_t *)(a.refined + (size_t)(v - 1) * 8);
+#pragma unroll
+                for (int ind = 0; ind < 8; ind++) m |= ((f >> (8 * ind)) & 0xff) != 0 ? 1 << ind : 0;
+            } else if (bnd && a.any_ref && v < 0) {
+                const int okey[3] = {ox0 + i % WX - 1, oy0 + i / WX % WY - 1, oz0 + i / (WX * WY) - 1};
+                for (int ind = 0; ind < 8; ind++) {
+                    const int c[3] = {ind & 1, (ind >> 1) & 1, ind >> 2};
+                    const uint8_t *rf = cell_ref3(a.uold, a.refined, v, okey, boxmin, boxmax, refl, c).rf;
+                    if (rf && *rf) m |= 1 << ind;
+                }
+            }
+            sm.sref[GEN ? i : 0] = (uint8_t)m;
+            mine = mine || m != 0;
+        }
+    }
+    const bool anyref = GEN && __syncthreads_or(mine);
+    if (!GEN) __syncthreads();
 
     // ROLE 1: a column of the brick's interior; 2: a column of the halo ring;
     // 0: either, tested per thread (shapes whose interior does not fill waves)
@@ -177,11 +203,10 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
         }
         const int pr = (ry + 2) * PX + (rx + 2);
 
-        auto fetch = [&](int px, int py, int tz, double u[5], uint8_t &rf, int &fl) __attribute__((always_inline)) {
+        auto fetch = [&](int px, int py, int tz, double u[5], int &fl) __attribute__((always_inline)) {
             const int ox = (px + 2) >> 1, oy = (py + 2) >> 1, oz = (tz + 2) >> 1;
             const int v = sm.swin[(oz * WY + oy) * WX + ox];
             fl = -1;
-            rf = 0;
             if (!bnd) {
                 // no boundary ghosts: an oct, or none (then nothing that the
                 // cell feeds is stored, and any cell's values do)
@@ -190,28 +215,26 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
                 const double *p = a.uold + o * 40 + ind;
 #pragma unroll
                 for (int n = 0; n < 5; n++) u[n] = p[8 * n];
-                if (anyref && v > 0) rf = a.refined[o * 8 + ind];
                 return;
             }
             const int okey[3] = {ox0 + ox - 1, oy0 + oy - 1, oz0 + oz - 1};
             const int c[3] = {px & 1, py & 1, tz & 1};
             CellRef cr = cell_ref3(a.uold, a.refined, v, okey, boxmin, boxmax, refl, c);
-            if (!anyref) cr.rf = nullptr;
+            cr.rf = nullptr;
+            uint8_t rf;
             cell_load3(cr, u, rf);
             fl = cr.flip;
         };
 
         double u_o[5], u_r[5];
-        uint8_t rf_o = 0, rf_r = 0;
         int fl_o = -1, fl_r = -1;
         auto convert = [&](double u[5], int fl, double q[5]) __attribute__((always_inline)) {
             if (bnd && fl >= 0) cell_flip(u, fl);  // reflexive ghosts only: skipped by waves without any
             return prim64(u, q, a.smallr, smalle, gm1, gdt);
         };
-        auto put = [&](const double q[5], uint8_t rf, int i, int par) __attribute__((always_inline)) {
+        auto put = [&](const double q[5], int i) __attribute__((always_inline)) {
 #pragma unroll
             for (int n = 0; n < 5; n++) sm.sq[n][i] = q[n];
-            if (anyref) sm.sref[GEN ? par : 0][GEN ? i : 0] = rf;
         };
 
         // own column: primitives of plane tt, their difference from plane tt-1
@@ -220,21 +243,21 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
         double q0[5], dzm[5], rho_m, ir0;
         {
             double q[5];
-            fetch(cx, cy, tlo - 2, u_o, rf_o, fl_o);
+            fetch(cx, cy, tlo - 2, u_o, fl_o);
             convert(u_o, fl_o, q);
-            fetch(cx, cy, tlo - 1, u_o, rf_o, fl_o);
-            if (ring) fetch(rx, ry, tlo - 1, u_r, rf_r, fl_r);
+            fetch(cx, cy, tlo - 1, u_o, fl_o);
+            if (ring) fetch(rx, ry, tlo - 1, u_r, fl_r);
             ir0 = convert(u_o, fl_o, q0);
             rho_m = q[0];
 #pragma unroll
             for (int n = 0; n < 5; n++) dzm[n] = q0[n] - q[n];
-            put(q0, rf_o, pc, 1);
+            put(q0, pc);
             if (ring) {
                 convert(u_r, fl_r, q);
-                put(q, rf_r, pr, 1);
+                put(q, pr);
             }
-            fetch(cx, cy, tlo, u_o, rf_o, fl_o);
-            if (ring) fetch(rx, ry, tlo, u_r, rf_r, fl_r);
+            fetch(cx, cy, tlo, u_o, fl_o);
+            if (ring) fetch(rx, ry, tlo, u_r, fl_r);
         }
         __syncthreads();
 
@@ -244,7 +267,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
         double fyo[5] = {0, 0, 0, 0, 0};
         double pp[5] = {0, 0, 0, 0, 0};    // plane tt-2 but for its high z face
         double ub[5] = {0, 0, 0, 0, 0};    // the update's base of plane tt-1 (GEN)
-        uint8_t ref1 = 0, ref2 = 0;        // refined flags of planes tt-1 and tt-2
+        bool ref1 = false, ref2 = false;   // refined flags of planes tt-1 and tt-2
 
         // plane tf of the column is final: un = pp - (dt/dx) fz
         auto finish = [&](int tf, const bool upper) __attribute__((always_inline)) {
@@ -271,6 +294,75 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
             if (courant && !ref2) c_sig = tmax(c_sig, courant_cell<3>(un, ck, ck.vol, c_mass, c_ekin, c_eint));
         };
 
+        auto wi = [&](int x, int y, int z) __attribute__((always_inline)) {
+            return (((z + 2) >> 1) * WY + ((y + 2) >> 1)) * WX + ((x + 2) >> 1);
+        };
+        auto refined = [&](int x, int y, int z) __attribute__((always_inline)) {
+            return ((sm.sref[GEN ? wi(x, y, z) : 0] >> ((x & 1) + 2 * (y & 1) + 4 * (z & 1))) & 1) != 0;
+        };
+        // a face next to a refined cell has no flux of this level; most waves
+        // have none and skip the ten selects
+        auto refzero = [&](bool z, double f[5]) __attribute__((always_inline)) {
+            if (__any(z))
+#pragma unroll
+                for (int n = 0; n < 5; n++) f[n] = z ? 0.0 : f[n];
+        };
+        // Coarse-fine refluxes.  The cells of an oct face share one ghost oct,
+        // so an x or y face adds the fluxes of both planes of the oct layer at
+        // the upper one (the lower plane's still in LDS where this thread
+        // stores its own next), and a z face can meet a ghost only below an
+        // even plane: a third of the tests and half of the atomics of adding
+        // every face by itself.
+        auto owned = [&](int x, int y, int z, int v) __attribute__((always_inline)) {
+            return x >= 0 && x < 2 * BX && y >= 0 && y < 2 * BY && z >= tlo && z <= thi && v >= a.head &&
+                   v < a.head + a.noct && ox0 + (x >> 1) < boxmax[0] && oy0 + (y >> 1) < boxmax[1] &&
+                   oz0 + (z >> 1) < boxmax[2];
+        };
+        // F into the ghost oct v of window slot i: summed in LDS, or straight
+        // to the accumulator / parent cell
+        auto radd = [&](int i, int v, double sign, const double F[5], int slot) __attribute__((always_inline)) {
+            if (RA && rlds) {
+                const double w = sign * dtdx8;
+#pragma unroll
+                for (int n = 0; n < 5; n++) atomicAdd(&sm.sacc[RA ? i : 0][n], F[n] * w);
+            } else {
+                double G[5];
+#pragma unroll
+                for (int n = 0; n < 5; n++) G[n] = F[n] * dtdx;
+                reflux_add(a.unew, a.ghost_parent, a.ngridmax, v, sign, G, 8, a.racc, a.rdet, slot);
+            }
+        };
+        // the low x (y) face of the column, plane tt odd: f of this plane, the
+        // plane below's at fb (stride st)
+        auto reflux_xy = [&](int tt, const bool dy, const double *fb, int st, const double f[5]) __attribute__((always_inline)) {
+            const int xl = dy ? cx : cx - 1, yl = dy ? cy - 1 : cy;
+            const int il = wi(xl, yl, tt), ih = wi(cx, cy, tt), vl = sm.swin[il], vh = sm.swin[ih];
+            const bool gl = vl > a.ngridmax;
+            if (gl == (vh > a.ngridmax)) return;
+            if (!(gl ? owned(cx, cy, tt, vh) : owned(xl, yl, tt, vl))) return;
+            const int i = gl ? il : ih, v = gl ? vl : vh;
+            const double sign = gl ? -1.0 : 1.0;
+            const int slot = (dy ? 8 + (cx & 1) : (cy & 1)) + (gl ? 4 : 0);
+            double F[5];
+#pragma unroll
+            for (int n = 0; n < 5; n++) F[n] = fb[n * st];
+            if (!a.rdet) {
+#pragma unroll
+                for (int n = 0; n < 5; n++) F[n] = F[n] + f[n];
+            } else {
+                radd(i, v, sign, f, slot + 2);
+            }
+            radd(i, v, sign, F, slot);
+        };
+        // the low z face, plane tt even
+        auto reflux_z = [&](int tt, const double f[5]) __attribute__((always_inline)) {
+            const int il = wi(cx, cy, tt - 1), ih = wi(cx, cy, tt), vl = sm.swin[il], vh = sm.swin[ih];
+            const bool gl = vl > a.ngridmax;
+            if (gl == (vh > a.ngridmax)) return;
+            if (!(gl ? owned(cx, cy, tt, vh) : owned(cx, cy, tt - 1, vl))) return;
+            radd(gl ? il : ih, gl ? vl : vh, gl ? -1.0 : 1.0, f, (gl ? 20 : 16) + (cx & 1) + 2 * (cy & 1));
+        };
+
         // one plane; par = tt & 1
         auto plane = [&](const int tt, const int par) __attribute__((always_inline)) {
             // ---- A: update of plane tt-1, plane tt-2 stored ----
@@ -293,10 +385,9 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
                     for (int n = 0; n < 5; n++) sm.sub[GEN ? 0 : par ^ 1][n][GEN ? 0 : icol] = u_o[n];
             }
             const double irp = convert(u_o, fl_o, qp);
-            const uint8_t rfp = rf_o;
             // the next loads below the conversion that consumes the current ones, so that both use the same registers
             __builtin_amdgcn_sched_barrier(0);
-            fetch(cx, cy, tt < thi ? tt + 2 : thi + 2, u_o, rf_o, fl_o);
+            fetch(cx, cy, tt < thi ? tt + 2 : thi + 2, u_o, fl_o);
             // ---- T: slopes and predictor of plane tt ----
             double dq[3][5];
             auto slopes = [&](const int sl) __attribute__((always_inline)) {
@@ -327,16 +418,16 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
             if (has_qy)
 #pragma unroll
                 for (int n = 0; n < 5; n++) sm.qy[n][iyh] = ql[1][n];
-            const uint8_t myref = anyref ? sm.sref[GEN ? par : 0][GEN ? pc : 0] : 0;
+            const bool myref = anyref && refined(cx, cy, tt);
             __syncthreads();
             // ---- B: primitives of plane tt+1 to LDS ----
-            put(qp, rfp, pc, par ^ 1);
+            put(qp, pc);
             if (ring) {
                 double q[5];
                 convert(u_r, fl_r, q);
-                put(q, rf_r, pr, par ^ 1);
+                put(q, pr);
                 __builtin_amdgcn_sched_barrier(0);
-                fetch(rx, ry, tt < thi ? tt + 2 : thi + 1, u_r, rf_r, fl_r);
+                fetch(rx, ry, tt < thi ? tt + 2 : thi + 1, u_r, fl_r);
             }
             // ---- F: the low x, y and z faces of plane tt ----
             const bool xy = tt >= tlo && tt <= thi;
@@ -353,12 +444,11 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
                     const double r5[5] = {dy ? qr[1][0] : qr[0][0], dy ? qr[1][2] : qr[0][1], dy ? qr[1][1] : qr[0][2],
                                           dy ? qr[1][3] : qr[0][3], dy ? qr[1][4] : qr[0][4]};
                     solve64<RS>(l5, r5, g, k);
-                    bool z = false;
-                    if (anyref) z = myref || sm.sref[GEN ? par : 0][GEN ? (dy ? pc - PX : pc - 1) : 0];
-                    const double f[5] = {z ? 0.0 : g[0], z ? 0.0 : (dy ? g[2] : g[1]), z ? 0.0 : (dy ? g[1] : g[2]),
-                                         z ? 0.0 : g[3], z ? 0.0 : g[4]};
+                    double f[5] = {g[0], dy ? g[2] : g[1], dy ? g[1] : g[2], g[3], g[4]};
+                    if (anyref) refzero(myref || (dy ? refined(cx, cy - 1, tt) : refined(cx - 1, cy, tt)), f);
                     double *fb = dy ? &sm.fy[0][iyl] : &sm.fx[0][ixl];
                     const int st = dy ? Brick64Lds<BX, BY, BZ, GEN>::NFY : Brick64Lds<BX, BY, BZ, GEN>::NFX;
+                    if (reflux && par == 1) reflux_xy(tt, dy, fb, st, f);
 #pragma unroll
                     for (int n = 0; n < 5; n++) {
                         fb[n * st] = f[n];
@@ -371,11 +461,9 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
 #pragma unroll
                     for (int n = 0; n < 5; n++) l[n] = sm.qx[n][ixl];
                     face64<RS>(0, l, qr[0], f_x, k);
-                    if (anyref) {
-                        const bool z = myref || sm.sref[GEN ? par : 0][GEN ? pc - 1 : 0];
-#pragma unroll
-                        for (int n = 0; n < 5; n++) f_x[n] = z ? 0.0 : f_x[n];
-                    }
+                    if (anyref) refzero(myref || refined(cx - 1, cy, tt), f_x);
+                    if (reflux && par == 1)
+                        reflux_xy(tt, false, &sm.fx[0][ixl], Brick64Lds<BX, BY, BZ, GEN>::NFX, f_x);
 #pragma unroll
                     for (int n = 0; n < 5; n++) sm.fx[n][ixl] = f_x[n];
                 }
@@ -384,22 +472,17 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
 #pragma unroll
                     for (int n = 0; n < 5; n++) l[n] = sm.qy[n][iyl];
                     face64<RS>(1, l, qr[1], f_y, k);
-                    if (anyref) {
-                        const bool z = myref || sm.sref[GEN ? par : 0][GEN ? pc - PX : 0];
-#pragma unroll
-                        for (int n = 0; n < 5; n++) f_y[n] = z ? 0.0 : f_y[n];
-                    }
+                    if (anyref) refzero(myref || refined(cx, cy - 1, tt), f_y);
+                    if (reflux && par == 1)
+                        reflux_xy(tt, true, &sm.fy[0][iyl], Brick64Lds<BX, BY, BZ, GEN>::NFY, f_y);
 #pragma unroll
                     for (int n = 0; n < 5; n++) sm.fy[n][iyl] = f_y[n];
                 }
             }
             if (ROLE != 2 && interior && tt >= tlo) {
                 face64<RS>(2, qmz, qr[2], fz, k);
-                if (anyref) {
-                    const bool z = myref || ref1;
-#pragma unroll
-                    for (int n = 0; n < 5; n++) fz[n] = z ? 0.0 : fz[n];
-                }
+                if (anyref) refzero(myref || ref1, fz);
+                if (reflux && par == 0) reflux_z(tt, fz);
             }
             if constexpr (GEN) {
                 // the base of this plane's update (unew for the drop-in call,
@@ -409,46 +492,6 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
                     const double *pb = a.ubase + (size_t)(v > 1 ? v - 1 : 0) * 40 + icell + 4 * par;
 #pragma unroll
                     for (int n = 0; n < 5; n++) ub[n] = pb[8 * n];
-                }
-            }
-            if (reflux) {
-                auto wi = [&](int x, int y, int z) { return (((z + 2) >> 1) * WY + ((y + 2) >> 1)) * WX + ((x + 2) >> 1); };
-                // one fine face's reflux into the ghost oct of window slot i:
-                // summed in LDS, or straight to the accumulator / parent cell
-                auto radd = [&](int i, int v, double sign, const double F[5], int slot) {
-                    if (RA && rlds) {
-#pragma unroll
-                        for (int n = 0; n < 5; n++)
-                            atomicAdd(&sm.sacc[RA ? i : 0][n], sign * ((F[n] * dt) * a.inv_dx * 0.125));
-                    } else {
-                        double G[5];
-#pragma unroll
-                        for (int n = 0; n < 5; n++) G[n] = (F[n] * dt) * a.inv_dx;
-                        reflux_add(a.unew, a.ghost_parent, a.ngridmax, v, sign, G, 8, a.racc, a.rdet, slot);
-                    }
-                };
-                auto owned = [&](int x, int y, int z, int v) {
-                    return x >= 0 && x < 2 * BX && y >= 0 && y < 2 * BY && z >= 2 * zlo && z <= 2 * zhi + 1 &&
-                           v >= a.head && v < a.head + a.noct && ox0 + (x >> 1) < boxmax[0] &&
-                           oy0 + (y >> 1) < boxmax[1] && oz0 + (z >> 1) < boxmax[2];
-                };
-                if (xy && do_fx && !(anyref && (myref || sm.sref[GEN ? par : 0][GEN ? pc - 1 : 0]))) {
-                    const int il = wi(cx - 1, cy, tt), ih = wi(cx, cy, tt), vl = sm.swin[il], vh = sm.swin[ih];
-                    const int s = (cy & 1) + 2 * (tt & 1);
-                    if (vl > a.ngridmax && owned(cx, cy, tt, vh)) radd(il, vl, -1.0, f_x, 4 + s);
-                    if (vh > a.ngridmax && owned(cx - 1, cy, tt, vl)) radd(ih, vh, 1.0, f_x, s);
-                }
-                if (xy && do_fy && !(anyref && (myref || sm.sref[GEN ? par : 0][GEN ? pc - PX : 0]))) {
-                    const int il = wi(cx, cy - 1, tt), ih = wi(cx, cy, tt), vl = sm.swin[il], vh = sm.swin[ih];
-                    const int s = (cx & 1) + 2 * (tt & 1);
-                    if (vl > a.ngridmax && owned(cx, cy, tt, vh)) radd(il, vl, -1.0, f_y, 12 + s);
-                    if (vh > a.ngridmax && owned(cx, cy - 1, tt, vl)) radd(ih, vh, 1.0, f_y, 8 + s);
-                }
-                if (interior && tt >= tlo && !(myref || ref1)) {
-                    const int il = wi(cx, cy, tt - 1), ih = wi(cx, cy, tt), vl = sm.swin[il], vh = sm.swin[ih];
-                    const int s = (cx & 1) + 2 * (cy & 1);
-                    if (vl > a.ngridmax && owned(cx, cy, tt, vh)) radd(il, vl, -1.0, fz, 20 + s);
-                    if (vh > a.ngridmax && owned(cx, cy, tt - 1, vl)) radd(ih, vh, 1.0, fz, 16 + s);
                 }
             }
             __syncthreads();

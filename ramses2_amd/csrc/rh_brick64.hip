@@ -30,22 +30,22 @@
 
 namespace rh {
 
-template <int BX, int BY, int BZ, int RS, bool GEN>
+template <int BX, int BY, int BZ, int RS, int KIND>
 __global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2), kBrick64Waves) k_brick64(const GodArgs a)
 {
-    __shared__ Brick64Lds<BX, BY, BZ, GEN> sm;
+    __shared__ Brick64Lds<BX, BY, BZ, KIND != kBrickUniform> sm;
     int bid, zlo, zhi, pslot;
     if (!level_item(a, BZ, bid, zlo, zhi, pslot)) return;
-    brick64<BX, BY, BZ, RS, GEN>(a, bid, zlo, zhi, pslot, sm);
+    brick64<BX, BY, BZ, RS, KIND>(a, bid, zlo, zhi, pslot, sm);
 }
 
 // Work-list form, see k_godunov3d_wl: workgroup b runs item range[b % 8] + b / 8.
 typedef const __attribute__((address_space(4))) GodArgs ConstGodArgs;
 
-template <int BX, int BY, int BZ, int RS, bool GEN>
+template <int BX, int BY, int BZ, int RS, int KIND>
 __global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2), kBrick64Waves) k_brick64_wl(const WorkList w)
 {
-    __shared__ Brick64Lds<BX, BY, BZ, GEN> sm;
+    __shared__ Brick64Lds<BX, BY, BZ, KIND != kBrickUniform> sm;
     const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
     const int i = w.range[x] + l;
     if (i >= w.range[x + 1]) return;
@@ -55,41 +55,45 @@ __global__ void __launch_bounds__((2 * BX + 2) * (2 * BY + 2), kBrick64Waves) k_
     auto &a = ((ConstGodArgs *)w.descs)[di];
     int zlo, zhi;
     part_layers(a.zr ? a.zr[bid] : ((BZ - 1) << 16), part, n, zlo, zhi);
-    brick64<BX, BY, BZ, RS, GEN>(a, bid, zlo, zhi, bid * n + part, sm);
+    brick64<BX, BY, BZ, RS, KIND>(a, bid, zlo, zhi, bid * n + part, sm);
 }
 
 template <int BX, int BY, int BZ, int RS>
-static void level_launch(const GodArgs &a, bool gen, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int *nparts)
+static void level_launch(const GodArgs &a, int kind, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int *nparts)
 {
     constexpr int nt = (2 * BX + 2) * (2 * BY + 2);
-    if (gen)
-        launch_brick(k_brick64<BX, BY, BZ, RS, true>, nt, BZ, kBrick64Waves, a, s, e0, e1, nparts);
+    if (kind == kBrickUniform)
+        launch_brick(k_brick64<BX, BY, BZ, RS, kBrickUniform>, nt, BZ, kBrick64Waves, a, s, e0, e1, nparts);
+    else if (kind == kBrickPeriodic)
+        launch_brick(k_brick64<BX, BY, BZ, RS, kBrickPeriodic>, nt, BZ, kBrick64Waves, a, s, e0, e1, nparts);
     else
-        launch_brick(k_brick64<BX, BY, BZ, RS, false>, nt, BZ, kBrick64Waves, a, s, e0, e1, nparts);
+        launch_brick(k_brick64<BX, BY, BZ, RS, kBrickBounded>, nt, BZ, kBrick64Waves, a, s, e0, e1, nparts);
 }
 
 template <int BX, int BY, int BZ, int RS>
-static void list_launch(const WorkList &w, int nblocks, bool gen, hipStream_t s)
+static void list_launch(const WorkList &w, int nblocks, int kind, hipStream_t s)
 {
     const dim3 g(nblocks), b((2 * BX + 2) * (2 * BY + 2));
-    if (gen)
-        hipLaunchKernelGGL((k_brick64_wl<BX, BY, BZ, RS, true>), g, b, 0, s, w);
+    if (kind == kBrickUniform)
+        hipLaunchKernelGGL((k_brick64_wl<BX, BY, BZ, RS, kBrickUniform>), g, b, 0, s, w);
+    else if (kind == kBrickPeriodic)
+        hipLaunchKernelGGL((k_brick64_wl<BX, BY, BZ, RS, kBrickPeriodic>), g, b, 0, s, w);
     else
-        hipLaunchKernelGGL((k_brick64_wl<BX, BY, BZ, RS, false>), g, b, 0, s, w);
+        hipLaunchKernelGGL((k_brick64_wl<BX, BY, BZ, RS, kBrickBounded>), g, b, 0, s, w);
 }
 
 // The launches of this object's shapes; false for a shape of another set.
-bool RH_CAT(brick64_level_, RH_SET)(const GodArgs &a, int bx, int by, int bz, bool gen, hipStream_t s, hipEvent_t e0,
+bool RH_CAT(brick64_level_, RH_SET)(const GodArgs &a, int bx, int by, int bz, int kind, hipStream_t s, hipEvent_t e0,
                                     hipEvent_t e1, int *nparts)
 {
 #define RH_ONE(A, B, C)                                                \
     if (bx == A && by == B && bz == C) {                               \
         if (a.riemann == 3)                                            \
-            level_launch<A, B, C, 3>(a, gen, s, e0, e1, nparts);       \
+            level_launch<A, B, C, 3>(a, kind, s, e0, e1, nparts);       \
         else if (a.riemann == 2)                                       \
-            level_launch<A, B, C, 2>(a, gen, s, e0, e1, nparts);       \
+            level_launch<A, B, C, 2>(a, kind, s, e0, e1, nparts);       \
         else                                                           \
-            level_launch<A, B, C, 1>(a, gen, s, e0, e1, nparts);       \
+            level_launch<A, B, C, 1>(a, kind, s, e0, e1, nparts);       \
         return true;                                                   \
     }
     RH_SHAPES(RH_ONE)
@@ -97,17 +101,17 @@ bool RH_CAT(brick64_level_, RH_SET)(const GodArgs &a, int bx, int by, int bz, bo
     return false;
 }
 
-bool RH_CAT(brick64_list_, RH_SET)(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, bool gen,
+bool RH_CAT(brick64_list_, RH_SET)(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, int kind,
                                    hipStream_t s)
 {
 #define RH_ONE(A, B, C)                                                \
     if (bx == A && by == B && bz == C) {                               \
         if (riemann == 3)                                              \
-            list_launch<A, B, C, 3>(w, nblocks, gen, s);               \
+            list_launch<A, B, C, 3>(w, nblocks, kind, s);               \
         else if (riemann == 2)                                         \
-            list_launch<A, B, C, 2>(w, nblocks, gen, s);               \
+            list_launch<A, B, C, 2>(w, nblocks, kind, s);               \
         else                                                           \
-            list_launch<A, B, C, 1>(w, nblocks, gen, s);               \
+            list_launch<A, B, C, 1>(w, nblocks, kind, s);               \
         return true;                                                   \
     }
     RH_SHAPES(RH_ONE)

@@ -115,22 +115,33 @@ hipError_t launch_godunov1d(const God1Args &a, int prec, hipStream_t s);
 bool tube_fits(const God1Args &a);
 hipError_t launch_tube(const God1Args &a, int nsteps, double dt_fixed, double *out, double *dt_dev, double *t_dev,
                        hipStream_t s);
-// The specialised brick bodies (GEN = false) are used where a level allows
-// them unless this is 0 (rh_set_specialized; the general body then runs
-// everywhere, for checking that both give the same bits).
+// The specialised brick bodies (GEN = false, the lower kinds below) are used
+// where a level allows them unless this is 0 (rh_set_specialized; the general
+// body then runs everywhere, for checking that both give the same bits).
 extern int g_specialized;
+// What a brick kernel's instance takes, each kind all of the one before:
+// uniform: a level periodic in every dimension, without refined cells, refluxes
+// or gravity, whose update adds to uold; periodic: any of these but boundary
+// ghosts; bounded: everything.  The boundary ghosts' addressing and flips alone
+// cost a refined periodic mesh 3% (4.9 M cells on five levels, 32.4 -> 31.7 ms
+// per 40 steps).
+enum BrickKind { kBrickUniform = 0, kBrickPeriodic = 1, kBrickBounded = 2 };
+inline int brick_kind(const GodArgs &a)
+{
+    if (a.bnd) return kBrickBounded;
+    const bool plain = !a.any_ref && !a.reflux && a.ubase == a.uold && a.g[0] == 0.0 && a.g[1] == 0.0 && a.g[2] == 0.0;
+    return plain ? kBrickUniform : kBrickPeriodic;
+}
 // Work-list launch: items[i] = (descriptor index, brick index), one workgroup per item.
-// gen = false: every descriptor is a periodic level without refined cells,
-// refluxes (bnd, any_ref and reflux all 0) or gravity, whose update adds to uold
-// (ubase == uold), which the specialised body needs.
+// kind: the largest brick_kind of the descriptors.
 hipError_t launch_godunov3d_wl(const WorkList &w, int bx, int by, int bz, int slope, int riemann, int prec,
-                               hipStream_t s, bool gen = true);
+                               hipStream_t s, int kind);
 
 // The FP64 brick kernels of rh_brick64.hip (slopes 0-2); nblocks: the grid of
 // the work-list launch.
-hipError_t launch_brick64(const GodArgs &a, int bx, int by, int bz, bool gen, hipStream_t s, hipEvent_t e0,
+hipError_t launch_brick64(const GodArgs &a, int bx, int by, int bz, int kind, hipStream_t s, hipEvent_t e0,
                           hipEvent_t e1, int *nparts);
-hipError_t launch_brick64_wl(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, bool gen,
+hipError_t launch_brick64_wl(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, int kind,
                              hipStream_t s);
 
 // Courant reduction over cells of octs [head, head+noct): per-block partials,

@@ -1559,27 +1559,27 @@ int g_specialized = 1;
 // The objects of rh_brick64.hip, one per set of brick shapes
 #define RH_SETS(X) X(0) X(1) X(2) X(3) X(4) X(5)
 #define RH_DECL(N)                                                                                               \
-    bool brick64_level_##N(const GodArgs &a, int bx, int by, int bz, bool gen, hipStream_t s, hipEvent_t e0,      \
+    bool brick64_level_##N(const GodArgs &a, int bx, int by, int bz, int kind, hipStream_t s, hipEvent_t e0,      \
                            hipEvent_t e1, int *nparts);                                                          \
-    bool brick64_list_##N(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, bool gen, hipStream_t s);
+    bool brick64_list_##N(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, int kind, hipStream_t s);
 RH_SETS(RH_DECL)
 #undef RH_DECL
 
-hipError_t launch_brick64(const GodArgs &a, int bx, int by, int bz, bool gen, hipStream_t s, hipEvent_t e0,
+hipError_t launch_brick64(const GodArgs &a, int bx, int by, int bz, int kind, hipStream_t s, hipEvent_t e0,
                           hipEvent_t e1, int *nparts)
 {
 #define RH_TRY(N) \
-    if (brick64_level_##N(a, bx, by, bz, gen, s, e0, e1, nparts)) return hipGetLastError();
+    if (brick64_level_##N(a, bx, by, bz, kind, s, e0, e1, nparts)) return hipGetLastError();
     RH_SETS(RH_TRY)
 #undef RH_TRY
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_brick64_wl(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, bool gen,
+hipError_t launch_brick64_wl(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, int kind,
                              hipStream_t s)
 {
 #define RH_TRY(N) \
-    if (brick64_list_##N(w, nblocks, bx, by, bz, riemann, gen, s)) return hipGetLastError();
+    if (brick64_list_##N(w, nblocks, bx, by, bz, riemann, kind, s)) return hipGetLastError();
     RH_SETS(RH_TRY)
 #undef RH_TRY
     return hipErrorInvalidValue;
@@ -1590,13 +1590,11 @@ hipError_t launch_godunov3d(const GodArgs &a, int bx, int by, int bz, int prec, 
 {
     if (nparts) *nparts = a.nbricks > 0 ? a.nbricks : 0;
     if (a.nbricks <= 0) return hipSuccess;
-    // the specialised body: periodic in every dimension, no refined cells,
-    // no refluxes, (FP64) no gravity
-    bool gen = a.bnd || a.any_ref || a.reflux || a.ubase != a.uold || !g_specialized;
-    if (prec == 0 && a.slope != 3) {
-        gen = gen || a.g[0] != 0.0 || a.g[1] != 0.0 || a.g[2] != 0.0;
-        return launch_brick64(a, bx, by, bz, gen, s, e0, e1, nparts);
-    }
+    if (prec == 0 && a.slope != 3)
+        return launch_brick64(a, bx, by, bz, g_specialized ? brick_kind(a) : kBrickBounded, s, e0, e1, nparts);
+    // the specialised mixed-precision body: periodic in every dimension, no
+    // refined cells, no refluxes, the update added to uold
+    const bool gen = a.bnd || a.any_ref || a.reflux || a.ubase != a.uold || !g_specialized;
 #define RH_LAUNCH_SHAPE(A, B, C)                                                                         \
     if (bx == A && by == B && bz == C) {                                                                 \
         constexpr int nt = (2 * A + 2) * (2 * B + 2);                                                     \
@@ -1626,14 +1624,15 @@ int worklist_zsplit(long nbricks, int bx, int by, int bz, int prec)
 }
 
 hipError_t launch_godunov3d_wl(const WorkList &w, int bx, int by, int bz, int slope, int riemann,
-                               int prec, hipStream_t s, bool gen)
+                               int prec, hipStream_t s, int kind)
 {
     if (w.range[8] <= 0) return hipSuccess;
-    gen = gen || !g_specialized;
+    if (!g_specialized) kind = kBrickBounded;
+    const bool gen = kind != kBrickUniform;
     int maxr = 0;
     for (int r = 0; r < 8; r++) maxr = w.range[r + 1] - w.range[r] > maxr ? w.range[r + 1] - w.range[r] : maxr;
     const int nblocks = 8 * maxr;
-    if (prec == 0 && slope != 3) return launch_brick64_wl(w, nblocks, bx, by, bz, riemann, gen, s);
+    if (prec == 0 && slope != 3) return launch_brick64_wl(w, nblocks, bx, by, bz, riemann, kind, s);
 #define RH_LAUNCH_WL(A, B, C)                                                                            \
     if (bx == A && by == B && bz == C) {                                                                 \
         constexpr int nt = (2 * A + 2) * (2 * B + 2);                                                     \

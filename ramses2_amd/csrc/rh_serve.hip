@@ -331,7 +331,7 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
     if (njobs == 0 || nsteps == 0) return 0;
     std::vector<State *> js(njobs);
     long nbricks = 0;
-    bool gen = false;  // some job needs the general brick body
+    int kind = kBrickUniform;  // the body that all jobs can use
     for (int j = 0; j < njobs; j++) {
         State *s = ctx_get(ids[j]);
         if (!s || !s->job_ready)
@@ -343,9 +343,6 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
             s->job.slope != js[0]->job.slope || s->job.riemann != js[0]->job.riemann)
             return efail(RH_ERR_ARG, "the jobs of one batch need the same brick shape, slope and Riemann solver");
         nbricks += s->job.nbricks;
-        // (batches add to uold: ubase == uold)
-        gen = gen || s->job.bnd || s->job.any_ref || s->job.reflux || s->job.g[0] != 0.0 || s->job.g[1] != 0.0 ||
-              s->job.g[2] != 0.0;
     }
     if (nbricks > (1l << 29)) return efail(RH_ERR_ARG, "too many bricks in one batch");
     // few bricks: each in nz parts along z (no more parts than the chip runs at
@@ -368,6 +365,7 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
         a.uold = s.uold;
         a.unew = s.unew;
         a.ubase = s.uold;
+        kind = std::max(kind, brick_kind(a));
         h_descs[j] = a;
         a.uold = s.unew;
         a.unew = s.uold;
@@ -388,7 +386,7 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
     for (int k = 0; k < nsteps; k++) {
         w.descs = d_descs + (k & 1) * njobs;
         RH_HIP_CHECK(launch_godunov3d_wl(w, js[0]->job_bx, js[0]->job_by, js[0]->job_bz, js[0]->job.slope,
-                                         js[0]->job.riemann, precision, stream, gen));
+                                         js[0]->job.riemann, precision, stream, kind));
         RH_HIP_CHECK(launch_courant_reduce_batch(d_cjobs, njobs, stream));
     }
     if (nsteps & 1)

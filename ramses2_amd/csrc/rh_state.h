@@ -67,6 +67,7 @@ struct AmrPlan {
     double boxlen = 1.0, dx_finest = 0.0;
     double gamma = 1.4, smallr = 0.0, smallc2 = 0.0, courant = 0.0, g[3] = {0, 0, 0};
     int slope = 0, riemann = 0;
+    int kind = 0;                  // brick_kind of the levels together
     int ndesc = 0, nitems = 0;
     GodArgs *d_descs = nullptr;    // [2][ndesc]: arrays in both orders
     std::vector<GodArgs> h_descs;  // host copy of d_descs
