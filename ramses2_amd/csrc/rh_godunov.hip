@@ -1176,41 +1176,33 @@ __global__ void k_zero(double *p, long n)
 // With nslot = kRefluxSlots (deterministic mode) each ghost has one slot per
 // face of its oct, added to the parent cell one after another in slot order:
 // the same sums on every run.
-__global__ void k_reflux_fold(double *unew, double *__restrict__ racc, const int32_t *__restrict__ ghost_parent,
-                              const int32_t *__restrict__ order, int nghost, int ttd, int nslot)
+// One thread per ghost and variable: the fold is a chain of dependent gathers
+// (order, accumulator, parent cell), so what counts is how many are in flight.
+// 4.9 M cells on five levels: 26.0 -> 25.6 us; 1.1 M cells on four: 5.2 -> 4.9.
+__global__ void __launch_bounds__(256) k_reflux_fold(double *unew, double *__restrict__ racc,
+                                                     const int32_t *__restrict__ ghost_parent,
+                                                     const int32_t *__restrict__ order, int nghost, int ttd, int nslot)
 {
     // in parent-cell order (see k_refresh_ghosts)
-    const int t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int t = i / 5, n = i - 5 * t;
     if (t >= nghost) return;
     const int g = order[t];
-    double *rg = racc + 5 * (size_t)g * nslot;
+    double *rg = racc + 5 * (size_t)g * nslot + n;
     const int igrid = ghost_parent[2 * g], icell = ghost_parent[2 * g + 1];
-    double *p = igrid > 0 ? unew + (size_t)(igrid - 1) * 5 * ttd + (icell - 1) : nullptr;
-    double acc[5];
+    double *p = igrid > 0 ? unew + (size_t)(igrid - 1) * 5 * ttd + n * ttd + (icell - 1) : nullptr;
+    double acc = 0.0;
     bool touched = false;
     for (int k = 0; k < nslot; k++) {
-        double f[5];
-        bool any = false;
-#pragma unroll
-        for (int n = 0; n < 5; n++) {
-            f[n] = rg[5 * k + n];
-            any = any || f[n] != 0.0;
-        }
-        if (!any) continue;
-#pragma unroll
-        for (int n = 0; n < 5; n++) rg[5 * k + n] = 0.0;
+        const double f = rg[5 * k];
+        if (f == 0.0) continue;
+        rg[5 * k] = 0.0;
         if (!p) continue;  // parent in a boundary oct: the reference drops it with the cache oct
-        if (!touched) {
-#pragma unroll
-            for (int n = 0; n < 5; n++) acc[n] = p[n * ttd];
-            touched = true;
-        }
-#pragma unroll
-        for (int n = 0; n < 5; n++) acc[n] = acc[n] + f[n];
+        if (!touched) acc = *p;
+        touched = true;
+        acc = acc + f;
     }
-    if (touched)
-#pragma unroll
-        for (int n = 0; n < 5; n++) p[n * ttd] = acc[n];
+    if (touched) *p = acc;
 }
 
 // Fixed-order reduction of the per-block partials by one 256-thread block:
@@ -1284,15 +1276,75 @@ __device__ __forceinline__ void cell_xc(int ndim, int ind, double xc[3])
     xc[2] = ndim > 2 ? (double)iz - 0.5 : 0.0;
 }
 
-// interpol_hydro (hydro/interpol_hydro.f90:5-113) with the limiters of
-// :610-752; u1[j][ivar], j = 0 (central parent) and 1..2ndim (-x,+x,-y,+y,-z,+z).
-// ND is a compile-time constant so that every loop unrolls and u1/u2 stay in
-// registers (a runtime ndim put them in scratch memory).
+// One variable of interpol_hydro (hydro/interpol_hydro.f90:5-113) with the
+// limiters of :610-752; a[j], j = 0 (central parent) and 1..2ndim
+// (-x,+x,-y,+y,-z,+z).  ND is a compile-time constant so that every loop
+// unrolls and the arrays stay in registers (a runtime ndim put them in scratch
+// memory).
+template <int ND>
+__device__ __forceinline__ void interpol_var_dev(const double a[7], double u[8], int interpol_type)
+{
+    constexpr int ndim = ND, twondim = 2 * ND, ttd = 1 << ND;
+    double w[3] = {0, 0, 0};
+    if (interpol_type == 1) {
+        #pragma unroll
+        for (int d = 1; d <= ndim; d++) {
+            const double dl = 0.5 * (a[2 * d] - a[0]), dr = 0.5 * (a[0] - a[2 * d - 1]);
+            w[d - 1] = (dl * dr <= 0.0) ? 0.0 : fmin(fabs(dl), fabs(dr)) * dl / fabs(dl);
+        }
+    } else if (interpol_type == 2 || interpol_type == 3) {
+        #pragma unroll
+        for (int d = 1; d <= ndim; d++) w[d - 1] = 0.25 * (a[2 * d] - a[2 * d - 1]);
+        if (interpol_type == 2) {
+            double ac[8];
+            #pragma unroll
+            for (int c = 0; c < ttd; c++) ac[c] = a[0];
+            #pragma unroll
+            for (int d = 1; d <= ndim; d++)
+                #pragma unroll
+                for (int c = 1; c <= ttd; c++) {
+                    double xc[3];
+                    cell_xc(ndim, c, xc);
+                    ac[c - 1] = ac[c - 1] + 2.0 * w[d - 1] * xc[d - 1];
+                }
+            double cmax = ac[0], cmin = ac[0], kmax = a[1], kmin = a[1];
+            #pragma unroll
+            for (int c = 1; c < ttd; c++) {
+                cmax = fmax(cmax, ac[c]);
+                cmin = fmin(cmin, ac[c]);
+            }
+            #pragma unroll
+            for (int j = 2; j <= twondim; j++) {
+                kmax = fmax(kmax, a[j]);
+                kmin = fmin(kmin, a[j]);
+            }
+            double dk = a[0] - kmax, dc = a[0] - cmax;
+            const double lmax = (dk * dc > 0.0) ? fmin(1.0, dk / dc) : 0.0;
+            dk = a[0] - kmin;
+            dc = a[0] - cmin;
+            const double lmin = (dk * dc > 0.0) ? fmin(1.0, dk / dc) : 0.0;
+            const double lim = fmin(lmin, lmax);
+            #pragma unroll
+            for (int d = 0; d < ndim; d++) w[d] = w[d] * lim;
+        }
+    }
+    #pragma unroll
+    for (int c = 1; c <= ttd; c++) {
+        double xc[3];
+        cell_xc(ndim, c, xc);
+        double v = a[0];
+        #pragma unroll
+        for (int d = 1; d <= ndim; d++) v = v + w[d - 1] * xc[d - 1];
+        u[c - 1] = v;
+    }
+}
+
+// All five variables, u1[j][ivar].
 template <int ND>
 __device__ __forceinline__ void interpol_hydro_dev(double u1[7][5], double u2[8][5], int interpol_var, int interpol_type,
                                    double smallr)
 {
-    constexpr int ndim = ND, twondim = 2 * ND, ttd = 1 << ND;
+    constexpr int twondim = 2 * ND, ttd = 1 << ND;
     if (interpol_var == 1)
         #pragma unroll
         for (int j = 0; j <= twondim; j++) {
@@ -1303,60 +1355,12 @@ __device__ __forceinline__ void interpol_hydro_dev(double u1[7][5], double u2[8]
         }
 #pragma unroll
     for (int iv = 0; iv < 5; iv++) {
-        double a[7], w[3] = {0, 0, 0};
+        double a[7], u[8];
         #pragma unroll
         for (int j = 0; j <= twondim; j++) a[j] = u1[j][iv];
-        if (interpol_type == 1) {
-            #pragma unroll
-            for (int d = 1; d <= ndim; d++) {
-                const double dl = 0.5 * (a[2 * d] - a[0]), dr = 0.5 * (a[0] - a[2 * d - 1]);
-                w[d - 1] = (dl * dr <= 0.0) ? 0.0 : fmin(fabs(dl), fabs(dr)) * dl / fabs(dl);
-            }
-        } else if (interpol_type == 2 || interpol_type == 3) {
-            #pragma unroll
-            for (int d = 1; d <= ndim; d++) w[d - 1] = 0.25 * (a[2 * d] - a[2 * d - 1]);
-            if (interpol_type == 2) {
-                double ac[8];
-                #pragma unroll
-                for (int c = 0; c < ttd; c++) ac[c] = a[0];
-                #pragma unroll
-                for (int d = 1; d <= ndim; d++)
-                    #pragma unroll
-                    for (int c = 1; c <= ttd; c++) {
-                        double xc[3];
-                        cell_xc(ndim, c, xc);
-                        ac[c - 1] = ac[c - 1] + 2.0 * w[d - 1] * xc[d - 1];
-                    }
-                double cmax = ac[0], cmin = ac[0], kmax = a[1], kmin = a[1];
-                #pragma unroll
-                for (int c = 1; c < ttd; c++) {
-                    cmax = fmax(cmax, ac[c]);
-                    cmin = fmin(cmin, ac[c]);
-                }
-                #pragma unroll
-                for (int j = 2; j <= twondim; j++) {
-                    kmax = fmax(kmax, a[j]);
-                    kmin = fmin(kmin, a[j]);
-                }
-                double dk = a[0] - kmax, dc = a[0] - cmax;
-                const double lmax = (dk * dc > 0.0) ? fmin(1.0, dk / dc) : 0.0;
-                dk = a[0] - kmin;
-                dc = a[0] - cmin;
-                const double lmin = (dk * dc > 0.0) ? fmin(1.0, dk / dc) : 0.0;
-                const double lim = fmin(lmin, lmax);
-                #pragma unroll
-                for (int d = 0; d < ndim; d++) w[d] = w[d] * lim;
-            }
-        }
+        interpol_var_dev<ND>(a, u, interpol_type);
         #pragma unroll
-        for (int c = 1; c <= ttd; c++) {
-            double xc[3];
-            cell_xc(ndim, c, xc);
-            double v = a[0];
-            #pragma unroll
-            for (int d = 1; d <= ndim; d++) v = v + w[d - 1] * xc[d - 1];
-            u2[c - 1][iv] = v;
-        }
+        for (int c = 0; c < ttd; c++) u2[c][iv] = u[c];
     }
     if (interpol_var == 1)
         #pragma unroll
@@ -1451,10 +1455,82 @@ __global__ void __launch_bounds__(64) k_refresh_ghosts(const GhostArgs a)
     }
 }
 
+// k_refresh_ghosts<3> where the variables are interpolated independently
+// (interpol_var = 0): 64 ghosts per block, one wave per variable.  The refresh
+// is bound by the latency of its dependent gathers (order, source, cell); one
+// thread per ghost held 35 values, two waves per SIMD, and a mesh's ghosts did
+// not even fill those.  A thread per ghost and variable has a fifth of the
+// loads, five times the threads and the registers for all of them at once.
+// 4.9 M cells on five levels: 67.9 -> 57.7 us; 1.1 M cells on four: 10.5 -> 7.5.
+__global__ void __launch_bounds__(320) k_refresh_ghosts_var(const GhostArgs a)
+{
+    // (ghosts in parent-cell order and staged stores: see k_refresh_ghosts)
+    const int lane = threadIdx.x & 63, n = threadIdx.x >> 6;
+    const int t = xcd_block(blockIdx.x, gridDim.x) * 64 + lane;
+    int g = -1;
+    double u[8];
+    if (t < a.nghost) {
+        int k = 0;
+        for (int j = 1; j < a.nseg; j++) k = t >= a.seg_t[j] ? j : k;
+        const int pos = a.seg_o[k] + (t - a.seg_t[k]);
+        int code[7], ind[7];
+        g = a.order[pos] - a.gi0;
+#pragma unroll
+        for (int j = 0; j < 7; j++) {
+            code[j] = a.src[(size_t)(2 * j) * a.src_ld + pos];
+            ind[j] = a.src[(size_t)(2 * j + 1) * a.src_ld + pos] - 1;
+        }
+        const int boxmin[3] = {a.seg_box[k][0], a.seg_box[k][1], a.seg_box[k][2]};
+        const int boxmax[3] = {a.seg_box[k][3], a.seg_box[k][4], a.seg_box[k][5]};
+        const int refl = reflexive_mask(a.btype);
+        const double *p[7];
+        bool neg[7];
+#pragma unroll
+        for (int j = 0; j < 7; j++) {
+            p[j] = code[j] > 0 ? a.uold + (size_t)(code[j] - 1) * 40 + ind[j] + 8 * n : a.uold;
+            neg[j] = false;
+            if (code[j] < 0) {
+                // the source's oct key locates boundary ghosts only
+                const int *key = a.srckey + (g * 7 + j) * 3;
+                const int okey[3] = {key[0], key[1], key[2]};
+                const int c[3] = {ind[j] & 1, (ind[j] >> 1) & 1, (ind[j] >> 2) & 1};
+                const CellRef r = cell_ref3(a.uold, a.refined, code[j], okey, boxmin, boxmax, refl, c);
+                p[j] = r.p + 8 * n;
+                neg[j] = r.flip >= 0 && r.flip == n - 1;
+            }
+        }
+        double v[7];
+#pragma unroll
+        for (int j = 0; j < 7; j++) v[j] = *p[j];
+#pragma unroll
+        for (int j = 0; j < 7; j++) {
+            v[j] = code[j] == 0 ? 0.0 : v[j];
+            v[j] = neg[j] ? -v[j] : v[j];
+        }
+        interpol_var_dev<3>(v, u, a.interpol_type);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = 0.0;
+    }
+    __shared__ double2 sm[5][64 * 4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) sm[n][lane * 4 + c] = make_double2(u[2 * c], u[2 * c + 1]);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int gq = __shfl(g, (q * 64 + lane) >> 2);
+        if (gq >= 0)
+            reinterpret_cast<double2 *>(a.uold + (size_t)(a.first - 1 + gq) * 40)[n * 4 + (lane & 3)] =
+                sm[n][q * 64 + lane];
+    }
+}
+
 hipError_t launch_refresh_ghosts(const GhostArgs &a, hipStream_t s)
 {
     if (a.nghost <= 0) return hipSuccess;
-    if (a.ndim == 3)
+    if (a.ndim == 3 && a.interpol_var == 0)
+        hipLaunchKernelGGL(k_refresh_ghosts_var, dim3((a.nghost + 63) / 64), dim3(320), 0, s, a);
+    else if (a.ndim == 3)
         hipLaunchKernelGGL(k_refresh_ghosts<3>, dim3((a.nghost + 63) / 64), dim3(64), 0, s, a);
     else
         hipLaunchKernelGGL(k_refresh_ghosts<1>, dim3((a.nghost + 63) / 64), dim3(64), 0, s, a);
@@ -1857,7 +1933,7 @@ hipError_t launch_reflux_fold(double *unew, double *racc, const int32_t *ghost_p
                               int nghost, int ttd, hipStream_t s, int nslot)
 {
     if (nghost <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_reflux_fold, dim3((nghost + 255) / 256), dim3(256), 0, s, unew, racc, ghost_parent, order,
+    hipLaunchKernelGGL(k_reflux_fold, dim3((unsigned)((5l * nghost + 255) / 256)), dim3(256), 0, s, unew, racc, ghost_parent, order,
                        nghost, ttd, nslot);
     return hipGetLastError();
 }
