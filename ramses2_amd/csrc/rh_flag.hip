@@ -32,35 +32,35 @@ struct FlagArgs {
     int periodic[3];
     int refl;                 // reflexive faces (bit 2*dim+side)
     double gamma, smallr, err_d, err_p, floor_d, floor_p;
-    int *counter;             // [0] cells newly flagged, [1] a neighbour's cell missing
+    int *counter;             // [1] a neighbour's cell missing
 };
 
-// hydro_refine's density and pressure tests for one direction (ug, um, ud:
-// left, cell, right conservative states), in the reference's order.
-__device__ bool refine_dp(const FlagArgs &a, double ug[5], double um[5], double ud[5])
+// Density and pressure of a cell as hydro_refine forms them from a
+// conservative state, in the reference's order.
+__device__ __forceinline__ void cell_dp(const FlagArgs &a, const double u[5], double &r, double &p)
 {
 #pragma clang fp contract(off)
-    ug[0] = ug[0] > a.smallr ? ug[0] : a.smallr;
-    um[0] = um[0] > a.smallr ? um[0] : a.smallr;
-    ud[0] = ud[0] > a.smallr ? ud[0] : a.smallr;
+    r = u[0] > a.smallr ? u[0] : a.smallr;
+    double ekin = 0.0;
+#pragma unroll
     for (int d = 1; d <= 3; d++) {
-        ug[d] = ug[d] / ug[0];
-        um[d] = um[d] / um[0];
-        ud[d] = ud[d] / ud[0];
+        const double v = u[d] / r;
+        ekin = ekin + 0.5 * r * (v * v);
     }
-    double eking = 0.0, ekinm = 0.0, ekind = 0.0;
-    for (int d = 1; d <= 3; d++) {
-        eking = eking + 0.5 * ug[0] * (ug[d] * ug[d]);
-        ekinm = ekinm + 0.5 * um[0] * (um[d] * um[d]);
-        ekind = ekind + 0.5 * ud[0] * (ud[d] * ud[d]);
-    }
-    const double pg = (a.gamma - 1.0) * (ug[4] - eking);
-    const double pm = (a.gamma - 1.0) * (um[4] - ekinm);
-    const double pd = (a.gamma - 1.0) * (ud[4] - ekind);
+    p = (a.gamma - 1.0) * (u[4] - ekin);
+}
+
+// hydro_refine's density and pressure tests for one direction (densities and
+// pressures of the left cell, the cell and the right cell), in the reference's
+// order.
+__device__ __forceinline__ bool refine_dp(const FlagArgs &a, double rg, double pg, double rm, double pm, double rd,
+                                          double pd)
+{
+#pragma clang fp contract(off)
     bool ok = false;
     if (a.err_d >= 0.0) {
-        const double x = __builtin_fabs((ud[0] - um[0]) / (ud[0] + um[0] + a.floor_d));
-        const double y = __builtin_fabs((um[0] - ug[0]) / (um[0] + ug[0] + a.floor_d));
+        const double x = __builtin_fabs((rd - rm) / (rd + rm + a.floor_d));
+        const double y = __builtin_fabs((rm - rg) / (rm + rg + a.floor_d));
         ok = ok || 2.0 * (x > y ? x : y) > a.err_d;
     }
     if (a.err_p >= 0.0) {
@@ -71,67 +71,81 @@ __device__ bool refine_dp(const FlagArgs &a, double ug[5], double um[5], double 
     return ok;
 }
 
+// Eight lanes per oct, one per cell.  The pass is bound by the latency of its
+// dependent gathers (key, hash table, cell), so the lanes share them: six of
+// them look up one neighbour oct each (a lookup per cell and neighbour was
+// eight times as many), and of a cell's six neighbours the three in its own oct
+// give their density and pressure through the lanes, so four cells are read and
+// divided per lane instead of seven.  No count is kept (one address that every
+// flagged cell added to).  96 -> 26 us per level on average, 297 k octs on five
+// levels.
 __global__ void __launch_bounds__(256) k_hydro_flag(const FlagArgs a)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)a.noct * 8) return;
-    const int o = a.head - 1 + (int)(i >> 3), ind = (int)(i & 7);
-    int hk[3];
-    for (int d = 0; d < 3; d++) hk[d] = 2 * a.ckey[3 * o + d] + ((ind >> d) & 1);
-    double un[6][5];
-    for (int nb = 0; nb < 6; nb++) {
-        int kn[3] = {hk[0], hk[1], hk[2]};
-        const int d0 = nb >> 1;
-        kn[d0] += (nb & 1) ? 1 : -1;
-        if (a.periodic[d0]) {
-            if (kn[d0] < a.cmin[d0]) kn[d0] = a.cmax[d0] - 1;
-            if (kn[d0] >= a.cmax[d0]) kn[d0] = a.cmin[d0];
+    if (i >= (long)a.noct * 8) return;  // (whole octs: the eight lanes of one leave together)
+    const int o = a.head - 1 + (int)(i >> 3), ind = (int)(i & 7), oct0 = threadIdx.x & 56;
+    const int ck[3] = {a.ckey[3 * o], a.ckey[3 * o + 1], a.ckey[3 * o + 2]};
+    // the neighbour cell across side sd of the oct in dimension d: the key kp of
+    // its oct, its place c there
+    auto beyond = [&](int d, int sd, int kp[3], int c[3]) {
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+            int kn = 2 * ck[e] + ((ind >> e) & 1);
+            if (e == d) {
+                kn = 2 * ck[e] + (sd ? 2 : -1);
+                if (a.periodic[e]) {
+                    if (kn < a.cmin[e]) kn = a.cmax[e] - 1;
+                    if (kn >= a.cmax[e]) kn = a.cmin[e];
+                }
+            }
+            kp[e] = kn >> 1;
+            c[e] = kn & 1;
         }
+    };
+    // lane 2d + sd of the oct: the oct there, or the one of level l-1 that holds
+    // the neighbour cells where it is not one of the level's own; 0: neither
+    int nb = 0, up = 0;
+    if (ind < 6) {
         int kp[3], c[3];
-        for (int d = 0; d < 3; d++) {
-            kp[d] = kn[d] >> 1;
-            c[d] = kn[d] & 1;
+        beyond(ind >> 1, ind & 1, kp, c);
+        nb = resolve_oct(a.fine, kp[0], kp[1], kp[2]);
+        if (nb > a.fine.ngridmax || nb == 0) {
+            up = 1;
+            nb = a.coarse.nx ? resolve_oct(a.coarse, kp[0] >> 1, kp[1] >> 1, kp[2] >> 1) : 0;
+            if (nb > a.coarse.ngridmax) nb = 0;
         }
-        int v = resolve_oct(a.fine, kp[0], kp[1], kp[2]);
-        const int *bmin = a.fine.boxmin, *bmax = a.fine.boxmax;
-        if (v > a.fine.ngridmax || v == 0) {
-            // not one of the level's octs: the level l-1 cell holding the neighbour
-            int kq[3];
-            for (int d = 0; d < 3; d++) {
-                c[d] = kp[d] & 1;
-                kq[d] = kp[d] >> 1;
-            }
-            v = a.coarse.nx ? resolve_oct(a.coarse, kq[0], kq[1], kq[2]) : 0;
-            if (v > a.coarse.ngridmax || v == 0) {
-                atomicOr(&a.counter[1], 1);
-                return;
-            }
-            for (int d = 0; d < 3; d++) kp[d] = kq[d];
-            bmin = a.coarse.boxmin;
-            bmax = a.coarse.boxmax;
-        }
-        const CellRef r = cell_ref3(a.uold, a.refined, v, kp, bmin, bmax, a.refl, c);
-        uint8_t rf;
-        cell_load3(r, un[nb], rf);
-        cell_flip(un[nb], r.flip);
     }
-    double um0[5];
-    for (int n = 0; n < 5; n++) um0[n] = a.uold[(size_t)o * 40 + n * 8 + ind];
-    bool ok = false;
+    double um[5], r0, p0;
+#pragma unroll
+    for (int n = 0; n < 5; n++) um[n] = a.uold[(size_t)o * 40 + n * 8 + ind];
+    cell_dp(a, um, r0, p0);
+    bool ok = false, missing = false;
+#pragma unroll
     for (int d = 0; d < 3; d++) {
-        double ug[5], um[5], ud[5];
-        for (int n = 0; n < 5; n++) {
-            ug[n] = un[2 * d][n];
-            um[n] = um0[n];
-            ud[n] = un[2 * d + 1][n];
-        }
-        ok = refine_dp(a, ug, um, ud) || ok;
+        const int sd = (ind >> d) & 1;
+        const int v = __shfl(nb, oct0 + 2 * d + sd), u = __shfl(up, oct0 + 2 * d + sd);
+        const double rs = __shfl_xor(r0, 1 << d), ps = __shfl_xor(p0, 1 << d);
+        int kp[3], c[3];
+        beyond(d, sd, kp, c);
+        if (u)
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                c[e] = kp[e] & 1;
+                kp[e] >>= 1;
+            }
+        missing = missing || v == 0;
+        const CellRef cr = cell_ref3(a.uold, a.refined, v, kp, u ? a.coarse.boxmin : a.fine.boxmin,
+                                     u ? a.coarse.boxmax : a.fine.boxmax, a.refl, c);
+        double un[5], rn, pn;
+#pragma unroll
+        for (int n = 0; n < 5; n++) un[n] = cr.p ? cr.p[8 * n] : 0.0;
+        cell_dp(a, un, rn, pn);  // (a reflexive ghost's momentum sign drops out)
+        ok = refine_dp(a, sd ? rs : rn, sd ? ps : pn, r0, p0, sd ? rn : rs, sd ? pn : ps) || ok;
     }
-    if (ok) {
-        int32_t *f = a.flag1 + (size_t)o * 8 + ind;
-        if (*f == 0) atomicAdd(&a.counter[0], 1);
-        *f = 1;
-    }
+    if (missing)
+        atomicOr(&a.counter[1], 1);
+    else if (ok)
+        a.flag1[(size_t)o * 8 + ind] = 1;
 }
 
 __global__ void k_fill_flag1(int32_t *flag1, long first, long n, int32_t v)
@@ -140,12 +154,23 @@ __global__ void k_fill_flag1(int32_t *flag1, long first, long n, int32_t v)
     if (i < n) flag1[first + i] = v;
 }
 
-__global__ void k_count_flag1(const int32_t *flag1, long first, long n, int *count)
+// Nonzero flags of n/8 octs (n is a multiple of 8), one atomic per block of a
+// grid of at most kCountBlocks: device-scope additions to one address take
+// about 40 ns each, one after another (a sum per wave: 40 us, now 3.8).
+constexpr int kCountBlocks = 128;
+__global__ void __launch_bounds__(256) k_count_flag1(const int4 *__restrict__ flag, long n4, int *count)
 {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    int v = i < n && flag1[first + i] != 0 ? 1 : 0;
+    int v = 0;
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (long)gridDim.x * blockDim.x) {
+        const int4 f = flag[i];
+        v += (f.x != 0) + (f.y != 0) + (f.z != 0) + (f.w != 0);
+    }
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd(count, v);
+    __shared__ int w[4];
+    if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = w[0] + w[1] + w[2] + w[3];
+    if (threadIdx.x == 0 && v) atomicAdd(count, v);
 }
 
 }  // namespace rh
@@ -281,8 +306,9 @@ int rh_count_flag1(int head_idx, int num_octs, int32_t *count)
     if (num_octs == 0) return 0;
     const long n = (long)num_octs * 8;
     RH_HIP_CHECK(hipMemsetAsync(s.d_counter, 0, sizeof(int), s.stream));
-    hipLaunchKernelGGL(k_count_flag1, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s.stream, s.flag1,
-                       (long)(head_idx - 1) * 8, n, s.d_counter);
+    const long n4 = n / 4, nb = (n4 + 255) / 256;
+    hipLaunchKernelGGL(k_count_flag1, dim3((unsigned)(nb < kCountBlocks ? nb : kCountBlocks)), dim3(256), 0, s.stream,
+                       (const int4 *)(s.flag1 + (size_t)(head_idx - 1) * 8), n4, s.d_counter);
     RH_HIP_CHECK(hipGetLastError());
     int c = 0;
     RH_HIP_CHECK(hipMemcpyAsync(&c, s.d_counter, sizeof(int), hipMemcpyDeviceToHost, s.stream));
