@@ -63,6 +63,11 @@ int rh_get_brick_shape(int32_t *bx, int32_t *by, int32_t *bz);
  * copy happens when capacity >= *len (else RH_ERR_ARG). */
 int rh_get_level_table(int ilevel, int which, int32_t *out, int64_t capacity, int64_t *len);
 
+/* Refinement flags (8 per oct) of octs head_idx .. head_idx+num_octs-1 into
+ * flag1[8*num_octs]: rh_transfer_flag1_host copies the whole mesh's, once per
+ * level when each level is flagged in turn. */
+int rh_get_flag1(int head_idx, int num_octs, int32_t *flag1);
+
 /* The brick lattice rh_build_nbor gives a 3D level whose octs have these keys
  * ([noct][3], each >= box_min): bricks of bx*by*bz octs with origins at
  * box_min + off + multiples of the shape, off chosen per level to minimise

@@ -36,6 +36,7 @@ SIGNATURES = {
     "rh_job_status": [_c, _dp],
     "rh_fence_record": [_ip, _c, _ip],
     "rh_fence_wait": [_c, _dp],
+    "rh_get_flag1": [_c, _c, _ip],
     "rh_get_level_table": [_c, _c, _ip, ctypes.c_int64, ctypes.POINTER(ctypes.c_int64)],
     "rh_brick_lattice": [_ip, _c, _ip, _ip, _c, _c, _c, _ip, _dp],
 }

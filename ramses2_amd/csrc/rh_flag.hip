@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/ramses2_hip.h"
+#include "../../include/ramses2_hip_ext.h"
 #include "rh_gather.h"
 #include "rh_mesh.h"
 #include "rh_state.h"
@@ -324,6 +325,19 @@ int rh_upload_flag1(const int32_t *flag1, int ngridmax)
     if (!flag1 || ngridmax != s.ngridmax) return efail(RH_ERR_ARG, "rh_upload_flag1: flag1(8, ngridmax) expected");
     RH_HIP_CHECK(hipMemcpyAsync(s.flag1, flag1, (size_t)ngridmax * 8 * sizeof(int32_t), hipMemcpyHostToDevice,
                                 s.stream));
+    RH_HIP_CHECK(hipStreamSynchronize(s.stream));
+    return 0;
+}
+
+int rh_get_flag1(int head_idx, int num_octs, int32_t *flag1)
+{
+    if (int r = ensure_flag1()) return r;
+    if (int r = oct_range(head_idx, num_octs)) return r;
+    if (num_octs == 0) return 0;
+    if (!flag1) return efail(RH_ERR_ARG, "rh_get_flag1: null flag1");
+    State &s = st();
+    RH_HIP_CHECK(hipMemcpyAsync(flag1, s.flag1 + (size_t)(head_idx - 1) * 8, (size_t)num_octs * 8 * sizeof(int32_t),
+                                hipMemcpyDeviceToHost, s.stream));
     RH_HIP_CHECK(hipStreamSynchronize(s.stream));
     return 0;
 }

@@ -107,9 +107,9 @@ class HipHydro:
              float(floor_d), float(floor_p))
         n = ctypes.c_int32()
         call("rh_count_flag1", head, num, ctypes.byref(n))
-        f = np.zeros((self.ngrid, 8), dtype=np.int32)
-        call("rh_transfer_flag1_host", ptr(f, _lib._ip), self.ngrid)
-        return f[head - 1:head - 1 + num], n.value
+        f = np.empty((num, 8), dtype=np.int32)
+        call("rh_get_flag1", head, num, ptr(f, _lib._ip))
+        return f, n.value
 
     def level_table(self, ilevel, which):
         """One of the level's device index tables (rh_get_level_table) as a
