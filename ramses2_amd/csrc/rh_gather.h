@@ -17,6 +17,72 @@ __device__ __forceinline__ int reflexive_mask(const int btype[3][2])
     return refl;
 }
 
+// Gather the conservative state of cell (i2,j2,k2) of the oct at window slot
+// value v, whose oct key is okey.  Boundary ghosts (v<0) follow
+// init_bound_refine (amr/boundaries.f90:39-165): zero gradient copies the
+// adjacent interior cell, reflexive mirrors it and flips the normal momentum.
+// refl: bit 2*d+side set where that face of the domain is reflexive
+// (bound_type 1), else zero gradient (bound_type 2).
+__device__ __forceinline__ void gather_cell_m(const double *__restrict__ uold, const uint8_t *__restrict__ refined,
+                                              int v, const int okey[3], int ndim, const int boxmin[3],
+                                              const int boxmax[3], int refl, int c[3], double u[5], uint8_t &rf)
+{
+    if (v > 0) {
+        const int ind = c[0] + 2 * c[1] + 4 * c[2];
+        const double *p = uold + (size_t)(v - 1) * 40 + ind;
+        if (ndim == 1) p = uold + (size_t)(v - 1) * 10 + ind;
+        const int stride = ndim == 1 ? 2 : 8;
+#pragma unroll
+        for (int n = 0; n < 5; n++) u[n] = p[n * stride];
+        rf = refined[(size_t)(v - 1) * 8 + ind];
+        return;
+    }
+    if (v == 0) {
+#pragma unroll
+        for (int n = 0; n < 5; n++) u[n] = 0.0;
+        rf = 0;
+        return;
+    }
+    // boundary ghost: first direction in which the oct key leaves the domain
+    int dir = 0, side = 0;
+    for (int d = ndim - 1; d >= 0; d--) {
+        if (okey[d] < boxmin[d]) { dir = d; side = 0; }
+        else if (okey[d] >= boxmax[d]) { dir = d; side = 1; }
+    }
+    const int type = (refl >> (2 * dir + side)) & 1 ? 1 : 2;
+    int s[3] = {c[0], c[1], c[2]};
+    uint8_t rflag_src_valid;
+    int rs[3] = {c[0], c[1], c[2]};
+    if (side == 0) {
+        // reference oct lies at +1: refined(ind) = ref cell with c_dir-1 (ref_right)
+        rflag_src_valid = c[dir] == 1;
+        rs[dir] = 0;
+    } else {
+        rflag_src_valid = c[dir] == 0;
+        rs[dir] = 1;
+    }
+    if (type == 1)
+        s[dir] = 1 - c[dir];
+    else
+        s[dir] = side == 0 ? 0 : 1;
+    const int ref = -v;
+    const int ind = s[0] + 2 * s[1] + 4 * s[2];
+    const int stride = ndim == 1 ? 2 : 8;
+    const double *p = uold + (size_t)(ref - 1) * 5 * stride + ind;
+#pragma unroll
+    for (int n = 0; n < 5; n++) u[n] = p[n * stride];
+    if (type == 1) u[1 + dir] = -u[1 + dir];
+    rf = rflag_src_valid ? refined[(size_t)(ref - 1) * 8 + rs[0] + 2 * rs[1] + 4 * rs[2]] : 0;
+}
+
+__device__ __forceinline__ void gather_cell(const double *__restrict__ uold, const uint8_t *__restrict__ refined,
+                                            int v, const int okey[3], int ndim, const int boxmin[3],
+                                            const int boxmax[3], const int btype[3][2], int c[3], double u[5],
+                                            uint8_t &rf)
+{
+    gather_cell_m(uold, refined, v, okey, ndim, boxmin, boxmax, reflexive_mask(btype), c, u, rf);
+}
+
 // gather_cell_m for 3D split into the address computation and the loads, so
 // that the loads of the next plane can be issued a plane ahead: the cell's
 // five values start at p (stride 8; null: no oct, zero state), its refined
