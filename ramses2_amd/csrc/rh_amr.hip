@@ -9,9 +9,10 @@
 //      go to a per-ghost-oct accumulator, because the parent cell's own update
 //      runs in the same launch;
 //   3. the accumulated refluxes are added to the parent cells;
-//   4. upload_fine, finest level first;
-//   5. courant_fine over the leaf cells of all levels in one pass: the dt of
-//      the next step and the conservation sums, kept on the device.
+//   4. upload_fine, finest level first, and with each level's octs its leaf
+//      cells' share of courant_fine (two passes where interpol_var = 1);
+//   5. the reduction of the Courant partials: the dt of the next step and the
+//      conservation sums, kept on the device.
 // The arrays then swap roles.  A pair of steps can be captured as a hipGraph.
 #include <hip/hip_runtime.h>
 
@@ -103,6 +104,17 @@ hipError_t enqueue_amr_step(State &s, int parity, int precision)
     if ((e = launch_reflux_fold(unext, m.racc, s.ghost_parent, s.ghost_order, s.nghost_total, 8, s.stream,
                                 m.nslot)) != hipSuccess)
         return e;
+    if (s.interpol_var != 1) {
+        std::vector<UploadLevel> lv;
+        for (size_t i = 0; i < m.levels.size(); i++) {
+            const int l = m.levels[i];
+            const bool up = i > 0 && m.levels[i - 1] == l - 1;
+            lv.push_back(UploadLevel{up ? s.nbors.at(l).father : nullptr, m.h_descs[i].head, m.h_descs[i].noct, l});
+        }
+        return launch_upload_courant(unext, s.refined, lv.data(), (int)lv.size(), m.boxlen, m.dx_finest, m.gamma,
+                                     m.smallr, __builtin_sqrt(m.smallc2), m.courant, m.g, s.red_part, s.red_cap,
+                                     s.red_out, s.dt_dev, s.stream, s.t_dev, precision == 1);
+    }
     for (int i = (int)m.levels.size() - 1; i >= 1; i--) {
         const int lf = m.levels[i];
         if (m.levels[i - 1] != lf - 1) continue;

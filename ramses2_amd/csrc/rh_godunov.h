@@ -166,6 +166,17 @@ hipError_t launch_courant_ml(const double *uold, const uint8_t *refined, const i
                              double boxlen, double dx_finest, double gamma, double smallr, double smallc,
                              double courant_factor, const double g[3], double *partials, int max_blocks, double *out,
                              double *dt_out, hipStream_t s, double *t_acc, bool mixed = false);
+// Restriction of the levels lv[0 .. nlev) (coarse to fine, 3D, interpol_var = 0)
+// and launch_courant_ml's pass over them in one read of each level's octs;
+// max_parts partials of 4 doubles.  father null: not restricted.
+struct UploadLevel {
+    const int32_t *father;
+    int head, noct, level;
+};
+hipError_t launch_upload_courant(double *uold, const uint8_t *refined, const UploadLevel *lv, int nlev, double boxlen,
+                                 double dx_finest, double gamma, double smallr, double smallc, double courant_factor,
+                                 const double g[3], double *partials, int max_parts, double *out, double *dt_out,
+                                 hipStream_t s, double *t_acc, bool mixed);
 // racc[0 .. 5*n) = 0 (a kernel: safe inside captured graphs)
 hipError_t launch_zero(double *p, long n, hipStream_t s);
 // unew(parent cell of ghost g) += the nslot accumulators of g (racc[5*nslot*g
