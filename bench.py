@@ -576,7 +576,7 @@ def main():
         traffic = load_traffic(bricks[0])
         roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                "kernel": "k_godunov3d<%d,%d,%d,double> (FP64)" % bricks[0], "kernel_ms": kms64,
+                "kernel": "k_brick64<%d,%d,%d> (FP64)" % bricks[0], "kernel_ms": kms64,
                 "bytes_per_launch": BYTES_PER_CELL * ncells}
         valu = valu_ceiling(bricks[0], ncells, kms64)
         if valu:
