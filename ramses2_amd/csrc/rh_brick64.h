@@ -25,10 +25,10 @@
 // halo loop solves one face per lane, converts the ring and updates nothing.
 // Measured against the one-body kernel this replaced (four barriers, every
 // thread testing its role, the expressions of rh_physics.h), with the Courant
-// reduction: 256^3 in 8x6x16 bricks 843 -> 660 us (25.4 G cell-updates/s, 2.0
+// reduction: 256^3 in 8x6x16 bricks 843 -> 641 us (26.2 G cell-updates/s, 2.1
 // TB/s of the 80 algorithmic bytes per cell; 680 with the column's own low faces
 // read back from LDS and two reciprocals per HLLC face), 128^3 in 8x6x8 bricks
-// 140 -> 106 us, 90^3 MinMod + LLF (a run-time solver choice before) 105 -> 64 us.
+// 140 -> 103 us, 90^3 MinMod + LLF (a run-time solver choice before) 105 -> 64 us.
 #pragma once
 #include <type_traits>
 
