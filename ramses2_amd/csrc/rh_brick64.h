@@ -25,10 +25,10 @@
 // halo loop solves one face per lane, converts the ring and updates nothing.
 // Measured against the one-body kernel this replaced (four barriers, every
 // thread testing its role, the expressions of rh_physics.h), with the Courant
-// reduction: 256^3 in 8x6x16 bricks 843 -> 641 us (26.2 G cell-updates/s, 2.1
+// reduction: 256^3 in 8x6x16 bricks 843 -> 629 us (26.7 G cell-updates/s, 2.1
 // TB/s of the 80 algorithmic bytes per cell; 680 with the column's own low faces
 // read back from LDS and two reciprocals per HLLC face), 128^3 in 8x6x8 bricks
-// 140 -> 103 us, 90^3 MinMod + LLF (a run-time solver choice before) 105 -> 64 us.
+// 140 -> 100 us, 90^3 MinMod + LLF (a run-time solver choice before) 105 -> 64 us.
 #pragma once
 #include <type_traits>
 
@@ -78,6 +78,13 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
 {
 #pragma clang fp contract(off)
     constexpr bool GEN = KIND != kBrickUniform;
+    // Phase A, whose LDS reads wait most, runs at a raised wave priority, so that
+    // the CU's other workgroup fills its gaps with solves instead of delaying
+    // it.  Workgroups of four waves and more, of which two share a CU: 8x6x16
+    // at 256^3 646 -> 629 us, 8x6x8 at 128^3 104 -> 100, 7x7x8 at 128^3 135 ->
+    // 129.  With four workgroups of two waves the raised ones starve the others:
+    // 4x4x8 at 128^3 125 -> 136 us.
+    constexpr bool kPrioA = (2 * BX + 2) * (2 * BY + 2) > 192;
     constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY, NI = 4 * BX * BY;
     constexpr int PX = 2 * BX + 4;
     constexpr int WX = BX + 2, WY = BY + 2, NW = WX * WY * (BZ + 2);
@@ -366,6 +373,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
         // one plane; par = tt & 1
         auto plane = [&](const int tt, const int par) __attribute__((always_inline)) {
             // ---- A: update of plane tt-1, plane tt-2 stored ----
+            if constexpr (kPrioA) __builtin_amdgcn_s_setprio(1);
             if (interior && tt > tlo) {
                 double part[5];
 #pragma unroll
@@ -419,6 +427,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
 #pragma unroll
                 for (int n = 0; n < 5; n++) sm.qy[n][iyh] = ql[1][n];
             const bool myref = anyref && refined(cx, cy, tt);
+            if constexpr (kPrioA) __builtin_amdgcn_s_setprio(0);
             __syncthreads();
             // ---- B: primitives of plane tt+1 to LDS ----
             put(qp, pc);
