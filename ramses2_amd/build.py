@@ -14,14 +14,13 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIBNAME = "libramses2_hip.so"
-# (source, flags of its own): rh_brick64.hip once per set of brick shapes; the
-# step kernels without NaN quieting (see rh_brick64.hip), the FP64 brick kernel
-# scheduled for instruction-level parallelism (see there)
+# (source, flags of its own): rh_brick64.hip once per set of brick shapes, the FP64
+# brick kernel scheduled for instruction-level parallelism (see there)
 MAX_ILP = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
-UNITS = [("rh_godunov.hip", ["-fno-honor-nans"])]
-UNITS += [("rh_brick64.hip", ["-fno-honor-nans", "-DRH_SET=%d" % i] + MAX_ILP) for i in range(6)]
-UNITS += [("rh_tube.hip", ["-fno-honor-nans"])]
-UNITS += [(f, []) for f in ("rh_passes.hip", "rh_abi.hip", "rh_ext.hip", "rh_serve.hip", "rh_amr.hip", "rh_flag.hip")]
+UNITS = [("rh_godunov.hip", [])]
+UNITS += [("rh_brick64.hip", ["-DRH_SET=%d" % i] + MAX_ILP) for i in range(6)]
+UNITS += [(f, []) for f in ("rh_tube.hip", "rh_passes.hip", "rh_abi.hip", "rh_ext.hip", "rh_serve.hip", "rh_amr.hip",
+                            "rh_flag.hip")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("RH_OFFLOAD_ARCH", "gfx950")
 

@@ -397,7 +397,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
             __builtin_amdgcn_sched_barrier(0);
             fetch(cx, cy, tt < thi ? tt + 2 : thi + 2, u_o, fl_o);
             // ---- T: slopes and predictor of plane tt ----
-            double dq[3][5];
+            double dq[3][5], hr = 0.0, hp = 0.0;
             auto slopes = [&](const int sl) __attribute__((always_inline)) {
 #pragma unroll
                 for (int n = 0; n < 5; n++) {
@@ -405,6 +405,8 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
                     dq[1][n] = slope64(sl, q0[n] - sm.sq[n][pc - PX], sm.sq[n][pc + PX] - q0[n]);
                     dq[2][n] = slope64(sl, dzm[n], qp[n] - q0[n]);
                 }
+                hr = vmax_abs(vmax_abs(dq[0][0], dq[1][0]), dq[2][0]);
+                hp = vmax_abs(vmax_abs(dq[0][4], dq[1][4]), dq[2][4]);
                 dq[0][1] = vel_bound64(dq[0][1], sm.sq[0][pc - 1], q0[1] - sm.sq[1][pc - 1], ir0, sm.sq[0][pc + 1],
                                        sm.sq[1][pc + 1] - q0[1]);
                 dq[1][2] = vel_bound64(dq[1][2], sm.sq[0][pc - PX], q0[2] - sm.sq[2][pc - PX], ir0,
@@ -419,7 +421,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
 #pragma unroll
                 for (int n = 0; n < 5; n++) dq[0][n] = dq[1][n] = dq[2][n] = 0.0;
             double qr[3][5], ql[3][5];
-            trace64(q0, dq, qr, ql, k, ir0);
+            trace64(q0, dq, qr, ql, k, ir0, hr, hp);
             if (has_qx)
 #pragma unroll
                 for (int n = 0; n < 5; n++) sm.qx[n][ixh] = ql[0][n];

@@ -1,11 +1,10 @@
 // FP64 brick kernels: the instances of brick64 and their launches.  Compiled
 // once per set of brick shapes (RH_SET), so that the sets build in parallel.
 //
-// This file is compiled with -fno-honor-nans: min and max are then single
-// instructions, where the IEEE mode otherwise quiets every operand that comes
-// from memory or from another block (two more instructions per Riemann solve
-// and floor, about 40 of 810 per plane; 256^3 kernel 794 -> 753 us).  No path
-// depends on a NaN: a state that holds one is lost either way.
+// Compiled with NaNs honoured: a level that has lost its state still has a dt (the
+// bound that the cells without a NaN give), and the solvers may form a NaN on the
+// side of a select that is not taken.  What that costs in quieted operands of
+// fmax and fmin is avoided by vmax and vmin of rh_physics64.h.
 //
 // The scheduler is told to look for instruction-level parallelism: the kernel
 // runs at two waves per SIMD whatever its registers (its LDS and 210-250 VGPRs),

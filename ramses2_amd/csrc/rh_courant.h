@@ -122,7 +122,7 @@ __device__ __forceinline__ double courant_cell(const double u[5], const CourantK
                                                double &ekin, double &eint)
 {
 #pragma clang fp contract(off)
-    const double r = u[0] > c.smallr ? u[0] : c.smallr;
+    const double r = tmax(u[0], c.smallr);
     const double ir = rcp_nr(r), hr = 0.5 * r;
     const double v[3] = {u[1] * ir, u[2] * ir, u[3] * ir};
     double e = u[4];
@@ -132,10 +132,10 @@ __device__ __forceinline__ double courant_cell(const double u[5], const CourantK
     ekin = __builtin_fma(u[4], vol, ekin);
     eint = __builtin_fma(e, vol, eint);
     const double pe = (c.gamma - 1.0) * e, pf = r * c.smallp;
-    const double a2 = c.gamma * (pe > pf ? pe : pf) * ir;
+    const double a2 = c.gamma * tmax(pe, pf) * ir;
     // a2 >= gamma smallp = smallc^2: the square root of the Riemann solvers
     // (floored where smallc^2 < 2^-900)
-    const double cf = sqrt_pos(a2 > 0x1p-900 ? a2 : 0x1p-900);
+    const double cf = sqrt_pos(tmax(a2, 0x1p-900));
     double ctot = 0.0;
 #pragma unroll
     for (int d = 0; d < ND; d++) ctot = ctot + __builtin_fabs(v[d]) + cf;

@@ -24,10 +24,11 @@
 // where the FP64 ones moved on.
 // No MFMA: the work is divides, square roots and compares, not a contraction.
 //
-// Compiled with -fno-honor-nans as rh_brick64.hip is, and for the same reason:
-// 256^3 in mixed precision 549 -> 537 us, the bits of its results unchanged.
-// The separate passes, some of which a caller may use to look for a NaN, are in
-// rh_passes.hip, without that flag.
+// NaNs are honoured here: the mixed solver can lose a state (two floored cells
+// that move apart leave its denominator 0 in FP32), and a cell that is NaN must
+// drop out of the dt as it does in the reference, whose compares it fails.
+// (With -fno-honor-nans the 256^3 kernel took 535 instead of 546 us, and a level
+// whose cells were all lost returned courant_factor times its dt.)
 #include <type_traits>
 
 #include "rh_courant.h"
