@@ -5,13 +5,13 @@
 // One workgroup per oct brick, one thread per column of the brick's cells plus
 // one halo cell, marching along z.  Per plane tt there are two phases, each
 // ended by a barrier:
-//   A: the update of plane tt-1 from the face fluxes (the column's own low faces
+//   A: the update of plane tt-1 from the x and y fluxes (the column's own low faces
 //      in registers, its high faces in LDS), tt-2 final and stored; the own cell
 //      of plane tt+1 converted to primitives, the loads of plane tt+2 issued;
 //      slopes and Hancock predictor of plane tt, its left x and y states to LDS;
 //   B: primitives of plane tt+1 to LDS (every slope of plane tt has read the
 //      plane by now, so one plane is kept), and the Riemann problems of plane tt,
-//      the x and y fluxes to LDS.
+//      the x and y fluxes to LDS, the z fluxes into the update of plane tt-1.
 // The states and the fluxes have buffers of their own: two barriers per plane
 // instead of four when the fluxes overwrite the states, and the update's LDS
 // latency overlaps the conversion and the slopes.
@@ -269,22 +269,22 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
         __syncthreads();
 
         double qmz[5] = {0, 0, 0, 0, 0};   // left state of the low z face of plane tt
-        double fz[5] = {0, 0, 0, 0, 0};    // flux of the low z face of plane tt-1
+        double fz[5] = {0, 0, 0, 0, 0};    // flux of the low z face of plane tt-1, after its solve that of plane tt
         double fxo[5] = {0, 0, 0, 0, 0};   // fluxes of the low x and y faces of plane tt-1
         double fyo[5] = {0, 0, 0, 0, 0};
-        double pp[5] = {0, 0, 0, 0, 0};    // plane tt-2 but for its high z face
+        // plane tt-1 without its z faces, after the solve of its high one its new
+        // state.  The two z fluxes are subtracted before they are added, as those of
+        // x and y: equal fluxes (a planar flow's pressure) then cancel exactly.
+        double pp[5] = {0, 0, 0, 0, 0};
         double ub[5] = {0, 0, 0, 0, 0};    // the update's base of plane tt-1 (GEN)
         bool ref1 = false, ref2 = false;   // refined flags of planes tt-1 and tt-2
 
-        // plane tf of the column is final: un = pp - (dt/dx) fz
+        // plane tf of the column is final: its new state pp to unew
         auto finish = [&](int tf, const bool upper) __attribute__((always_inline)) {
             const int v = sm.swin[((tf + 2) >> 1) * (WX * WY) + wcol];
             const bool own = v >= a.head && v < a.head + a.noct && ox0 + (cx >> 1) < boxmax[0] &&
                              oy0 + (cy >> 1) < boxmax[1] && oz0 + (tf >> 1) < boxmax[2];
             if (!own) return;
-            double un[5];
-#pragma unroll
-            for (int n = 0; n < 5; n++) un[n] = tfma(-dtdx, fz[n], pp[n]);
             // the two planes of an oct fill each 64-byte line of unew: the
             // lower plane's values wait in LDS and both are stored together
             if (upper) {
@@ -292,13 +292,13 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
 #pragma unroll
                 for (int n = 0; n < 5; n++) {
                     po[8 * n] = sm.sun[n][icol];
-                    po[8 * n + 4] = un[n];
+                    po[8 * n + 4] = pp[n];
                 }
             } else {
 #pragma unroll
-                for (int n = 0; n < 5; n++) sm.sun[n][icol] = un[n];
+                for (int n = 0; n < 5; n++) sm.sun[n][icol] = pp[n];
             }
-            if (courant && !ref2) c_sig = tmax(c_sig, courant_cell<3>(un, ck, ck.vol, c_mass, c_ekin, c_eint));
+            if (courant && !ref2) c_sig = tmax(c_sig, courant_cell<3>(pp, ck, ck.vol, c_mass, c_ekin, c_eint));
         };
 
         auto wi = [&](int x, int y, int z) __attribute__((always_inline)) {
@@ -383,7 +383,7 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
                 }
                 if (tt - 2 >= tlo) finish(tt - 2, par != 0);
 #pragma unroll
-                for (int n = 0; n < 5; n++) pp[n] = tfma(dtdx, fz[n], part[n]);
+                for (int n = 0; n < 5; n++) pp[n] = part[n];
             }
             // ---- the own cell of plane tt+1 ----
             double qp[5];
@@ -491,9 +491,15 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
                 }
             }
             if (ROLE != 2 && interior && tt >= tlo) {
-                face64<RS>(2, qmz, qr[2], fz, k);
-                if (anyref) refzero(myref || ref1, fz);
-                if (reflux && par == 0) reflux_z(tt, fz);
+                double f[5];
+                face64<RS>(2, qmz, qr[2], f, k);
+                if (anyref) refzero(myref || ref1, f);
+                if (reflux && par == 0) reflux_z(tt, f);
+#pragma unroll
+                for (int n = 0; n < 5; n++) {
+                    pp[n] = tfma(dtdx, fz[n] - f[n], pp[n]);
+                    fz[n] = f[n];
+                }
             }
             if constexpr (GEN) {
                 // the base of this plane's update (unew for the drop-in call,
