@@ -97,8 +97,9 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
     const int tlo = 2 * zlo, thi = 2 * zhi + 1;
 
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
-    const HydroK<double> k = make_k<double>(dt, a.dx, a.gamma, a.smallr, a.smallc2, a.courant_factor, a.smax_cap,
-                                            a.use_smax, a.slope, a.riemann);
+    HydroK<double> k = make_k<double>(dt, a.dx, a.gamma, a.smallr, a.smallc2, a.courant_factor, a.smax_cap,
+                                      a.use_smax, a.slope, a.riemann);
+    if constexpr (RS == 3) k.smallp_riem = hllc_floor(k);
     const double gm1 = a.gamma - 1.0, smalle = a.smallc2 / a.gamma / gm1;
     double gvec[3] = {0.0, 0.0, 0.0}, gdt[3] = {0.0, 0.0, 0.0};
     if constexpr (GEN)

@@ -186,9 +186,10 @@ __device__ __forceinline__ void trace64(const double q[5], const double dqh[3][5
 // riemann_hllc, hydro/godunov_utils.f90:638-857 (mass, momenta, energy fluxes).
 // Only the star state and the energy of the side that is sampled are formed;
 // the sampled values are those of the reference, which forms both.  The states
-// come from trace64, whose densities are at least smallr, and with the
-// pressure floor no sound speed is below smallc, so those two floors of the
-// reference's are not repeated.
+// come from trace64, whose densities are at least smallr, and with the pressure
+// floor (hllc_floor) no sound speed is below smallc, so those two floors of the
+// reference's are not repeated.  Selecting the side's state costs the 256^3 kernel
+// 1% against forming it by the star formulas (647 -> 656 us).
 __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
 {
 #pragma clang fp contract(off)
@@ -206,19 +207,24 @@ __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], d
     T SR = vmax(ul, ur) + cmax;
     T dl = ul - SL, dr = SR - ur;
     T rcl = rl * dl, rcr = rr * dr;
-    T den = tfma(rr, dr, rcl);  // positive: ustar = num/den has the sign of num
+    T den = tfma(rr, dr, rcl);
     T num = (Pl - Pr) + tfma(rcr, ur, rcl * ul);
     // The reference samples, in this order: SL > 0 -> left state; ustar > 0
     // -> left star state; SR > 0 -> right star state; else right state.  The
     // side whose values are used is left exactly when SL > 0 or ustar > 0,
     // and the star state is taken when SL <= 0 and (ustar > 0 or SR > 0); in
     // both star cases the side is the reference's ustar > 0.  So one select
-    // of the side's values gives the reference's result (its chain costs three
-    // selects per value), and the total energy is formed for that side only.
-    // Outside the star states the contact's velocity and pressure are the
-    // side's own, with which the star state's formulas return the side's state
-    // (S - ustar = S - us): two selects instead of one for each of four values.
-    const bool sl_pos = SL > T(0), us_pos = num > T(0);
+    // of the side's values and one of four values (state or star) give the
+    // reference's result (its chain costs three selects per value), and the
+    // total energy is formed for that side only.
+    //
+    // The side's state has to be selected: the star state's formulas return it
+    // too when given the side's own velocity and pressure, but only to a rounding of
+    // S - us, which loses a factor |u|/c, and all of it where the sound speed is
+    // below half an ulp of the velocity.  There den and num can be 0 and the star
+    // state NaN, which the selects discard.  ustar = num/den has the sign of num
+    // where den > 0, and is no positive number where den = 0.
+    const bool sl_pos = SL > T(0), us_pos = num > T(0) && den > T(0);
     const bool left = sl_pos || us_pos;
     const bool star = !sl_pos && (us_pos || SR > T(0));
     T S = left ? SL : SR;
@@ -228,19 +234,26 @@ __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], d
     T ds = S - us;
     // 1/den and 1/(S - ustar) = den/(S den - num) from one reciprocal: the
     // hardware one takes four issue slots, and the two would depend on each other
-    T nu = star ? num : us * den;
-    T t = tfma(S, den, -nu);
+    T t = tfma(S, den, -num);
     T ri = rcp_h(den * t);
     T inv_den = ri * t, inv_sd = (ri * den) * den;
-    T uo = nu * inv_den;
-    T Po = star ? tfma(rcl * rcr, ul - ur, tfma(rcr, Pl, rcl * Pr)) * inv_den : Ps;
-    T ro = rs * ds * inv_sd;
-    T eo = tfma(Po, uo, tfma(ds, es, -(Ps * us))) * inv_sd;
+    T un = num * inv_den;
+    T Pn = tfma(rcl * rcr, ul - ur, tfma(rcr, Pl, rcl * Pr)) * inv_den;
+    T uo = star ? un : us, Po = star ? Pn : Ps;
+    T ro = star ? rs * ds * inv_sd : rs;
+    T eo = star ? tfma(Pn, un, tfma(ds, es, -(Ps * us))) * inv_sd : es;
     f[0] = ro * uo;
     f[1] = tfma(f[0], uo, Po);
     f[2] = f[0] * vo;
     f[3] = f[0] * wo;
     f[4] = (eo + Po) * uo;
+}
+// The pressure floor of hllc64: smallc^2/gamma, and where smallc is (nearly) 0 that
+// of a sound speed of 2^-300, so that for gas at rest without pressure den and the
+// product under the reciprocal, of the order of rho^2 c^3, stay in range.
+__device__ __forceinline__ double hllc_floor(const HydroK<double> &k)
+{
+    return tmax(k.smallc2, 0x1p-600) / k.gamma;
 }
 
 // Conservative state and physical flux of one side (side_state).

@@ -89,6 +89,7 @@ template <int RS, int K> __global__ void __launch_bounds__(kTubeThreads + 64) k_
     const CourantK ck = make_courant_k(a.dx, 1, a.gamma, a.smallr, a.smallc2, a.courant_factor, gv);
     HydroK<double> k = make_k<double>(1.0, a.dx, a.gamma, a.smallr, a.smallc2, a.courant_factor, a.smax_cap, a.use_smax,
                                       a.slope < 2 ? a.slope : 2, a.riemann);
+    if constexpr (RS == 3) k.smallp_riem = hllc_floor(k);
     // without gravity dt = dtc / (largest signal speed) (signal_dt)
     const double dtc = signal_dt(1.0, ck), dtmax = a.dx / ck.smallc;
     const bool courant = t.dt_fixed <= 0.0;
