@@ -503,7 +503,7 @@ int rh_init(void)
     RH_HIP_CHECK(dmalloc((void **)&s.red_out, 8 * sizeof(double)));
     if (!g_hred) RH_HIP_CHECK(hipHostMalloc(&g_hred, 8 * sizeof(double), hipHostMallocDefault));
     s.h_red = g_hred;
-    s.red_cap = 4096;
+    s.red_cap = kMinPartials;
     RH_HIP_CHECK(dmalloc((void **)&s.red_part, (size_t)s.red_cap * 4 * sizeof(double)));
     RH_HIP_CHECK(dmalloc((void **)&s.dt_dev, 2 * sizeof(double)));
     RH_HIP_CHECK(dmalloc((void **)&s.d_counter, 4 * sizeof(int)));

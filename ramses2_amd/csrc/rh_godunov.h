@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "rh_physics.h"
+#include "rh_split.h"
 
 namespace rh {
 
@@ -97,14 +98,14 @@ struct God1Args {
 };
 
 // Parts along z for a work-list launch of nbricks bricks of one shape in
-// precision prec (see zsplit_for in rh_launch.h).
+// precision prec (see rh_split.h).
 int worklist_zsplit(long nbricks, int bx, int by, int bz, int prec);
 
 // Launch the 3D brick kernel for brick shape (bx,by,bz) in precision prec
 // (0 = FP64, 1 = FP32 reconstruction/fluxes with FP64 accumulation).
 // *nparts (if non-null) receives the number of Courant partials the launch
 // writes (bricks plus split halves, or the bricks' parts), at most
-// max(2 nbricks + 8, 4096).
+// max(2 nbricks + 8, kMinPartials).
 hipError_t launch_godunov3d(const GodArgs &a, int bx, int by, int bz, int prec, hipStream_t s,
                             hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, int *nparts = nullptr);
 hipError_t launch_godunov1d(const God1Args &a, int prec, hipStream_t s);

@@ -270,7 +270,7 @@ int rh_estimate_uniform_bytes(int n_octs_per_dim, int ncachemax, int hash_size, 
     b += cap * (8 + 4);                                       // hash keys, values
     b += (int64_t)std::max(ncachemax, 1) * (2 + 14 + 21 + 1 + 3) * 4;  // ghost-oct tables
     b += 8 * 8 + 2 * 8 + 4 * 4 + 2 * 8;                       // reduction / dt / counters
-    b += std::max<int64_t>(4096, nb) * 4 * 8;                 // Courant partials
+    b += std::max<int64_t>(kMinPartials, nb) * 4 * 8;         // Courant partials
     b += noct * 27 * 4 + noct * 2 * 4;                        // neighbour and father tables
     b += nb * ((int64_t)(bx + 2) * (by + 2) * (bz + 2) + 4) * 4;  // brick windows, origins, z ranges
     *bytes = b;
