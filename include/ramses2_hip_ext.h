@@ -180,14 +180,13 @@ int rh_job_prepare(int head_idx, int num_octs, int ilevel, double dx, double gam
  * launches: per step one work-list Godunov kernel over the bricks of
  * all the jobs (each job's Courant condition of the new state reduced in the
  * kernel's epilogue) and one per-job final reduction (dt of the job's next
- * step, its time).  Jobs advance independently: a job's state, dt and time do
- * not depend on the other jobs of the batch (its conservation sums do in their
- * last bits, whose order follows how the batch is cut into workgroups).
- * Asynchronous. */
+ * step, its time).  Jobs advance independently: a job's result does not depend
+ * on the other jobs of the batch.  Asynchronous. */
 int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps);
 
 /* Synchronous read of a job's {t, dt of the next step, mass, ekin, eint, emag,
- * dt} (the last four from the last Courant reduction). */
+ * dt}: the sums of its current state, by a pass over its octs where batched steps
+ * have advanced it, and the dt of the last Courant reduction. */
 int rh_job_status(int id, double out[7]);
 
 /* A fence on the library stream, for a request loop that keeps one batched

@@ -500,7 +500,7 @@ int rh_init(void)
     RH_HIP_CHECK(hipGetDevice(&s.device));
     if (!g_stream) RH_HIP_CHECK(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking));
     s.stream = g_stream;
-    RH_HIP_CHECK(dmalloc((void **)&s.red_out, 8 * sizeof(double)));
+    RH_HIP_CHECK(dmalloc((void **)&s.red_out, 16 * sizeof(double)));
     if (!g_hred) RH_HIP_CHECK(hipHostMalloc(&g_hred, 8 * sizeof(double), hipHostMallocDefault));
     s.h_red = g_hred;
     s.red_cap = kMinPartials;
@@ -582,6 +582,7 @@ int rh_alloc_amr(int ngridmax, int ncachemax, int nvar, int twotondim, int hash_
     s.ndim = twotondim == 8 ? 3 : 1;
     s.ttd = twotondim;
     s.nvar = nvar;
+    s.job_stepped = false;
     s.ngridmax = ngridmax;
     s.ncachemax = ncachemax;
     s.ngridtot = ngridmax + ncachemax;

@@ -150,7 +150,7 @@ struct State {
     // reduction scratch
     double *red_part = nullptr;
     int red_cap = 0;
-    double *red_out = nullptr;     // device, 8 doubles
+    double *red_out = nullptr;     // device: 8 doubles of the last reduction, 8 of a job's status
     double *h_red = nullptr;       // pinned host, 8 doubles
     std::string last_error;
     // device allocations of this context (bytes by pointer) and their total
@@ -158,6 +158,7 @@ struct State {
     int64_t dev_bytes = 0;
     // a job prepared for batched stepping (one 3D level, dt on the device)
     bool job_ready = false;
+    bool job_stepped = false;      // by rh_batch_step since it was prepared
     GodArgs job;
     int job_bx = 0, job_by = 0, job_bz = 0;
     double job_dtmax = 0.0;
