@@ -80,11 +80,11 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
     constexpr bool GEN = KIND != kBrickUniform;
     // Phase A, whose LDS reads wait most, runs at a raised wave priority, so that
     // the CU's other workgroup fills its gaps with solves instead of delaying
-    // it.  Workgroups of four waves and more, of which two share a CU: 8x6x16
-    // at 256^3 646 -> 629 us, 8x6x8 at 128^3 104 -> 100, 7x7x8 at 128^3 135 ->
-    // 129.  With four workgroups of two waves the raised ones starve the others:
-    // 4x4x8 at 128^3 125 -> 136 us.
-    constexpr bool kPrioA = (2 * BX + 2) * (2 * BY + 2) > 192;
+    // it, where two workgroups (of four waves) share a CU: 8x6x16 at 256^3 646 -> 629
+    // us, 8x6x8 at 128^3 104 -> 100, 7x7x8 at 128^3 135 -> 129.  With four workgroups
+    // of two waves the raised ones starve the others (4x4x8 at 128^3 125 -> 136 us),
+    // and where one fills the CU it changes nothing (15x7x8 at 256^3 833, 837).
+    constexpr bool kPrioA = Brick64Lds<BX, BY, BZ, GEN>::WGS == 2;
     constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY, NI = 4 * BX * BY;
     constexpr int PX = 2 * BX + 4;
     constexpr int WX = BX + 2, WY = BY + 2, NW = WX * WY * (BZ + 2);
