@@ -29,6 +29,13 @@ __device__ __forceinline__ double vmax(double a, double b)
     asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+// the same with a value uniform in the wave
+__device__ __forceinline__ double vmax_u(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "s"(b));
+    return r;
+}
 __device__ __forceinline__ double vmin(double a, double b)
 {
     double r;
@@ -188,7 +195,10 @@ __device__ __forceinline__ void trace64(const double q[5], const double dqh[3][5
 // the sampled values are those of the reference, which forms both.  The states
 // come from trace64, whose densities are at least smallr, and with the pressure
 // floor (hllc_floor) no sound speed is below smallc, so those two floors of the
-// reference's are not repeated.  Selecting the side's state costs the 256^3 kernel
+// reference's are not repeated but for the right density, which turns a lost state
+// there into one whose sound speed is no NaN (sqrt_quot_max takes the right one
+// where the comparison is false): the upwind side of a supersonic face is then
+// selected whatever the other holds.  Selecting the side's state costs the 256^3 kernel
 // 1% against forming it by the star formulas (647 -> 656 us).
 __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
 {
@@ -198,7 +208,7 @@ __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], d
     T rl = ql[0];
     T ul = ql[1], vl = ql[2], wl = ql[3];
     T Pl = vmax(ql[4], rl * k.smallp_riem);
-    T rr = qr[0];
+    T rr = vmax_u(qr[0], k.smallr);
     T ur = qr[1], vr = qr[2], wr = qr[3];
     T Pr = vmax(qr[4], rr * k.smallp_riem);
     // max(sqrt(a), sqrt(b)) = sqrt(max(a, b)): one root for the two sound speeds

@@ -11,6 +11,7 @@ from ramses2_amd import HydroParams, UniformLevel, UniformMesh
 from ramses2_amd._lib import call
 from ramses2_amd.autotune import DEFAULT_SHAPE
 from ramses2_amd.hydro import AmrHierarchy, HipHydro
+from ramses2_amd.mesh import prim_to_cons
 from tests.amr_cases import two_level_mesh
 
 pytestmark = pytest.mark.gpu
@@ -73,3 +74,37 @@ def test_lost_job(brick, precision):
         call("rh_set_brick_shape", *DEFAULT_SHAPE)
     bound = (1.0 / 32) / np.sqrt(1e-10 ** 2)
     assert st["dt_next"] == bound and st["t"] == 3 * bound
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("slope", [1, 2])
+@pytest.mark.parametrize("ndim,axis,brick", [(1, 0, (8, 6, 8)), (3, 0, (8, 6, 8)), (3, 1, (7, 7, 8)), (3, 2, (4, 4, 4))])
+def test_lost_cell_in_a_supersonic_stream(ndim, axis, brick, slope, sign, precision):
+    """HLLC takes the upwind state of a supersonic face, whatever lies downstream: a
+    lost cell loses no cell upstream of it, and those further off than its
+    neighbours' slopes reach keep their bits."""
+    n, at, nsteps = 32, 16, 4
+    rng = np.random.default_rng(8)
+    full = (n,) * ndim
+    vel = [np.zeros(full)] * 3
+    vel[axis] = sign * (8.0 + rng.random(full))
+    cells = prim_to_cons(0.5 + rng.random(full), vel, 0.5 + rng.random(full), 1.4)
+    ax = ndim - axis  # of a (5, ...) array
+    out = []
+    for lost in (True, False):
+        c = cells.copy()
+        if lost:
+            c[(slice(None),) + (at,) * ndim] = np.nan
+        HipHydro.set_brick_shape(*brick)
+        try:
+            lev = UniformLevel(UniformMesh.for_cells(ndim, n), c, _params(slope, "hllc"))
+        finally:
+            HipHydro.set_brick_shape(*DEFAULT_SHAPE)
+        lev.run_device(nsteps, dt_fixed=0.5 / (n * 12.0), precision=precision)
+        out.append(np.moveaxis(lev.cells(), ax, 1))
+    up = [at - sign * k for k in range(1, 9)]
+    assert np.isnan(out[0][:, at]).any()
+    assert np.all(np.isfinite(out[0][:, up]))
+    far = up[nsteps + 1:]
+    assert np.array_equal(out[0][:, far], out[1][:, far])
