@@ -185,8 +185,7 @@ int rh_job_prepare(int head_idx, int num_octs, int ilevel, double dx, double gam
 int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps);
 
 /* Synchronous read of a job's {t, dt of the next step, mass, ekin, eint, emag,
- * dt}: the sums of its current state, by a pass over its octs where batched steps
- * have advanced it, and the dt of the last Courant reduction. */
+ * dt} (the last four from the last Courant reduction). */
 int rh_job_status(int id, double out[7]);
 
 /* A fence on the library stream, for a request loop that keeps one batched

@@ -582,7 +582,7 @@ int rh_alloc_amr(int ngridmax, int ncachemax, int nvar, int twotondim, int hash_
     s.ndim = twotondim == 8 ? 3 : 1;
     s.ttd = twotondim;
     s.nvar = nvar;
-    s.job_stepped = false;
+    s.job_cut = false;
     s.ngridmax = ngridmax;
     s.ncachemax = ncachemax;
     s.ngridtot = ngridmax + ncachemax;

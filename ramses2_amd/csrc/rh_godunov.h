@@ -188,6 +188,11 @@ hipError_t launch_reflux_fold(double *unew, double *racc, const int32_t *ghost_p
 // Slots per ghost oct of the deterministic reflux: 6 faces x 4 cells
 constexpr int kRefluxSlotsPerGhost = 24;
 hipError_t launch_courant_reduce_batch(const CourantJob *jobs, int njobs, hipStream_t s);
+// Conservation sums of the bricks of a 3D level of shape (bx,by,bz) from `state`, with
+// the bits that launch_godunov3d_wl's partials give where no brick is cut, into
+// out[0..3]; nbricks partials of 4 doubles.
+hipError_t launch_brick_sums(const GodArgs &a, const double *state, int bx, int by, int bz, int prec, double *partials,
+                             double *out, hipStream_t s);
 hipError_t launch_courant_reduce(const double *partials, int nparts, double dtmax, double *out, double *dt_inout,
                                  double *t_acc, hipStream_t s);
 

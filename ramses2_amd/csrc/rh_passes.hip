@@ -320,6 +320,66 @@ __global__ void __launch_bounds__(256) k_courant_final(const double *__restrict_
     courant_final_block(part, nblocks, dtmax, out, dt_out, t_acc, acc_old);
 }
 
+// The conservation sums of whole bricks, added in the order in which a work-list
+// launch of uncut bricks adds them: FP64 per column of the brick, its cells along z
+// (hw: the kernel's interior columns come first, see brick64_hw), mixed per cell
+// index.  state: the state that the step wrote.
+__global__ void __launch_bounds__(512) k_brick_sums(const GodArgs a, const double *__restrict__ state, int bx, int by,
+                                                    int bz, int hw, int mixed, double *__restrict__ part)
+{
+    __shared__ double red[8][3];
+    const int wx = bx + 2, wy = by + 2, bid = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+    const int32_t *win = a.win + (size_t)bid * wx * wy * (bz + 2);
+    const int zr = a.zr ? a.zr[bid] : (bz - 1) << 16;
+    const double gv[3] = {a.g[0], a.g[1], a.g[2]};
+    const CourantK ck = make_courant_k(a.dx, 3, a.gamma, a.smallr, a.smallc2, a.courant_factor, gv);
+    double mass = 0.0, ekin = 0.0, eint = 0.0, dt = 0.0;
+    // cell (x, y, z) of the brick
+    auto add = [&](int x, int y, int z) {
+        const int v = win[((z >> 1) + 1) * (wx * wy) + ((y >> 1) + 1) * wx + (x >> 1) + 1];
+        if (v < a.head || v >= a.head + a.noct || a.org[3 * bid] + (x >> 1) >= a.boxmax[0] ||
+            a.org[3 * bid + 1] + (y >> 1) >= a.boxmax[1] || a.org[3 * bid + 2] + (z >> 1) >= a.boxmax[2])
+            return;
+        const int ind = (x & 1) + 2 * (y & 1) + 4 * (z & 1);
+        if (a.refined[(size_t)(v - 1) * 8 + ind]) return;
+        const double *p = state + (size_t)(v - 1) * 40 + ind;
+        const double u[5] = {p[0], p[8], p[16], p[24], p[32]};
+        if (mixed)
+            courant_cell_mixed(u, ck, mass, ekin, eint, dt);
+        else
+            (void)courant_cell<3>(u, ck, ck.vol, mass, ekin, eint);
+    };
+    if (mixed) {
+        for (int i = tid; i < bx * by * bz * 8; i += nt) {
+            const int oc = i >> 3;
+            const int oz = oc / (bx * by);
+            if (oz >= (zr & 0xffff) && oz <= zr >> 16)
+                add(2 * (oc % bx) + (i & 1), 2 * ((oc / bx) % by) + ((i >> 1) & 1), 2 * oz + ((i >> 2) & 1));
+        }
+    } else {
+        const int x = hw ? tid % (2 * bx) : tid % (2 * bx + 2) - 1, y = hw ? tid / (2 * bx) : tid / (2 * bx + 2) - 1;
+        if (x >= 0 && x < 2 * bx && y >= 0 && y < 2 * by)
+            for (int z = 2 * (zr & 0xffff); z <= 2 * (zr >> 16) + 1; z++) add(x, y, z);
+    }
+    const int nv = nt - (tid & ~63) < 64 ? nt - (tid & ~63) : 64;
+    mass = wave_sum_n(mass, nv);
+    ekin = wave_sum_n(ekin, nv);
+    eint = wave_sum_n(eint, nv);
+    if ((tid & 63) == 0) {
+        red[tid >> 6][0] = mass;
+        red[tid >> 6][1] = ekin;
+        red[tid >> 6][2] = eint;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double s[3] = {0, 0, 0};
+        for (int i = 0; i < (nt + 63) / 64; i++)
+            for (int k = 0; k < 3; k++) s[k] += red[i][k];
+        for (int k = 0; k < 3; k++) part[4 * bid + k] = s[k];
+        part[4 * bid + 3] = a.dx / ck.smallc;
+    }
+}
+
 // One block per job of a batch: each job's own partials, in its fixed order.
 __global__ void __launch_bounds__(256) k_courant_final_batch(const CourantJob *__restrict__ jobs)
 {
@@ -893,6 +953,20 @@ hipError_t launch_courant_reduce(const double *partials, int nparts, double dtma
                                  double *t_acc, hipStream_t s)
 {
     hipLaunchKernelGGL(k_courant_final, dim3(1), dim3(256), 0, s, partials, nparts, dtmax, out, dt_inout, t_acc, 1);
+    return hipGetLastError();
+}
+
+hipError_t launch_brick_sums(const GodArgs &a, const double *state, int bx, int by, int bz, int prec, double *partials,
+                             double *out, hipStream_t s)
+{
+    const int nt = (2 * bx + 2) * (2 * by + 2), ni = 4 * bx * by;
+    const int hw = prec == 0 && a.slope != 3 && ni % 64 == 0 && nt - ni <= 64;
+    if (a.nbricks <= 0 || nt > 512) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_brick_sums, dim3(a.nbricks), dim3(nt), 0, s, a, state, bx, by, bz, hw, prec, partials);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_courant_final, dim3(1), dim3(256), 0, s, partials, a.nbricks, a.dx / __builtin_sqrt(a.smallc2),
+                       out, nullptr, nullptr, 0);
     return hipGetLastError();
 }
 

@@ -115,24 +115,19 @@ constexpr int kMaxFences = 64;
 std::vector<Fence> g_fences;
 
 // The status of a context, enqueued on the stream into v: {t, dt of the next
-// step, mass, ekin, eint, emag, dt}.  The sums of a stepped job come from a Courant
-// pass over its octs, made here: those of the batched step are added up brick part
-// by brick part, and how many parts there are depends on the other jobs of the
-// batch (worklist_zsplit).  About 20 us a status for jobs of 32^3 to 128^3 cells.
+// step, mass, ekin, eint, emag, dt}.  The last batch of a job may have cut its
+// bricks into parts, as many as the other jobs left room for (worklist_zsplit): its
+// sums are then added up here, whole brick by whole brick.
 int enqueue_status(const State &s, double *v, hipStream_t stream)
 {
-    const double *sums = s.red_out;
-    if (s.job_stepped) {
-        const GodArgs &a = s.job;
-        sums = s.red_out + 8;
-        RH_HIP_CHECK(launch_courant(s.uold, s.refined, a.head, a.noct, 3, a.dx, a.gamma, a.smallr,
-                                    __builtin_sqrt(a.smallc2), a.courant_factor, a.g, s.red_part, kMinPartials,
-                                    s.red_out + 8, nullptr, stream));
-    }
     RH_HIP_CHECK(hipMemcpyAsync(v, s.t_dev, sizeof(double), hipMemcpyDeviceToHost, stream));
     RH_HIP_CHECK(hipMemcpyAsync(v + 1, s.dt_dev, sizeof(double), hipMemcpyDeviceToHost, stream));
-    RH_HIP_CHECK(hipMemcpyAsync(v + 2, sums, 4 * sizeof(double), hipMemcpyDeviceToHost, stream));
-    RH_HIP_CHECK(hipMemcpyAsync(v + 6, s.red_out + 4, sizeof(double), hipMemcpyDeviceToHost, stream));
+    RH_HIP_CHECK(hipMemcpyAsync(v + 2, s.red_out, 5 * sizeof(double), hipMemcpyDeviceToHost, stream));
+    if (s.job_cut) {
+        RH_HIP_CHECK(launch_brick_sums(s.job, s.uold, s.job_bx, s.job_by, s.job_bz, s.job_prec, s.red_part,
+                                       s.red_out + 8, stream));
+        RH_HIP_CHECK(hipMemcpyAsync(v + 2, s.red_out + 8, 4 * sizeof(double), hipMemcpyDeviceToHost, stream));
+    }
     return 0;
 }
 
@@ -343,7 +338,7 @@ int rh_job_prepare(int head_idx, int num_octs, int ilevel, double dx, double gam
                                 courant_factor, g ? g : gz, s.red_part, s.red_cap, s.red_out, s.dt_dev, s.stream,
                                 nullptr));
     s.job_ready = true;
-    s.job_stepped = false;
+    s.job_cut = false;
     return 0;
 }
 
@@ -414,7 +409,8 @@ int rh_batch_step(const int32_t *ids, int njobs, int precision, int nsteps)
     }
     for (State *s : js) {
         if (nsteps & 1) std::swap(s->uold, s->unew);
-        s->job_stepped = true;
+        s->job_cut = nz > 1;
+        s->job_prec = precision;
     }
     return 0;
 }

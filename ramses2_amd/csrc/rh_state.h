@@ -158,7 +158,8 @@ struct State {
     int64_t dev_bytes = 0;
     // a job prepared for batched stepping (one 3D level, dt on the device)
     bool job_ready = false;
-    bool job_stepped = false;      // by rh_batch_step since it was prepared
+    bool job_cut = false;          // its last batch cut its bricks into parts
+    int job_prec = 0;              // precision of that batch
     GodArgs job;
     int job_bx = 0, job_by = 0, job_bz = 0;
     double job_dtmax = 0.0;
