@@ -660,6 +660,7 @@ int rh_set_grid_device(const double *uold, const double *unew, const void *bold,
 {
     if (int r = ensure_mesh()) return r;
     State &s = st();
+    s.job_cut = false;
     if (bold) return fail(RH_ERR_ARG, "bold must be NULL (no MHD)");
     if (ngridmax < 0 || ngridmax > s.ngridtot || nvar != s.nvar || twotondim != s.ttd)
         return fail(RH_ERR_ARG, "rh_set_grid_device: sizes differ from rh_alloc_amr");
@@ -757,6 +758,7 @@ int rh_build_nbor(int head_idx, int num_octs, int hash_size, int ckey_max_l, int
     (void)key_off_l;
     if (!box_min || !box_max || !periodic) return fail(RH_ERR_ARG, "null box arrays");
     drop_level_graph(s);  // its tables are rebuilt
+    s.job_cut = false;
     if (s.ndim == 3 && !periodic[0] + !periodic[1] + !periodic[2] > 1)
         // stencil octs beyond an edge or a corner of the box: the reference
         // builds them from whichever neighbouring boundary oct its cache holds
@@ -1004,6 +1006,7 @@ int rh_set_uold(int head_idx, int num_octs)
 {
     if (int r = ensure_mesh()) return r;
     State &s = st();
+    s.job_cut = false;
     if (head_idx < 1 || num_octs < 0 || (int64_t)head_idx - 1 + num_octs > s.ngridtot)
         return fail(RH_ERR_ARG, "rh_set_uold: oct range out of bounds");
     const size_t per = (size_t)s.nvar * s.ttd;
@@ -1017,6 +1020,7 @@ int rh_cmpdt(int head_idx, int num_octs, double dx, double gamma, double smallr,
 {
     if (int r = ensure_mesh()) return r;
     State &s = st();
+    s.job_cut = false;
     if (head_idx < 1 || num_octs < 0 || (int64_t)head_idx - 1 + num_octs > s.ngridtot)
         return fail(RH_ERR_ARG, "rh_cmpdt: oct range out of bounds");
     if (!(dx > 0) || !(smallc2 > 0) || !(gamma > 1)) return fail(RH_ERR_ARG, "rh_cmpdt: bad physical parameters");
@@ -1068,6 +1072,7 @@ int rh_godunov(int head_idx, int num_subgrids, int ngridmax, int ilevel, int lev
 {
     if (int r = ensure_mesh()) return r;
     State &s = st();
+    s.job_cut = false;
     (void)ngridmax;
     (void)levelmax;
     if (num_subgrids == 0) return 0;

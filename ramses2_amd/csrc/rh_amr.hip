@@ -136,6 +136,7 @@ int rh_amr_prepare(int levelmin, int levelmax, const int32_t *head, const int32_
                    double smallr, double smallc2, double courant_factor, const double g[3], int slope, int riemann)
 {
     State &s = st();
+    s.job_cut = false;
     if (!s.inited || !s.uold) return efail(RH_ERR_STATE, "library not initialised / mesh not allocated");
     if (s.ndim != 3) return efail(RH_ERR_ARG, "batched AMR stepping is 3D");
     if (s.difmag > 0.0)

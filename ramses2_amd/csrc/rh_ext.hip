@@ -348,6 +348,7 @@ int rh_level_run(int head_idx, int num_octs, int ilevel, double dx, double gamma
                  int use_graph, double *dt_last, double *t_total, double sums[4], float *kernel_ms)
 {
     State &s = st();
+    s.job_cut = false;
     if (!s.inited || !s.uold) return efail(RH_ERR_STATE, "library not initialised / mesh not allocated");
     if (nsteps < 0) return efail(RH_ERR_ARG, "nsteps must be >= 0");
     if (!level_is_whole_mesh(head_idx, num_octs))

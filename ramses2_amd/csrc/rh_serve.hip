@@ -297,6 +297,7 @@ int rh_estimate_uniform_bytes(int n_octs_per_dim, int ncachemax, int hash_size, 
 int rh_init_ic(int head_idx, int num_octs, int ncell, int kind, const double params[5], double gamma)
 {
     State &s = st();
+    s.job_cut = false;
     if (!s.inited || !s.uold) return efail(RH_ERR_STATE, "library not initialised / mesh not allocated");
     if (s.ndim != 3) return efail(RH_ERR_ARG, "rh_init_ic builds 3D initial conditions");
     if (kind != 1 && kind != 2) return efail(RH_ERR_ARG, "kind must be 1 (blast) or 2 (Riemann)");

@@ -158,7 +158,8 @@ struct State {
     int64_t dev_bytes = 0;
     // a job prepared for batched stepping (one 3D level, dt on the device)
     bool job_ready = false;
-    bool job_cut = false;          // its last batch cut its bricks into parts
+    bool job_cut = false;          // its last batch cut its bricks into parts, and no other call has touched
+                                   // the state, its tables or red_out since
     int job_prec = 0;              // precision of that batch
     GodArgs job;
     int job_bx = 0, job_by = 0, job_bz = 0;

@@ -2,12 +2,14 @@
 for bit, however the batch is cut into workgroups: alone (bricks in parts along z),
 beside another small job, and beside one that fills the chip (whole bricks); by
 status and by fence, and against the host's sums of the state."""
+import ctypes
 import math
 
 import numpy as np
 import pytest
 
 from ramses2_amd import HydroParams
+from ramses2_amd._lib import call, ptr
 from ramses2_amd.serving import HipEngine, JobSpec
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +46,26 @@ def test_sums_do_not_depend_on_the_batch(kind, ic, brick, slope, riemann, precis
     mass, energy = (math.fsum(res[0][1][v].ravel()) * vol for v in (0, 4))
     # 39304 terms, added in 256 threads, their waves and blocks: far fewer roundings than 1e-13 allows
     assert abs(res[0][0]["mass"] - mass) <= 1e-13 * mass and abs(res[0][0]["ekin"] - energy) <= 1e-13 * energy
+
+
+def test_status_after_another_call_is_of_that_call():
+    """After a cut batch a status re-adds the job's sums only until another call
+    reduces or rebuilds: then it is what that call left, as before."""
+    eng = HipEngine(precision=0, brick=(8, 6, 8))
+    job = JobSpec(0, 0.0, 34, 1, (1.0, 1e-3, 400.0, 16.0, 0.0), 3)
+    h = eng.open(job)
+    try:
+        eng.step([h], 3)
+        mesh = eng._mesh_for(34)[0]
+        call("rh_ctx_select", h)
+        out = [ctypes.c_double() for _ in range(5)]
+        g = np.zeros(3)
+        half = mesh.noct // 2
+        call("rh_cmpdt", 1, half, mesh.dx, 1.4, 1e-10, 1e-20, 0.5, ptr(g), *[ctypes.byref(x) for x in out])
+        call("rh_ctx_select", 0)
+        st = eng.status(h)
+    finally:
+        call("rh_ctx_select", 0)
+        eng.close(h)
+        eng.close_all()
+    assert [st[k] for k in ("mass", "ekin", "eint")] == [x.value for x in out[:3]]
