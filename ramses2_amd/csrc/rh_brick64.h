@@ -23,12 +23,13 @@
 // wave, both loops pass the same barriers): the interior loop has no ring
 // loads, no divergent tests, and solves its three faces in straight line; the
 // halo loop solves one face per lane, converts the ring and updates nothing.
-// Measured against the one-body kernel this replaced (four barriers, every
-// thread testing its role, the expressions of rh_physics.h), with the Courant
-// reduction: 256^3 in 8x6x16 bricks 843 -> 629 us (26.7 G cell-updates/s, 2.1
-// TB/s of the 80 algorithmic bytes per cell; 680 with the column's own low faces
-// read back from LDS and two reciprocals per HLLC face), 128^3 in 8x6x8 bricks
-// 140 -> 100 us, 90^3 MinMod + LLF (a run-time solver choice before) 105 -> 64 us.
+// Measured in turn on one card against the one-body kernel this replaced (four
+// barriers, every thread testing its role, the expressions of rh_physics.h), with
+// the Courant reduction: 256^3 in 8x6x16 bricks 858 -> 668 us (25.1 G
+// cell-updates/s, 2.0 TB/s of the 80 algorithmic bytes per cell; reading the column's
+// own low faces back from LDS and two reciprocals per HLLC face cost another 3%),
+// 128^3 in 8x6x8 bricks 135 -> 99 us, 90^3 MinMod + LLF (a run-time solver choice
+// before) 107 -> 59 us.
 #pragma once
 #include <type_traits>
 
@@ -82,8 +83,9 @@ __device__ __forceinline__ void brick64(A &a, const int bid, const int zlo, cons
     // the CU's other workgroup fills its gaps with solves instead of delaying
     // it, where two workgroups (of four waves) share a CU: 8x6x16 at 256^3 646 -> 629
     // us, 8x6x8 at 128^3 104 -> 100, 7x7x8 at 128^3 135 -> 129.  With four workgroups
-    // of two waves the raised ones starve the others (4x4x8 at 128^3 125 -> 136 us),
-    // and where one fills the CU it changes nothing (15x7x8 at 256^3 833, 837).
+    // of two waves the raised ones starve the others (4x4x8 at 128^3 125 -> 136 us);
+    // where one fills the CU there is none to yield to (256^3 without and with it:
+    // 15x7x8 833 and 837 us, 15x7x16 788 and 782).
     constexpr bool kPrioA = Brick64Lds<BX, BY, BZ, GEN>::WGS == 2;
     constexpr int CX = 2 * BX + 2, CY = 2 * BY + 2, NT = CX * CY, NI = 4 * BX * BY;
     constexpr int PX = 2 * BX + 4;

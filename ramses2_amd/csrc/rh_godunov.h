@@ -145,10 +145,6 @@ hipError_t launch_brick64(const GodArgs &a, int bx, int by, int bz, int kind, hi
 hipError_t launch_brick64_wl(const WorkList &w, int nblocks, int bx, int by, int bz, int riemann, int kind,
                              hipStream_t s);
 
-// Courant reduction over cells of octs [head, head+noct): per-block partials,
-// then a fixed-order final pass -> out[0..4] = mass, ekin, eint, emag, dt.
-// Fixed-order reduction of fused-Courant partials: t_acc += the dt the step
-// used (*dt_inout on entry), then *dt_inout = min(dtmax, partial dts).
 // Per-job final Courant reduction of a batch (one block per job).
 struct CourantJob {
     const double *part;   // per-brick partials of the job
@@ -193,9 +189,13 @@ hipError_t launch_courant_reduce_batch(const CourantJob *jobs, int njobs, hipStr
 // out[0..3]; nbricks partials of 4 doubles.
 hipError_t launch_brick_sums(const GodArgs &a, const double *state, int bx, int by, int bz, int prec, double *partials,
                              double *out, hipStream_t s);
+// Fixed-order reduction of fused-Courant partials: t_acc += the dt the step
+// used (*dt_inout on entry), then *dt_inout = min(dtmax, partial dts).
 hipError_t launch_courant_reduce(const double *partials, int nparts, double dtmax, double *out, double *dt_inout,
                                  double *t_acc, hipStream_t s);
 
+// Courant reduction over cells of octs [head, head+noct): per-block partials,
+// then a fixed-order final pass -> out[0..4] = mass, ekin, eint, emag, dt.
 hipError_t launch_courant(const double *uold, const uint8_t *refined, int head, int noct, int ndim,
                           double dx, double gamma, double smallr, double smallc, double courant_factor,
                           const double g[3], double *partials, int max_blocks, double *out,

@@ -199,7 +199,7 @@ __device__ __forceinline__ void trace64(const double q[5], const double dqh[3][5
 // there into one whose sound speed is no NaN (sqrt_quot_max takes the right one
 // where the comparison is false): the upwind side of a supersonic face is then
 // selected whatever the other holds.  Selecting the side's state costs the 256^3 kernel
-// 1% against forming it by the star formulas (647 -> 656 us).
+// 1.4% against forming it by the star formulas (653 -> 663 us).
 __device__ __forceinline__ void hllc64(const double ql[5], const double qr[5], double f[5], const HydroK<double> &k)
 {
 #pragma clang fp contract(off)

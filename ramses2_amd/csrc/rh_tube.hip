@@ -7,9 +7,9 @@
 // through LDS, and all steps of a call run in one launch with three barriers
 // each.  What bounds a step is its dependent chain (conversion, dt reduction,
 // slopes, Riemann solve), at 1024 cells also the issue of one CU.  Measured,
-// MinMod + HLLC: 64 cells 13.9 -> 1.6 us per step, 512 14.9 -> 2.5, 1024 15.0 ->
-// 3.5.  Beyond, with four cells per thread, it spilled and took 16 us, no less
-// than the launches.
+// MinMod + HLLC, 2000 steps a call: 64 cells 13.4 -> 1.5 us per step, 512 14.3 ->
+// 2.4, 1024 14.4 -> 3.8.  Beyond, with four cells per thread, it spilled and took 16
+// us, no less than the launches (14.6).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
